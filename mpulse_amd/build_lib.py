@@ -6,7 +6,10 @@ import sys
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libmpulse_hip.so")
-SOURCES = ["mpx_kernels.hip", "mpx_pass.hip", "mpx_adjoint.hip", "mpx_gauss.hip", "mpx_solver.hip"]
+# (source, storage form): the template-heavy units are compiled once per form, in parallel
+SOURCES = [("mpx_pass.hip", 0), ("mpx_pass.hip", 1), ("mpx_pass.hip", 2), ("mpx_fused.hip", 0), ("mpx_fused.hip", 1),
+           ("mpx_sweep.hip", 0), ("mpx_sweep.hip", 1), ("mpx_kernels.hip", None), ("mpx_adjoint.hip", None),
+           ("mpx_gauss.hip", None), ("mpx_solver.hip", None)]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
     "--offload-arch=gfx950",
@@ -22,9 +25,9 @@ FLAGS = [
 
 def build(verbose=False):
     objs, procs = [], []
-    for src in SOURCES:  # the translation units compile in parallel
-        obj = os.path.join(CSRC, src.replace(".hip", ".o"))
-        cmd = [HIPCC, *FLAGS, "-c", os.path.join(CSRC, src), "-o", obj]
+    for src, form in SOURCES:  # the translation units compile in parallel
+        obj = os.path.join(CSRC, src[:-4] + ("" if form is None else f"_{form}") + ".o")
+        cmd = [HIPCC, *FLAGS, *([] if form is None else [f"-DMPX_FORM={form}"]), "-c", os.path.join(CSRC, src), "-o", obj]
         if verbose:
             print(" ".join(cmd), flush=True)
         procs.append((subprocess.Popen(cmd), cmd))

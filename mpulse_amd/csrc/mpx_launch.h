@@ -60,8 +60,7 @@ template <typename T>
 void launch_fused_B(const StepArgs<T> &a, const StepArgs<T> *dev, hipStream_t s);
 template <typename T>
 void launch_sweep(const SweepArgs<T> &a, int np, bool nonlin, hipStream_t s);
-// single-pass leapfrog kernel (mpx_pass.hip): blocks of 64 z cells x 4 rows of one plane
-void pass_tiles(const GridDims &g, int &nbx, int &nby, int &nbz);
+// single-pass leapfrog kernels (mpx_pass.hip)
 template <typename T>
 void launch_pass(const PassArgs<T> &a, const PassArgs<T> *dev, int np, bool nonlin, hipStream_t s);
 void sweep_tiles(const GridDims &g, int variant, int seg, int &ntz, int &nty, int &nseg);

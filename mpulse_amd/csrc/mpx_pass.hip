@@ -831,7 +831,7 @@ __global__ __launch_bounds__(64 * (R + 1)) void k_march_batch(const PassArgs<T> 
 }
 
 // tile grid: 64 z cells x 4 rows x 1 plane per block
-void pass_tiles(const GridDims &g, int &nbx, int &nby, int &nbz)
+static void pass_tiles(const GridDims &g, int &nbx, int &nby, int &nbz)
 {
     nbx = (g.n[2] + 63) / 64;
     nby = (g.n[1] + 3) / 4;
@@ -939,25 +939,48 @@ static void launch_march_t(const PassArgs<T> &a, const PassArgs<T> *dev, int np,
         launch_march_p<T, RES, false>(a, dev, np, nonlin, s);
 }
 
-template <typename T>
-void launch_pass(const PassArgs<T> &a, const PassArgs<T> *dev, int np, bool nonlin, hipStream_t s)
+// The file is compiled once per storage form (MPX_FORM 0: float64, 1: float32, 2: float32 +
+// residual), so that the variants of the kernels compile in parallel.
+#ifndef MPX_FORM
+#error "MPX_FORM selects the storage form this object holds"
+#endif
+template <typename T, bool RES>
+void launch_pass_form(const PassArgs<T> &a, const PassArgs<T> *dev, int np, bool nonlin, hipStream_t s)
 {
-    if constexpr (sizeof(T) == 4) {
-        if (a.Eolo) {
-            if (a.kernel == 1)
-                launch_march_t<T, true>(a, dev, np, nonlin, s);
-            else
-                launch_pass_t<T, true>(a, dev, np, nonlin, s);
-            return;
-        }
-    }
     if (a.kernel == 1)
-        launch_march_t<T, false>(a, dev, np, nonlin, s);
+        launch_march_t<T, RES>(a, dev, np, nonlin, s);
     else
-        launch_pass_t<T, false>(a, dev, np, nonlin, s);
+        launch_pass_t<T, RES>(a, dev, np, nonlin, s);
 }
-template void launch_pass<double>(const PassArgs<double> &, const PassArgs<double> *, int, bool, hipStream_t);
-template void launch_pass<float>(const PassArgs<float> &, const PassArgs<float> *, int, bool, hipStream_t);
+#if MPX_FORM == 0
+template void launch_pass_form<double, false>(const PassArgs<double> &, const PassArgs<double> *, int, bool,
+                                              hipStream_t);
+extern template void launch_pass_form<float, false>(const PassArgs<float> &, const PassArgs<float> *, int, bool,
+                                                    hipStream_t);
+extern template void launch_pass_form<float, true>(const PassArgs<float> &, const PassArgs<float> *, int, bool,
+                                                   hipStream_t);
+template <>
+void launch_pass<double>(const PassArgs<double> &a, const PassArgs<double> *dev, int np, bool nonlin,
+                         hipStream_t s)
+{
+    launch_pass_form<double, false>(a, dev, np, nonlin, s);
+}
+template <>
+void launch_pass<float>(const PassArgs<float> &a, const PassArgs<float> *dev, int np, bool nonlin,
+                        hipStream_t s)
+{
+    if (a.Eolo)
+        launch_pass_form<float, true>(a, dev, np, nonlin, s);
+    else
+        launch_pass_form<float, false>(a, dev, np, nonlin, s);
+}
+#elif MPX_FORM == 1
+template void launch_pass_form<float, false>(const PassArgs<float> &, const PassArgs<float> *, int, bool,
+                                             hipStream_t);
+#else
+template void launch_pass_form<float, true>(const PassArgs<float> &, const PassArgs<float> *, int, bool,
+                                            hipStream_t);
+#endif
 
 // Batched x march (no residual words, no plasma): tile height of the one-grid kernel of the
 // same variant unless `rows` (3 or 7) is given
@@ -1000,11 +1023,14 @@ void launch_march_batch(const PassArgs<T> *table, const BatchRun *runs, int nrun
     else
         launch_march_batch_r<T, 7>(table, runs, nruns, total, np, nonlin, cp, s);
 }
+#if MPX_FORM == 0
 template int march_batch_rows<double>(int, int, bool, bool);
-template int march_batch_rows<float>(int, int, bool, bool);
 template void launch_march_batch<double>(const PassArgs<double> *, const BatchRun *, int, int, int, int, bool, bool,
                                          hipStream_t);
+#elif MPX_FORM == 1
+template int march_batch_rows<float>(int, int, bool, bool);
 template void launch_march_batch<float>(const PassArgs<float> *, const BatchRun *, int, int, int, int, bool, bool,
                                         hipStream_t);
+#endif
 
 }  // namespace mpx
