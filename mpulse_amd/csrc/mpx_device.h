@@ -345,14 +345,15 @@ __device__ __forceinline__ int layer_index(const CpmlFace &f, int i, int j, int 
     return ((i - f.lo[0]) * f.n1 + (j - f.lo[1])) * f.n2 + (k - f.lo[2]);
 }
 
-// add the current-sheet layers that contain cell (i, j, k), in list order
+// add the current-sheet layers that contain cell (i, j, k), in list order, from the slot at
+// element offset soff of their planes
 template <typename T>
-__device__ __forceinline__ void add_sheets(const StepArgs<T> &a, int i, int j, int k, double &x, double &y,
+__device__ __forceinline__ void add_sheets(const StepArgs<T> &a, int i, int j, int k, int soff, double &x, double &y,
                                            double &z)
 {
     for (int s = 0; s < a.nsheets; ++s)
         if (k == a.sheet[s].kp) {
-            int q = i * a.g.py + j;
+            int q = i * a.g.py + j + soff;
             x += gld(a.sheet[s].J[0] + q);
             y += gld(a.sheet[s].J[1] + q);
             z += gld(a.sheet[s].J[2] + q);
@@ -439,12 +440,12 @@ __device__ __forceinline__ void tile_jk(const GridDims &g, const int lo[3], int 
 }
 
 // add the current-sheet layers of list `sh` that contain cell (i, j, k), in list order
-__device__ __forceinline__ void add_sheet_planes(const Sheet *sh, int n, int py, int i, int j, int k, double &x,
-                                                 double &y, double &z)
+__device__ __forceinline__ void add_sheet_planes(const Sheet *sh, int n, int py, int i, int j, int k, int soff,
+                                                 double &x, double &y, double &z)
 {
     for (int s = 0; s < n; ++s)
         if (k == sh[s].kp) {
-            int q = i * py + j;
+            int q = i * py + j + soff;
             x += gld(sh[s].J[0] + q);
             y += gld(sh[s].J[1] + q);
             z += gld(sh[s].J[2] + q);

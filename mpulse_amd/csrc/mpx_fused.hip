@@ -19,7 +19,7 @@ namespace mpx {
 // Fused E side of one step.  A thread owns one (j, k) column segment of L cells along x and
 // walks it plane by plane, keeping B of the previous plane in registers for the x difference.
 template <typename T, int NP, bool NONLIN, bool CPML, int L, bool LIN = false, bool RES = false>
-__device__ __forceinline__ void fused_E_tile(const StepArgs<T> &a, int tbx, int tby, int tbz)
+__device__ __forceinline__ void fused_E_tile(const StepArgs<T> &a, int tbx, int tby, int tbz, int soff)
 {
     using V = typename Word<T, RES>::V;
     const GridDims &g = a.g;
@@ -143,14 +143,14 @@ __device__ __forceinline__ void fused_E_tile(const StepArgs<T> &a, int tbx, int 
         };
         add_plasma(0);
         if (a.sheets_first)
-            add_sheets(a, i, j, k, jx, jy, jz);
+            add_sheets(a, i, j, k, soff, jx, jy, jz);
         else
             add_cpml();
         add_plasma(1);
         if (a.sheets_first)
             add_cpml();
         else
-            add_sheets(a, i, j, k, jx, jy, jz);
+            add_sheets(a, i, j, k, soff, jx, jy, jz);
         add_plasma(2);
         double idenom = a.idenom, numer = a.numer;
         if (a.epsf || a.plasma) {
@@ -175,7 +175,7 @@ __device__ __forceinline__ void fused_E_tile(const StepArgs<T> &a, int tbx, int 
 // Fused B side of one step: a thread walks L planes along x keeping E of the next plane in
 // registers as the centre of the following iteration.
 template <typename T, bool CPML, int L, bool LIN = false, bool RES = false>
-__device__ __forceinline__ void fused_B_tile(const StepArgs<T> &a, int tbx, int tby, int tbz)
+__device__ __forceinline__ void fused_B_tile(const StepArgs<T> &a, int tbx, int tby, int tbz, int soff)
 {
     using V = typename Word<T, RES>::V;
     const GridDims &g = a.g;
@@ -255,7 +255,7 @@ __device__ __forceinline__ void fused_B_tile(const StepArgs<T> &a, int tbx, int 
         const double dEz_x = ez1 - ez;
         const double dEy_x = ey1 - ey;
         double mx = 0.0, my = 0.0, mz = 0.0;
-        if (a.sheets_first) add_sheets(a, i, j, k, mx, my, mz);
+        if (a.sheets_first) add_sheets(a, i, j, k, soff, mx, my, mz);
         if (CPML) {
 #pragma unroll
             for (int s = 0; s < 2; ++s)
@@ -287,7 +287,7 @@ __device__ __forceinline__ void fused_B_tile(const StepArgs<T> &a, int tbx, int 
                     my += v1;
                 }
         }
-        if (!a.sheets_first) add_sheets(a, i, j, k, mx, my, mz);
+        if (!a.sheets_first) add_sheets(a, i, j, k, soff, mx, my, mz);
         const double kdx = gld(a.ikdH[0] + i);
         unsigned wn = 0;
         const T hx = put<T, RES>((double)pb[u][0] + a.dt * ((dEy_z * kdz - dEz_y * kdy) + mx), wn, 0);
@@ -316,19 +316,20 @@ struct FusedEWaves {
 
 template <typename T, int NP, bool NONLIN, bool CPML, int L, bool RES = false>
 __global__ __attribute__((amdgpu_waves_per_eu(FusedEWaves<T, NP, NONLIN, L, RES>::v))) __launch_bounds__(256) void k_fused_E(
-    const StepArgs<T> *__restrict__ pa, int nbx, int nby, int nbz)
+    const StepArgs<T> *__restrict__ pa, int nbx, int nby, int nbz, int soff)
 {
     int tbx, tby, tbz;
     fused_tile_of(pa->order, pa->band, pa->rev, nbx, nby, nbz, tbx, tby, tbz);
-    fused_E_tile<T, NP, NONLIN, CPML, L, false, RES>(*pa, tbx, tby, tbz);
+    fused_E_tile<T, NP, NONLIN, CPML, L, false, RES>(*pa, tbx, tby, tbz, soff);
 }
 
 template <typename T, bool CPML, int L, bool RES = false>
-__global__ __launch_bounds__(256) void k_fused_B(const StepArgs<T> *__restrict__ pa, int nbx, int nby, int nbz)
+__global__ __launch_bounds__(256) void k_fused_B(const StepArgs<T> *__restrict__ pa, int nbx, int nby, int nbz,
+                                                 int soff)
 {
     int tbx, tby, tbz;
     fused_tile_of(pa->order, pa->band, pa->rev, nbx, nby, nbz, tbx, tby, tbz);
-    fused_B_tile<T, CPML, L, false, RES>(*pa, tbx, tby, tbz);
+    fused_B_tile<T, CPML, L, false, RES>(*pa, tbx, tby, tbz, soff);
 }
 
 // the fused kernels over the tiles of many independent runs, one persistent launch
@@ -337,7 +338,7 @@ __global__ __launch_bounds__(256) void k_fused_E_batch(const StepArgs<T> *__rest
                                                        const BatchRun *__restrict__ runs, int nruns, int total)
 {
     batch_tiles(runs, nruns, total, [&](int r, int tz, int ty, int tx) {
-        fused_E_tile<T, NP, NONLIN, CPML, L, true>(args[r], tz, ty, tx);
+        fused_E_tile<T, NP, NONLIN, CPML, L, true>(args[r], tz, ty, tx, 0);
     });
 }
 
@@ -346,7 +347,7 @@ __global__ __launch_bounds__(256) void k_fused_B_batch(const StepArgs<T> *__rest
                                                        const BatchRun *__restrict__ runs, int nruns, int total)
 {
     batch_tiles(runs, nruns, total,
-                [&](int r, int tz, int ty, int tx) { fused_B_tile<T, CPML, L, true>(args[r], tz, ty, tx); });
+                [&](int r, int tz, int ty, int tx) { fused_B_tile<T, CPML, L, true>(args[r], tz, ty, tx, 0); });
 }
 
 #if MPX_FORM == 0
@@ -427,14 +428,15 @@ template void launch_fused_B_batch<float>(const StepArgs<float> *, const BatchRu
 #endif
 
 template <typename T, int L, bool RES = false>
-static void launch_fused_E_L(const StepArgs<T> &a, const StepArgs<T> *dev, int np, bool nonlin, hipStream_t s)
+static void launch_fused_E_L(const StepArgs<T> &a, const StepArgs<T> *dev, int np, bool nonlin, int soff,
+                             hipStream_t s)
 {
     const GridDims &g = a.g;
     int nbx = (g.n[2] + 63) / 64, nby = (g.n[1] + 3) / 4, nbz = (g.n[0] + L - 1) / L;
     dim3 blk(64, 4);
     dim3 grd(nbx, nby, nbz);
     bool cp = a.nfaces > 0;
-#define MPX_FE(NPV, NL, CP) hipLaunchKernelGGL((k_fused_E<T, NPV, NL, CP, L, RES>), grd, blk, 0, s, dev, nbx, nby, nbz)
+#define MPX_FE(NPV, NL, CP) hipLaunchKernelGGL((k_fused_E<T, NPV, NL, CP, L, RES>), grd, blk, 0, s, dev, nbx, nby, nbz, soff)
 #define MPX_FE_NP(NL, CP)            \
     switch (np) {                    \
     case 0: MPX_FE(0, NL, CP); break; \
@@ -452,24 +454,24 @@ static void launch_fused_E_L(const StepArgs<T> &a, const StepArgs<T> *dev, int n
 }
 
 template <typename T>
-void launch_fused_E(const StepArgs<T> &a, const StepArgs<T> *dev, int np, bool nonlin, hipStream_t s)
+void launch_fused_E(const StepArgs<T> &a, const StepArgs<T> *dev, int np, bool nonlin, int soff, hipStream_t s)
 {
     if constexpr (sizeof(T) == 4) {
         // float32 + residual storage: one plane per thread (the march of the float32 default)
         if (a.Elo) {
-            launch_fused_E_L<T, 1, true>(a, dev, np, nonlin, s);
+            launch_fused_E_L<T, 1, true>(a, dev, np, nonlin, soff, s);
             return;
         }
     }
     switch (a.march) {
-    case 2: launch_fused_E_L<T, 2>(a, dev, np, nonlin, s); break;
-    case 4: launch_fused_E_L<T, 4>(a, dev, np, nonlin, s); break;
-    default: launch_fused_E_L<T, 1>(a, dev, np, nonlin, s); break;
+    case 2: launch_fused_E_L<T, 2>(a, dev, np, nonlin, soff, s); break;
+    case 4: launch_fused_E_L<T, 4>(a, dev, np, nonlin, soff, s); break;
+    default: launch_fused_E_L<T, 1>(a, dev, np, nonlin, soff, s); break;
     }
 }
 
 template <typename T, int L, bool RES = false>
-static void launch_fused_B_L(const StepArgs<T> &a, const StepArgs<T> *dev, hipStream_t s)
+static void launch_fused_B_L(const StepArgs<T> &a, const StepArgs<T> *dev, int soff, hipStream_t s)
 {
     const GridDims &g = a.g;
     int nk = g.n[2] - a.blo[2] + 1, nj = g.n[1] - a.blo[1] + 1, ni = g.n[0] - a.blo[0] + 1;
@@ -477,37 +479,37 @@ static void launch_fused_B_L(const StepArgs<T> &a, const StepArgs<T> *dev, hipSt
     dim3 blk(64, 4);
     dim3 grd(nbx, nby, nbz);
     if (a.nfaces > 0)
-        hipLaunchKernelGGL((k_fused_B<T, true, L, RES>), grd, blk, 0, s, dev, nbx, nby, nbz);
+        hipLaunchKernelGGL((k_fused_B<T, true, L, RES>), grd, blk, 0, s, dev, nbx, nby, nbz, soff);
     else
-        hipLaunchKernelGGL((k_fused_B<T, false, L, RES>), grd, blk, 0, s, dev, nbx, nby, nbz);
+        hipLaunchKernelGGL((k_fused_B<T, false, L, RES>), grd, blk, 0, s, dev, nbx, nby, nbz, soff);
 }
 
 template <typename T>
-void launch_fused_B(const StepArgs<T> &a, const StepArgs<T> *dev, hipStream_t s)
+void launch_fused_B(const StepArgs<T> &a, const StepArgs<T> *dev, int soff, hipStream_t s)
 {
     if constexpr (sizeof(T) == 4) {
         // float32 + residual storage: one or two planes per thread
         if (a.Blo) {
             if (a.march == 1)
-                launch_fused_B_L<T, 1, true>(a, dev, s);
+                launch_fused_B_L<T, 1, true>(a, dev, soff, s);
             else
-                launch_fused_B_L<T, 2, true>(a, dev, s);
+                launch_fused_B_L<T, 2, true>(a, dev, soff, s);
             return;
         }
     }
     switch (a.march) {
-    case 2: launch_fused_B_L<T, 2>(a, dev, s); break;
-    case 4: launch_fused_B_L<T, 4>(a, dev, s); break;
-    default: launch_fused_B_L<T, 1>(a, dev, s); break;
+    case 2: launch_fused_B_L<T, 2>(a, dev, soff, s); break;
+    case 4: launch_fused_B_L<T, 4>(a, dev, soff, s); break;
+    default: launch_fused_B_L<T, 1>(a, dev, soff, s); break;
     }
 }
 
 #if MPX_FORM == 0
-template void launch_fused_E<double>(const StepArgs<double> &, const StepArgs<double> *, int, bool, hipStream_t);
-template void launch_fused_B<double>(const StepArgs<double> &, const StepArgs<double> *, hipStream_t);
+template void launch_fused_E<double>(const StepArgs<double> &, const StepArgs<double> *, int, bool, int, hipStream_t);
+template void launch_fused_B<double>(const StepArgs<double> &, const StepArgs<double> *, int, hipStream_t);
 #else
-template void launch_fused_E<float>(const StepArgs<float> &, const StepArgs<float> *, int, bool, hipStream_t);
-template void launch_fused_B<float>(const StepArgs<float> &, const StepArgs<float> *, hipStream_t);
+template void launch_fused_E<float>(const StepArgs<float> &, const StepArgs<float> *, int, bool, int, hipStream_t);
+template void launch_fused_B<float>(const StepArgs<float> &, const StepArgs<float> *, int, hipStream_t);
 #endif
 
 }  // namespace mpx

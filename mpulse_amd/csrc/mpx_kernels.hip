@@ -1,8 +1,9 @@
 // gfx950 kernels of the reference-structured path -- one kernel per loop of
 // FDTD_PLRCSolver::stepScheme (src/fdtd_plrc.t:127-168): CPML currents, current totals, E
 // update, ghost wrap, and the same for the magnetic side -- of the plain / Kerr-only / ADE
-// solvers, of the source sheets, and of the diagnostics and field output.  The fused kernels are in mpx_fused.hip,
-// the pass kernels in mpx_pass.hip, the sweep in mpx_sweep.hip.  Threads run along z (the contiguous dimension), 64 per wavefront, so every
+// solvers, and of the diagnostics and field output.  The fused kernels are in mpx_fused.hip,
+// the pass kernels in mpx_pass.hip, the sweep in mpx_sweep.hip, the source sheets in
+// mpx_sheet.hip.  Threads run along z (the contiguous dimension), 64 per wavefront, so every
 // field load of a wavefront is one coalesced 256/512-byte segment.
 #include <hip/hip_runtime.h>
 
@@ -10,185 +11,6 @@
 #include "mpx_launch.h"
 
 namespace mpx {
-
-// ------------------------------------------------------------------------------------
-// source sheets: IncidentSource{E,H}Current::stepScheme, src/incsource.t:40-73, 112-145
-// ------------------------------------------------------------------------------------
-
-__device__ inline void plane_getH(const PlaneParams &W, int i, int j, int l, int time, double out[3])
-{
-    // PlaneWaveSourceEFunc::getHField src/sources.cpp:107-125 / PlaneGaussSourceEFunc src/sources.cpp:266-284
-    double realtime = W.dt * (time - 0.5);
-    double posx = W.k[0] * i * W.dx + W.k[1] * (j + 0.5) * W.dy + W.k[2] * (l + 0.5) * W.dz + W.om * realtime;
-    double posy = W.k[0] * (i + 0.5) * W.dx + W.k[1] * j * W.dy + W.k[2] * (l + 0.5) * W.dz + W.om * realtime;
-    double posz = W.k[0] * (i + 0.5) * W.dx + W.k[1] * (j + 0.5) * W.dy + W.k[2] * l * W.dz + W.om * realtime;
-    double pos[3] = {posx, posy, posz};
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        if (!W.gauss) {
-            double h = W.H[d] * sin(pos[d]) + W.H_bg[d];
-            if (pos[d] < W.ramp) h *= pos[d] / W.ramp;
-            out[d] = h;
-        } else {
-            double q = (pos[d] - W.offset) / W.width;
-            out[d] = (W.H[d] * exp(-(q * q))) * sin(pos[d]);
-        }
-    }
-}
-
-__device__ inline void plane_getE(const PlaneParams &W, int i, int j, int l, int time, double out[3])
-{
-    // PlaneWaveSourceHFunc::getEField src/sources.cpp:150-173 / PlaneGaussSourceHFunc src/sources.cpp:308-331
-    double realtime = W.dt * time;
-    double posx = W.k[0] * (i + 0.5) * W.dx + W.k[1] * j * W.dy + W.k[2] * l * W.dz + W.om * realtime;
-    double posy = W.k[0] * i * W.dx + W.k[1] * (j + 0.5) * W.dy + W.k[2] * l * W.dz + W.om * realtime;
-    double posz = W.k[0] * i * W.dx + W.k[1] * j * W.dy + W.k[2] * (l + 0.5) * W.dz + W.om * realtime;
-    double pos[3] = {posx, posy, posz};
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        if (!W.gauss) {
-            double e = W.E[d] * sin(pos[d]) + W.E_bg[d];
-            if (pos[d] < W.ramp) e *= pos[d] / W.ramp;
-            out[d] = e;
-        } else {
-            double q = (pos[d] - W.offset) / W.width;
-            out[d] = (W.E[d] * exp(-(q * q))) * sin(pos[d]);
-        }
-    }
-}
-
-// one sheet cell (i, j) at step `time`; KIND > 0 fixes the source kind at compile time (each
-// kind then gets only the registers it needs), KIND = 0 reads it from the descriptor
-template <int KIND = 0>
-__device__ __forceinline__ void sheet_eval_point(const SheetEval &a, const FaddeevaTables &ft, int i, int j, int time)
-{
-    const int kind = KIND > 0 ? KIND : a.kind;
-    int z = a.sheet.kp + a.off;
-    double f[3] = {0, 0, 0};
-    const PulseParams &P = a.pulse;
-    if (kind == 1) {
-        if (!a.isH) {
-            // getHField, src/shortpulseinject.cpp:151-178
-            double posxo = (i - P.centrex) * P.DX;
-            double posxh = (i + 0.5 - P.centrex) * P.DX;
-            double posyo = (j - P.centrey) * P.DY;
-            double posyh = (j + 0.5 - P.centrey) * P.DY;
-            double poszh = (z - 0.5 - P.centrez) * P.DZ - P.ZShift;
-            double posTime = (time - 0.5) * P.DT - P.TShift;
-            f[0] = P.amp * pulse_bfunc(P, ft, posxo, posyh, poszh, posTime, true).re;
-            f[1] = P.amp * pulse_bfunc(P, ft, posxh, posyo, poszh, posTime, false).re;
-        } else {
-            // getEField, src/shortpulseinject.cpp:126-149
-            double posxh = (i + 0.5 - P.centrex) * P.DX;
-            double posyo = (j - P.centrey) * P.DY;
-            double poszo = (z - P.centrez) * P.DZ - P.ZShift;
-            double posTime = time * P.DT - P.TShift;
-            f[0] = P.amp * pulse_efunc(P, ft, posxh, posyo, poszo, posTime).re;
-        }
-    } else if (kind == 4) {
-        // GaussInjectSourceFunc::getHField / getEField, src/gaussinject.cpp:203-224
-        const GaussSheetParams &G = a.gauss;
-        if (G.active) {
-            const size_t q = ((size_t)(time - G.blockToff) * a.nx2 + i) * a.ny2 + j;
-            if (!a.isH) {
-                f[0] = G.sqeps * G.amp * G.F1[q];
-            } else {
-                f[0] = G.amp * G.F1[q];
-                f[1] = G.amp * G.F2[q];
-            }
-        }
-        (void)z;
-    } else if (kind == 3) {
-        // amp Re[env(t - z/v) U exp(-i(om0 t - phase))], env(s) = exp(-s^2/T^2)
-        const FocusedParams &F = a.focused;
-        size_t p = (size_t)i * a.ny2 + j;
-        double t = a.isH ? time * F.DT - F.TShift : (time - 0.5) * F.DT - F.TShift;
-        double z = a.isH ? F.zE : F.zB;
-        double s = t - z / F.v;
-        double env = F.amp * exp(-(s * s) / (F.T * F.T));
-        double sn, cs;
-        sincos(-(F.om0 * t - F.phase), &sn, &cs);
-        if (a.isH) {
-            double2 u = F.ex[p];
-            f[0] = env * (u.x * cs - u.y * sn);
-        } else {
-            double2 u = F.bx[p], w = F.by[p];
-            f[0] = env * (u.x * cs - u.y * sn);
-            f[1] = env * (w.x * cs - w.y * sn);
-        }
-        (void)z;
-    } else {
-        if (!a.isH)
-            plane_getH(a.plane, i, j, z, time, f);
-        else
-            plane_getE(a.plane, i, j, z, time, f);
-    }
-    size_t q = (size_t)i * a.ny2 + j;
-    a.sheet.J[a.t1][q] = f[a.t2] / a.DX;
-    a.sheet.J[a.t2][q] = f[a.t1] / a.DX;
-}
-
-template <int KIND>
-__global__ __launch_bounds__(256) void k_sheet_eval(SheetEval a, FaddeevaTables ft)
-{
-    int j = blockIdx.x * blockDim.x + threadIdx.x;
-    int i = blockIdx.y;
-    if (j >= a.ny2 || i >= a.nx2) return;
-    sheet_eval_point<KIND>(a, ft, i, j, a.time);
-}
-
-// The sheets of many runs in one launch.  Sheet s owns blocks first[s] .. first[s+1]-1, one
-// block per 64 cells of a row; the step is *time + tstep (the counter lives on the device so
-// that a captured graph can be replayed at later steps), hshift less for the H currents.  Only
-// the sheets of the sides in `sides` (bit 0: E currents, bit 1: H currents) are evaluated.
-__global__ __launch_bounds__(64) void k_sheet_eval_batch(const SheetEval *__restrict__ list,
-                                                         const int *__restrict__ first, int n, FaddeevaTables ft,
-                                                         const int *__restrict__ time, int tstep, int hshift,
-                                                         int sides)
-{
-    const int b = blockIdx.x;
-    int lo = 0, hi = n - 1;  // last sheet with first[s] <= b
-    while (lo < hi) {
-        int mid = (lo + hi + 1) >> 1;
-        if (first[mid] <= b) lo = mid; else hi = mid - 1;
-    }
-    const SheetEval &a = list[lo];
-    if (!(sides >> (a.isH ? 1 : 0) & 1)) return;
-    const int nyb = (a.ny2 + 63) >> 6;
-    const int local = b - first[lo];
-    const int i = local / nyb, j = (local - i * nyb) * 64 + threadIdx.x;
-    if (i >= a.nx2 || j >= a.ny2) return;
-    sheet_eval_point(a, ft, i, j, *time + tstep - (a.isH ? hshift : 0));
-}
-
-__global__ void k_advance_time(int *time, int k)
-{
-    if (threadIdx.x == 0) *time += k;
-}
-
-void launch_sheet_eval_batch(const SheetEval *list, const int *first, int n, int blocks, const FaddeevaTables &ft,
-                             const int *time, int tstep, hipStream_t s, int hshift, int sides)
-{
-    hipLaunchKernelGGL(k_sheet_eval_batch, dim3(blocks), dim3(64), 0, s, list, first, n, ft, time, tstep, hshift,
-                       sides);
-}
-
-void launch_advance_time(int *time, int k, hipStream_t s)
-{
-    hipLaunchKernelGGL(k_advance_time, dim3(1), dim3(64), 0, s, time, k);
-}
-
-void launch_sheet_eval(const SheetEval &a, const FaddeevaTables &ft, hipStream_t s)
-{
-    dim3 blk(64);
-    dim3 grd((a.ny2 + 63) / 64, a.nx2);
-    switch (a.kind) {
-    case 1: hipLaunchKernelGGL(k_sheet_eval<1>, grd, blk, 0, s, a, ft); break;
-    case 3: hipLaunchKernelGGL(k_sheet_eval<3>, grd, blk, 0, s, a, ft); break;
-    case 4: hipLaunchKernelGGL(k_sheet_eval<4>, grd, blk, 0, s, a, ft); break;
-    default: hipLaunchKernelGGL(k_sheet_eval<2>, grd, blk, 0, s, a, ft); break;
-    }
-}
 
 // ------------------------------------------------------------------------------------
 // reference-structured path
@@ -685,28 +507,6 @@ template void launch_energy<double>(const GridDims &, double *const[3], double *
                                     hipStream_t, const unsigned *, const unsigned *, double);
 template void launch_energy<float>(const GridDims &, float *const[3], float *const[3], double *, double *,
                                    hipStream_t, const unsigned *, const unsigned *, double);
-
-}  // namespace mpx
-
-namespace mpx {
-
-// Re Efunc(0,0,0,0) with Phase = TShift = ZShift = 0: the amplitude normalisation of
-// ShortPulseInjectSourceFunc::setParam, src/shortpulseinject.cpp:101-112
-__global__ void k_pulse_norm(PulseParams P, FaddeevaTables ft, double *out)
-{
-    if (threadIdx.x == 0 && blockIdx.x == 0) *out = pulse_efunc(P, ft, 0, 0, 0, 0).re;
-}
-
-double pulse_norm_device(const PulseParams &P, const FaddeevaTables &ft, hipStream_t s)
-{
-    double *d = nullptr, h = 0;
-    if (hipMalloc(&d, sizeof(double)) != hipSuccess) return NAN;
-    hipLaunchKernelGGL(k_pulse_norm, dim3(1), dim3(64), 0, s, P, ft, d);
-    if (hipMemcpyAsync(&h, d, sizeof(double), hipMemcpyDeviceToHost, s) != hipSuccess) h = NAN;
-    if (hipStreamSynchronize(s) != hipSuccess) h = NAN;
-    (void)hipFree(d);
-    return h;
-}
 
 }  // namespace mpx
 

@@ -43,7 +43,13 @@ struct ProbeArgs {
     const size_t *idx;
 };
 
-void launch_sheet_eval(const SheetEval &a, const FaddeevaTables &ft, hipStream_t s);
+// source sheets (mpx_sheet.hip): one source's E sheet (e, may be null) at steps tE .. and its H
+// sheet (h, may be null) at steps tH .., step q of n into slot n - 1 - q of its planes
+void launch_sheet_steps(const SheetEval *e, int tE, int nE, const SheetEval *h, int tH, int nH,
+                        const FaddeevaTables &ft, hipStream_t s);
+int sheet_tasks(const SheetEval &a);             // separately evaluated components
+int sheet_points(const SheetEval &a, int task);  // points evaluated for one of them
+int sheet_slots(long long points);               // slots for that many points per step
 void launch_ref_cpml(const StepArgs<double> &a, int fi, bool isH, hipStream_t s);
 void launch_ref_sum(const GridDims &g, const SumList &L, double *const T[3], hipStream_t s);
 template <typename T>
@@ -53,16 +59,17 @@ void launch_ref_stepB(const StepArgs<double> &a, hipStream_t s);
 void launch_ref_plasma_density(const StepArgs<double> &a, hipStream_t s);
 void launch_ref_plasma_current(const StepArgs<double> &a, hipStream_t s);
 void launch_init_accumulator(const StepArgs<double> &a, int np, hipStream_t s);
-// `a` is the host copy (launch shape), `dev` the same block in device memory
+// `a` is the host copy (launch shape), `dev` the same block in device memory; soff: element offset
+// of the step's slot in the source sheets' planes
 template <typename T>
-void launch_fused_E(const StepArgs<T> &a, const StepArgs<T> *dev, int np, bool nonlin, hipStream_t s);
+void launch_fused_E(const StepArgs<T> &a, const StepArgs<T> *dev, int np, bool nonlin, int soff, hipStream_t s);
 template <typename T>
-void launch_fused_B(const StepArgs<T> &a, const StepArgs<T> *dev, hipStream_t s);
+void launch_fused_B(const StepArgs<T> &a, const StepArgs<T> *dev, int soff, hipStream_t s);
 template <typename T>
 void launch_sweep(const SweepArgs<T> &a, int np, bool nonlin, hipStream_t s);
 // single-pass leapfrog kernels (mpx_pass.hip)
 template <typename T>
-void launch_pass(const PassArgs<T> &a, const PassArgs<T> *dev, int np, bool nonlin, hipStream_t s);
+void launch_pass(const PassArgs<T> &a, const PassArgs<T> *dev, int np, bool nonlin, int soff, hipStream_t s);
 void sweep_tiles(const GridDims &g, int variant, int seg, int &ntz, int &nty, int &nseg);
 template <typename T>
 void launch_sweep_batch(const SweepArgs<T> *args, const BatchRun *runs, int nruns, int total, int variant,
@@ -76,8 +83,10 @@ void launch_fused_B_batch(const StepArgs<T> *args, const BatchRun *runs, int nru
                           bool cpml, hipStream_t s);
 // the sheets of the sides in `sides` (bit 0: E currents, bit 1: H currents); H currents at
 // step *time + tstep - hshift, E currents at *time + tstep
-void launch_sheet_eval_batch(const SheetEval *list, const int *first, int n, int blocks, const FaddeevaTables &ft,
-                             const int *time, int tstep, hipStream_t s, int hshift = 0, int sides = 3);
+// (pulses: every entry is a short pulse)
+void launch_sheet_eval_batch(const SheetTask *list, const int *first, int n, int blocks, bool pulses,
+                             const FaddeevaTables &ft, const int *time, int tstep, hipStream_t s, int hshift = 0,
+                             int sides = 3);
 // batched x march (mpx_pass.hip): run r's tiles are runs[r].first .. of a list of `total`
 template <typename T>
 int march_batch_rows(int rows, int np, bool nonlin, bool cp);

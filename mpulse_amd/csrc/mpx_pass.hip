@@ -55,10 +55,10 @@ __device__ __forceinline__ void cpml_hface_pp(const CpmlFace &f, const T *o0, co
 template <typename T, bool CPML, bool RES>
 __device__ __forceinline__ void pass_m(const PassArgs<T> &a, int i, int j, int k, bool store, double dEy_z,
                                        double dEx_z, double dEz_y, double dEx_y, double dEz_x, double dEy_x,
-                                       double &mx, double &my, double &mz, bool cp, bool sh, bool live = true)
+                                       double &mx, double &my, double &mz, bool cp, bool sh, int soff, bool live = true)
 {
     mx = my = mz = 0.0;
-    if (sh && a.sheets_first) add_sheet_planes(a.hsheet, a.nhsheets, a.g.py, i, j, k, mx, my, mz);
+    if (sh && a.sheets_first) add_sheet_planes(a.hsheet, a.nhsheets, a.g.py, i, j, k, soff, mx, my, mz);
     if (CPML && cp) {
         bool in[2];
         in_faces(a.hfbd, a.hface, 1, j, in);
@@ -104,14 +104,14 @@ __device__ __forceinline__ void pass_m(const PassArgs<T> &a, int i, int j, int k
                 my += v1;
             }
     }
-    if (sh && !a.sheets_first) add_sheet_planes(a.hsheet, a.nhsheets, a.g.py, i, j, k, mx, my, mz);
+    if (sh && !a.sheets_first) add_sheet_planes(a.hsheet, a.nhsheets, a.g.py, i, j, k, soff, mx, my, mz);
 }
 
 // Electric current total at (i, j, k) (CPML E auxiliaries updated in place; owned cells only).
 template <typename T, bool CPML, bool RES>
 __device__ __forceinline__ void pass_j(const PassArgs<T> &a, int i, int j, int k, double dBz_y, double dBy_z,
                                        double dBx_z, double dBz_x, double dBy_x, double dBx_y, double &jx,
-                                       double &jy, double &jz, bool cp, bool sh, bool live = true,
+                                       double &jy, double &jz, bool cp, bool sh, int soff, bool live = true,
                                        const double *jpv = nullptr)
 {
     jx = jy = jz = 0.0;
@@ -167,13 +167,13 @@ __device__ __forceinline__ void pass_j(const PassArgs<T> &a, int i, int j, int k
     };
     add_plasma(0);
     if (a.sheets_first) {
-        if (sh) add_sheet_planes(a.sheet, a.nsheets, a.g.py, i, j, k, jx, jy, jz);
+        if (sh) add_sheet_planes(a.sheet, a.nsheets, a.g.py, i, j, k, soff, jx, jy, jz);
         add_plasma(1);
         add_cpml();
     } else {
         add_cpml();
         add_plasma(1);
-        if (sh) add_sheet_planes(a.sheet, a.nsheets, a.g.py, i, j, k, jx, jy, jz);
+        if (sh) add_sheet_planes(a.sheet, a.nsheets, a.g.py, i, j, k, soff, jx, jy, jz);
     }
     add_plasma(2);
 }
@@ -212,19 +212,19 @@ __device__ __forceinline__ Cell3<T, RES> ld3(const T *const f[3], const unsigned
 template <typename T, bool CPML, bool RES>
 __device__ __forceinline__ void b_cell_k(const PassArgs<T> &a, int i, int j, int k, const Cell3<T, RES> &b0,
                                          const double d[6], bool store, T h[3], unsigned &w, double b[3], bool cp,
-                                         bool sh, bool live, double kdx, double kdy, double kdz)
+                                         bool sh, int soff, bool live, double kdx, double kdy, double kdz)
 {
     double mx, my, mz;
-    pass_m<T, CPML, RES>(a, i, j, k, store, d[0], d[1], d[2], d[3], d[4], d[5], mx, my, mz, cp, sh, live);
+    pass_m<T, CPML, RES>(a, i, j, k, store, d[0], d[1], d[2], d[3], d[4], d[5], mx, my, mz, cp, sh, soff, live);
     b_update<T, RES>((double)b0.x, (double)b0.y, (double)b0.z, d[0], d[1], d[2], d[3], d[4], d[5], kdx, kdy, kdz,
                      a.dt, mx, my, mz, h, w, b);
 }
 template <typename T, bool CPML, bool RES>
 __device__ __forceinline__ void b_cell(const PassArgs<T> &a, int i, int j, int k, const Cell3<T, RES> &b0,
                                        const double d[6], bool store, T h[3], unsigned &w, double b[3], bool cp,
-                                       bool sh, bool live = true)
+                                       bool sh, int soff, bool live = true)
 {
-    b_cell_k<T, CPML, RES>(a, i, j, k, b0, d, store, h, w, b, cp, sh, live, gld(a.ikdH[0] + i), gld(a.ikdH[1] + j),
+    b_cell_k<T, CPML, RES>(a, i, j, k, b0, d, store, h, w, b, cp, sh, soff, live, gld(a.ikdH[0] + i), gld(a.ikdH[1] + j),
                            gld(a.ikdH[2] + k));
 }
 
@@ -237,7 +237,8 @@ __device__ __forceinline__ void b_cell(const PassArgs<T> &a, int i, int j, int k
 // stored, so that one wait covers them; the neighbours' B is computed before the cell's own
 // (whose CPML H auxiliaries are stored), and all field stores come last.
 template <typename T, int NP, bool NONLIN, bool CPML, bool RES>
-__global__ __launch_bounds__(256) void k_pass(const PassArgs<T> *__restrict__ pa, int nbx, int nby, int nbz)
+__global__ __launch_bounds__(256) void k_pass(const PassArgs<T> *__restrict__ pa, int nbx, int nby, int nbz,
+                                              int soff)
 {
     using V = typename Word<T, RES>::V;
     using C3 = Cell3<T, RES>;
@@ -326,19 +327,19 @@ __global__ __launch_bounds__(256) void k_pass(const PassArgs<T> *__restrict__ pa
         const double x_ = exm.x, y_ = exm.y, z_ = exm.z;
         const double d[6] = {(double)zx.y - y_, (double)zx.x - x_, (double)exm_yp.z - z_, (double)exm_yp.x - x_,
                              ez - z_, ey - y_};
-        b_cell<T, CPML, RES>(a, im, j, k, bxm, d, false, hh, hw, bx_m, cp, sh);
+        b_cell<T, CPML, RES>(a, im, j, k, bxm, d, false, hh, hw, bx_m, cp, sh, soff);
     }
     {
         const double x_ = eym.x, y_ = eym.y, z_ = eym.z;
         const double d[6] = {(double)zy.y - y_, (double)zy.x - x_, ez - z_, ex - x_, (double)eym_xp.z - z_,
                              (double)eym_xp.y - y_};
-        b_cell<T, CPML, RES>(a, i, jm, k, bym, d, false, hh, hw, by_m, cp, sh);
+        b_cell<T, CPML, RES>(a, i, jm, k, bym, d, false, hh, hw, by_m, cp, sh, soff);
     }
     {
         const double x_ = ezm.x, y_ = ezm.y, z_ = ezm.z;
         const double d[6] = {ey - y_, ex - x_, (double)ezm_yp.z - z_, (double)ezm_yp.x - x_, (double)ezm_xp.z - z_,
                              (double)ezm_xp.y - y_};
-        b_cell<T, CPML, RES>(a, i, j, km, bzm, d, false, hh, hw, bz_m, cp, sh);
+        b_cell<T, CPML, RES>(a, i, j, km, bzm, d, false, hh, hw, bz_m, cp, sh, soff);
     }
     // B^(n+1) at the cell (its CPML H auxiliaries stored)
     T bh[3];
@@ -347,14 +348,14 @@ __global__ __launch_bounds__(256) void k_pass(const PassArgs<T> *__restrict__ pa
     {
         const double d[6] = {(double)z0.y - ey, (double)z0.x - ex, (double)eyp.z - ez, (double)eyp.x - ex,
                              (double)exp_.z - ez, (double)exp_.y - ey};
-        b_cell<T, CPML, RES>(a, i, j, k, b0, d, true, bh, bw, b, cp, sh);
+        b_cell<T, CPML, RES>(a, i, j, k, b0, d, true, bh, bw, b, cp, sh, soff);
     }
     // E^(n+2) at the cell
     const double dBz_y = b[2] - by_m[2], dBx_y = b[0] - by_m[0];
     const double dBy_z = b[1] - bz_m[1], dBx_z = b[0] - bz_m[0];
     const double dBz_x = b[2] - bx_m[2], dBy_x = b[1] - bx_m[1];
     double jx, jy, jz;
-    pass_j<T, CPML, RES>(a, i, j, k, dBz_y, dBy_z, dBx_z, dBz_x, dBy_x, dBx_y, jx, jy, jz, cp, sh);
+    pass_j<T, CPML, RES>(a, i, j, k, dBz_y, dBy_z, dBx_z, dBz_x, dBy_x, dBx_y, jx, jy, jz, cp, sh, soff);
     double idenom = a.idenom, numer = a.numer;
     if (a.epsf) {
         double denom;
@@ -494,7 +495,7 @@ __device__ __forceinline__ void lds_barrier()
 // One tile (64 z cells x R rows from (k0, j0) = (64 tz + 1, R ty + 1), x planes
 // seg ts + 1 .. seg (ts + 1)) of the march; the kernels below map their blocks to tiles.
 template <typename T, int NP, bool NONLIN, bool CPML, bool RES, int R, bool PL>
-__device__ __forceinline__ void march_tile(const PassArgs<T> &a, int tz, int ty, int ts)
+__device__ __forceinline__ void march_tile(const PassArgs<T> &a, int tz, int ty, int ts, int soff)
 {
     using RW = Raw3<T, RES>;
     using C3 = Cell3<T, RES>;
@@ -584,7 +585,7 @@ __device__ __forceinline__ void march_tile(const PassArgs<T> &a, int tz, int ty,
                 T h[3];
                 unsigned hw;
                 double b[3];
-                b_cell_k<T, CPML, RES>(a, p, j, k, cell_of(b0), d, false, h, hw, b, cp, sh, ok, kxh, khy, khz);
+                b_cell_k<T, CPML, RES>(a, p, j, k, cell_of(b0), d, false, h, hw, b, cp, sh, soff, ok, kxh, khy, khz);
                 brow[bb][0].a[lane] = b[0];
                 brow[bb][0].b[lane] = b[2];
             }
@@ -596,7 +597,7 @@ __device__ __forceinline__ void march_tile(const PassArgs<T> &a, int tz, int ty,
                 unsigned hw;
                 double b[3];
                 b_cell_k<T, CPML, RES>(a, p, col ? jc : j, col ? kc : k, cell_of(cb0), d, kzero, h, hw, b, cp, sh,
-                                       col, kxh, khyc, khzc);
+                                       soff, col, kxh, khyc, khzc);
                 bcol[bb].a[lane] = b[0];
                 bcol[bb].b[lane] = b[1];
                 if (kzero && col) {
@@ -678,7 +679,7 @@ __device__ __forceinline__ void march_tile(const PassArgs<T> &a, int tz, int ty,
             }
             const double d[6] = {zy - e.y, zx - e.x, erow[be][w + 1].b[lane] - e.z, erow[be][w + 1].a[lane] - e.x,
                                  (double)n.z - e.z, (double)n.y - e.y};
-            b_cell_k<T, CPML, RES>(a, p, j, k, cell_of(b0w), d, store, h, hw, b, cp, sh, ok, kxh, khy, khz);
+            b_cell_k<T, CPML, RES>(a, p, j, k, cell_of(b0w), d, store, h, hw, b, cp, sh, soff, ok, kxh, khy, khz);
         };
         Stage cur;
         C3 e = cell_of(ldp3<T, RES>(a.Eo, a.Eolo, (size_t)pm * sx, o * SZ));  // E^(n+1) at plane pm
@@ -761,7 +762,7 @@ __device__ __forceinline__ void march_tile(const PassArgs<T> &a, int tz, int ty,
                 }
             }
             double jx, jy, jz;
-            pass_j<T, CPML, RES>(a, p, j, k, dBz_y, dBy_z, dBx_z, dBz_x, dBy_x, dBx_y, jx, jy, jz, cp, sh, ok,
+            pass_j<T, CPML, RES>(a, p, j, k, dBz_y, dBy_z, dBx_z, dBz_x, dBy_x, dBx_y, jx, jy, jz, cp, sh, soff, ok,
                                  PL ? jpv : nullptr);
             double idenom = a.idenom, numer = a.numer;
             if (a.epsf || (PL && a.plasma)) {  // cell_eps with the prefetched permittivity and Sigma dt / 2
@@ -804,12 +805,12 @@ __device__ __forceinline__ unsigned xcd_share(unsigned lin, unsigned total)
 // one grid: tiles in the order z tiles fastest, then tile rows, then x segments
 template <typename T, int NP, bool NONLIN, bool CPML, bool RES, int R, bool PL>
 __global__ __launch_bounds__(64 * (R + 1)) void k_march(const PassArgs<T> *__restrict__ pa, int nbz, int nby,
-                                                        int nseg)
+                                                        int nseg, int soff)
 {
     unsigned t = xcd_share(blockIdx.x, (unsigned)nbz * nby * nseg);
     const int tz = (int)(t % (unsigned)nbz);
     t /= (unsigned)nbz;
-    march_tile<T, NP, NONLIN, CPML, RES, R, PL>(*pa, tz, (int)(t % (unsigned)nby), (int)(t / (unsigned)nby));
+    march_tile<T, NP, NONLIN, CPML, RES, R, PL>(*pa, tz, (int)(t % (unsigned)nby), (int)(t / (unsigned)nby), soff);
 }
 
 // Independent runs in one launch: run r owns the tiles runs[r].first .. runs[r+1].first - 1
@@ -827,7 +828,7 @@ __global__ __launch_bounds__(64 * (R + 1)) void k_march_batch(const PassArgs<T> 
     }
     const BatchRun &B = runs[lo];
     const int local = t - B.first, tz = local % B.ntz, rest = local / B.ntz;
-    march_tile<T, NP, NONLIN, CPML, RES, R, PL>(pa[lo], tz, rest % B.nty, rest / B.nty);
+    march_tile<T, NP, NONLIN, CPML, RES, R, PL>(pa[lo], tz, rest % B.nty, rest / B.nty, 0);
 }
 
 // tile grid: 64 z cells x 4 rows x 1 plane per block
@@ -839,13 +840,13 @@ static void pass_tiles(const GridDims &g, int &nbx, int &nby, int &nbz)
 }
 
 template <typename T, bool RES>
-static void launch_pass_t(const PassArgs<T> &a, const PassArgs<T> *dev, int np, bool nonlin, hipStream_t s)
+static void launch_pass_t(const PassArgs<T> &a, const PassArgs<T> *dev, int np, bool nonlin, int soff, hipStream_t s)
 {
     int nbx, nby, nbz;
     pass_tiles(a.g, nbx, nby, nbz);
     dim3 grd(nbx, nby, nbz), blk(64, 4);
     const bool cp = a.nefaces > 0 || a.nhfaces > 0;
-#define MPX_PS(NPV, NL, CP) hipLaunchKernelGGL((k_pass<T, NPV, NL, CP, RES>), grd, blk, 0, s, dev, nbx, nby, nbz)
+#define MPX_PS(NPV, NL, CP) hipLaunchKernelGGL((k_pass<T, NPV, NL, CP, RES>), grd, blk, 0, s, dev, nbx, nby, nbz, soff)
 #define MPX_PS_NP(NL, CP)            \
     switch (np) {                    \
     case 0: MPX_PS(0, NL, CP); break; \
@@ -864,13 +865,13 @@ static void launch_pass_t(const PassArgs<T> &a, const PassArgs<T> *dev, int np, 
 
 // x march: 64 z cells x R rows x `seg` planes per block, R + 1 waves
 template <typename T, bool RES, int R, bool PL>
-static void launch_march_r(const PassArgs<T> &a, const PassArgs<T> *dev, int np, bool nonlin, hipStream_t s)
+static void launch_march_r(const PassArgs<T> &a, const PassArgs<T> *dev, int np, bool nonlin, int soff, hipStream_t s)
 {
     const int nbz = (a.g.n[2] + 63) / 64, nby = (a.g.n[1] + R - 1) / R, nseg = (a.g.n[0] + a.seg - 1) / a.seg;
     dim3 grd(nbz * nby * nseg), blk(64, R + 1);
     const bool cp = a.nefaces > 0 || a.nhfaces > 0;
 #define MPX_MS(NPV, NL, CP) \
-    hipLaunchKernelGGL((k_march<T, NPV, NL, CP, RES, R, PL>), grd, blk, 0, s, dev, nbz, nby, nseg)
+    hipLaunchKernelGGL((k_march<T, NPV, NL, CP, RES, R, PL>), grd, blk, 0, s, dev, nbz, nby, nseg, soff)
 #define MPX_MS_NP(NL, CP)             \
     switch (np) {                     \
     case 0: MPX_MS(0, NL, CP); break; \
@@ -920,23 +921,23 @@ static int march_auto_rows(int np, bool nonlin, bool cp)
 }
 
 template <typename T, bool RES, bool PL>
-static void launch_march_p(const PassArgs<T> &a, const PassArgs<T> *dev, int np, bool nonlin, hipStream_t s)
+static void launch_march_p(const PassArgs<T> &a, const PassArgs<T> *dev, int np, bool nonlin, int soff, hipStream_t s)
 {
     const int rows = a.rows ? a.rows : march_auto_rows<T, RES, PL>(np, nonlin, a.nefaces > 0 || a.nhfaces > 0);
     if (rows == 3)
-        launch_march_r<T, RES, 3, PL>(a, dev, np, nonlin, s);
+        launch_march_r<T, RES, 3, PL>(a, dev, np, nonlin, soff, s);
     else
-        launch_march_r<T, RES, 7, PL>(a, dev, np, nonlin, s);
+        launch_march_r<T, RES, 7, PL>(a, dev, np, nonlin, soff, s);
 }
 
 // the plasma updates are a separate instantiation: they raise the register count
 template <typename T, bool RES>
-static void launch_march_t(const PassArgs<T> &a, const PassArgs<T> *dev, int np, bool nonlin, hipStream_t s)
+static void launch_march_t(const PassArgs<T> &a, const PassArgs<T> *dev, int np, bool nonlin, int soff, hipStream_t s)
 {
     if (a.plasma || a.pcur)
-        launch_march_p<T, RES, true>(a, dev, np, nonlin, s);
+        launch_march_p<T, RES, true>(a, dev, np, nonlin, soff, s);
     else
-        launch_march_p<T, RES, false>(a, dev, np, nonlin, s);
+        launch_march_p<T, RES, false>(a, dev, np, nonlin, soff, s);
 }
 
 // The file is compiled once per storage form (MPX_FORM 0: float64, 1: float32, 2: float32 +
@@ -945,40 +946,40 @@ static void launch_march_t(const PassArgs<T> &a, const PassArgs<T> *dev, int np,
 #error "MPX_FORM selects the storage form this object holds"
 #endif
 template <typename T, bool RES>
-void launch_pass_form(const PassArgs<T> &a, const PassArgs<T> *dev, int np, bool nonlin, hipStream_t s)
+void launch_pass_form(const PassArgs<T> &a, const PassArgs<T> *dev, int np, bool nonlin, int soff, hipStream_t s)
 {
     if (a.kernel == 1)
-        launch_march_t<T, RES>(a, dev, np, nonlin, s);
+        launch_march_t<T, RES>(a, dev, np, nonlin, soff, s);
     else
-        launch_pass_t<T, RES>(a, dev, np, nonlin, s);
+        launch_pass_t<T, RES>(a, dev, np, nonlin, soff, s);
 }
 #if MPX_FORM == 0
-template void launch_pass_form<double, false>(const PassArgs<double> &, const PassArgs<double> *, int, bool,
+template void launch_pass_form<double, false>(const PassArgs<double> &, const PassArgs<double> *, int, bool, int,
                                               hipStream_t);
-extern template void launch_pass_form<float, false>(const PassArgs<float> &, const PassArgs<float> *, int, bool,
+extern template void launch_pass_form<float, false>(const PassArgs<float> &, const PassArgs<float> *, int, bool, int,
                                                     hipStream_t);
-extern template void launch_pass_form<float, true>(const PassArgs<float> &, const PassArgs<float> *, int, bool,
+extern template void launch_pass_form<float, true>(const PassArgs<float> &, const PassArgs<float> *, int, bool, int,
                                                    hipStream_t);
 template <>
-void launch_pass<double>(const PassArgs<double> &a, const PassArgs<double> *dev, int np, bool nonlin,
+void launch_pass<double>(const PassArgs<double> &a, const PassArgs<double> *dev, int np, bool nonlin, int soff,
                          hipStream_t s)
 {
-    launch_pass_form<double, false>(a, dev, np, nonlin, s);
+    launch_pass_form<double, false>(a, dev, np, nonlin, soff, s);
 }
 template <>
-void launch_pass<float>(const PassArgs<float> &a, const PassArgs<float> *dev, int np, bool nonlin,
+void launch_pass<float>(const PassArgs<float> &a, const PassArgs<float> *dev, int np, bool nonlin, int soff,
                         hipStream_t s)
 {
     if (a.Eolo)
-        launch_pass_form<float, true>(a, dev, np, nonlin, s);
+        launch_pass_form<float, true>(a, dev, np, nonlin, soff, s);
     else
-        launch_pass_form<float, false>(a, dev, np, nonlin, s);
+        launch_pass_form<float, false>(a, dev, np, nonlin, soff, s);
 }
 #elif MPX_FORM == 1
-template void launch_pass_form<float, false>(const PassArgs<float> &, const PassArgs<float> *, int, bool,
+template void launch_pass_form<float, false>(const PassArgs<float> &, const PassArgs<float> *, int, bool, int,
                                              hipStream_t);
 #else
-template void launch_pass_form<float, true>(const PassArgs<float> &, const PassArgs<float> *, int, bool,
+template void launch_pass_form<float, true>(const PassArgs<float> &, const PassArgs<float> *, int, bool, int,
                                             hipStream_t);
 #endif
 

@@ -73,6 +73,7 @@ struct Current {
     int factory;
     int layer = -1;   // index into layers (first of the three component layers)
     int face = -1;    // CPML: index into the side's face list
+    int sheet_layer[3] = {-1, -1, -1};  // source sheet: its component layers
     // source evaluation
     mpx::SheetEval ev{};
     std::shared_ptr<mpx::GaussInjectDev> gauss;  // GaussInject: block schedule and samples
@@ -139,6 +140,10 @@ struct mpx_solver {
     std::vector<Current> ecur, hcur;
     std::vector<CpmlFace> efaces, hfaces;
     int sheets_first = 0;
+    // source sheets: `slots` steps fit the sheet planes (the last step of an evaluated window lies
+    // in slot 0, the layer itself); the window in force holds `win_n` steps, the E sheets from step
+    // win_e on and the H sheets from win_h on, and lasts no longer than the call that made it
+    int slots = 1, win_n = 0, win_e = 0, win_h = 0;
 
     double *Jt[3] = {}, *Mt[3] = {};
     bool haveJ = false, haveM = false;
@@ -506,6 +511,33 @@ static void focused_plane(const mpx_factory &f, int nx, int ny, double dx, doubl
     for (size_t q = 0; q < out.size(); ++q) out[q] = make_double2(res[q].real() / norm, res[q].imag() / norm);
 }
 
+// Planes of the source sheets.  The fused and pass paths take the sheets of several steps from
+// one launch and keep as many slots as sheet_slots gives; GaussInject's samples are scheduled
+// from the host step by step, and the other paths evaluate step by step: one slot there.
+static int sheet_planes(mpx_solver *s)
+{
+    long long points = 0;
+    bool several = s->path == MPX_PATH_FUSED || s->path == MPX_PATH_PASS;
+    for (const std::vector<Current> *list : {&s->ecur, &s->hcur})
+        for (const Current &c : *list)
+            if (c.type == CUR_INC_E || c.type == CUR_INC_H) {
+                several = several && !c.gauss;
+                for (int t = 0; t < mpx::sheet_tasks(c.ev); ++t) points += mpx::sheet_points(c.ev, t);
+            }
+    s->slots = several ? mpx::sheet_slots(points) : 1;
+    int rc = MPX_OK;
+    for (std::vector<Current> *list : {&s->ecur, &s->hcur})
+        for (Current &c : *list)
+            if (c.type == CUR_INC_E || c.type == CUR_INC_H)
+                for (int w = 0; w < 3; ++w) {
+                    Layer &L = s->layers[c.sheet_layer[w]];
+                    if (!L.comp[0]) L.comp[0] = s->dalloc<double>(L.count() * s->slots, rc);
+                    if (rc) return rc;
+                    c.ev.sheet.J[w] = (double *)L.comp[0];
+                }
+    return MPX_OK;
+}
+
 // ---------------------------------------------------------------------------------------
 // C ABI
 // ---------------------------------------------------------------------------------------
@@ -846,12 +878,6 @@ static int build(mpx_solver *s, const mpx_desc *desc)
                     int l2 = add_border_layer(s, nm[2], c.dir, 1, distance);
                     if (l0 < 0 || l1 < 0 || l2 < 0) continue;
                     c.layer = l0;
-                    int lc[3] = {l0, l1, l2};
-                    for (int w = 0; w < 3; ++w)
-                        if (!s->layers[lc[w]].comp[0]) {
-                            s->layers[lc[w]].comp[0] = s->dalloc<double>(s->layers[lc[w]].count(), rc);
-                            if (rc) return rc;
-                        }
                     mpx::SheetEval &ev = c.ev;
                     ev.isH = isH ? 1 : 0;
                     // src/incsource.t:54 (E: offset -1) and :126 (H: +1 for east/north/up, else 0)
@@ -862,7 +888,7 @@ static int build(mpx_solver *s, const mpx_desc *desc)
                     ev.nx2 = g.n[0] + 2;
                     ev.ny2 = g.n[1] + 2;
                     ev.sheet.kp = s->layers[l0].lo[2];
-                    for (int w = 0; w < 3; ++w) ev.sheet.J[w] = (double *)s->layers[lc[w]].comp[0];
+                    for (int w = 0; w < 3; ++w) c.sheet_layer[w] = w == 0 ? l0 : (w == 1 ? l1 : l2);
                     if (f.kind == MPX_FACTORY_GAUSS_INJECT) {
                         ev.kind = 4;
                         if (f.gsize_t < 2 || !(f.eps > 0))
@@ -965,6 +991,7 @@ static int build(mpx_solver *s, const mpx_desc *desc)
         if ((rc = init_side(s->hcur, true)) != MPX_OK) return rc;
         if ((int)s->efaces.size() > mpx::kMaxFaces || (int)s->hfaces.size() > mpx::kMaxFaces)
             return fail(MPX_ERR_UNSUPPORTED, "too many CPML faces");
+        if ((rc = sheet_planes(s)) != MPX_OK) return rc;
         int nse = 0, nsh = 0;
         for (auto &c : s->ecur) nse += c.type == CUR_INC_E;
         for (auto &c : s->hcur) nsh += c.type == CUR_INC_H;
@@ -1262,20 +1289,67 @@ static int sheet_time(mpx_solver *s, Current &c, int t)
     }
     return MPX_OK;
 }
-static int sheet_time(mpx_solver *s, Current &c) { return sheet_time(s, c, s->time); }
+
+// one current's sheet at step t, into slot 0
+static int eval_sheet(mpx_solver *s, Current &c, int t)
+{
+    int rc = sheet_time(s, c, t);
+    if (rc) return rc;
+    s->win_n = 0;
+    s->tick(K_SHEET);
+    if (c.type == CUR_INC_H)
+        mpx::launch_sheet_steps(nullptr, 0, 0, &c.ev, t, 1, s->ft, s->stream);
+    else
+        mpx::launch_sheet_steps(&c.ev, t, 1, nullptr, 0, 0, s->ft, s->stream);
+    s->tock();
+    MPX_LAUNCHED("sheet evaluation");
+    return MPX_OK;
+}
 
 // the sheets of one side at step t (the step counter of the step they belong to)
 static int eval_sheets(mpx_solver *s, std::vector<Current> &list, int type, int t)
 {
     for (Current &c : list)
         if (c.type == type) {
-            int rc = sheet_time(s, c, t);
+            int rc = eval_sheet(s, c, t);
             if (rc) return rc;
+        }
+    return MPX_OK;
+}
+
+// Makes the E sheets of step te and the H sheets of step th available and returns (soff) the
+// element offset of their slot in the sheet planes.  Outside the window in force it evaluates a
+// new one, of at most `ahead` steps (what the call in progress still takes, counted from these)
+// and the slots there are.  Sources on one plane share its layer, the later one's values stand:
+// one launch per source, in list order.
+static int sheets_at(mpx_solver *s, int te, int th, int ahead, int *soff)
+{
+    const int plane = (s->g.n[0] + 2) * (s->g.n[1] + 2);
+    int q = te - s->win_e;
+    if (!(s->win_n && q >= 0 && q < s->win_n && th - s->win_h == q)) {
+        const int n = std::max(1, std::min(ahead, s->slots));
+        for (int f = 0; f < s->d.n_factories; ++f) {
+            Current *cur[2] = {nullptr, nullptr};
+            for (Current &c : s->ecur)
+                if (c.type == CUR_INC_E && c.factory == f) cur[0] = &c;
+            for (Current &c : s->hcur)
+                if (c.type == CUR_INC_H && c.factory == f) cur[1] = &c;
+            if (!cur[0] && !cur[1]) continue;
+            for (int side = 0; side < 2; ++side)
+                if (cur[side])
+                    if (int rc = sheet_time(s, *cur[side], side ? th : te)) return rc;
             s->tick(K_SHEET);
-            mpx::launch_sheet_eval(c.ev, s->ft, s->stream);
+            mpx::launch_sheet_steps(cur[0] ? &cur[0]->ev : nullptr, te, n, cur[1] ? &cur[1]->ev : nullptr, th, n, s->ft,
+                                    s->stream);
             s->tock();
             MPX_LAUNCHED("sheet evaluation");
         }
+        s->win_n = n;
+        s->win_e = te;
+        s->win_h = th;
+        q = 0;
+    }
+    *soff = (s->win_n - 1 - q) * plane;
     return MPX_OK;
 }
 
@@ -1449,16 +1523,16 @@ static const StepArgs<T> *dev_args(mpx_solver *s, const StepArgs<T> &a, int side
 // The E half (E-side sheets at step t, fused E kernel) or the B half (H-side sheets at step t,
 // fused B kernel) of step t on the fused path.
 template <typename T>
-static int fused_half_t(mpx_solver *s, bool hside)
+static int fused_half_t(mpx_solver *s, bool hside, int soff)
 {
     StepArgs<T> a = step_args<T>(s, hside);
     const StepArgs<T> *d = dev_args(s, a, hside ? 1 : 0);
     if (!d) return fail(MPX_ERR_HIP, "argument upload failed");
     s->tick(hside ? K_FUSED_B : K_FUSED_E);
     if (hside)
-        mpx::launch_fused_B<T>(a, d, s->stream);
+        mpx::launch_fused_B<T>(a, d, soff, s->stream);
     else
-        mpx::launch_fused_E<T>(a, d, s->np, s->nonlin, s->stream);
+        mpx::launch_fused_E<T>(a, d, s->np, s->nonlin, soff, s->stream);
     s->tock();
     MPX_LAUNCHED(hside ? "fused B" : "fused E");
     return MPX_OK;
@@ -1468,7 +1542,7 @@ static int fused_half(mpx_solver *s, bool hside, int t)
 {
     int rc = eval_sheets(s, hside ? s->hcur : s->ecur, hside ? CUR_INC_H : CUR_INC_E, t);
     if (rc) return rc;
-    return s->esz == 8 ? fused_half_t<double>(s, hside) : fused_half_t<float>(s, hside);
+    return s->esz == 8 ? fused_half_t<double>(s, hside, 0) : fused_half_t<float>(s, hside, 0);
 }
 
 template <typename T>
@@ -1581,7 +1655,7 @@ static void swap_pass_buffers(mpx_solver *s)
 }
 
 template <typename T>
-static int pass_launch_t(mpx_solver *s)
+static int pass_launch_t(mpx_solver *s, int soff)
 {
     const mpx::PassArgs<T> a = pass_args<T>(s);
     if (a.kernel == 0 && (!a.zper || a.plasma || a.pcur))
@@ -1605,7 +1679,7 @@ static int pass_launch_t(mpx_solver *s)
             return fail(MPX_ERR_HIP, "argument upload failed");
     }
     s->tick(K_PASS);
-    mpx::launch_pass<T>(a, (const mpx::PassArgs<T> *)s->d_pargs[side], s->np, s->nonlin, s->stream);
+    mpx::launch_pass<T>(a, (const mpx::PassArgs<T> *)s->d_pargs[side], s->np, s->nonlin, soff, s->stream);
     s->tock();
     MPX_LAUNCHED("pass");
     return MPX_OK;
@@ -1614,16 +1688,15 @@ static int pass_launch_t(mpx_solver *s)
 // One step on the pass path.  Settled state at time t (E^t, B^t): the E half of step t.
 // Pending state at time t (E^t, B^(t-1)): one pass, the B half of step t - 1 (H-side sheets
 // at t - 1) and the E half of step t (E-side sheets at t).  Either way the state is pending at
-// time t + 1 afterwards.
-static int pass_step(mpx_solver *s)
+// time t + 1 afterwards.  ahead: steps the call in progress still takes, this one included.
+static int pass_step(mpx_solver *s, int ahead)
 {
-    int rc;
+    int rc, soff;
     if (!s->pending) {
         if ((rc = fused_half(s, false, s->time))) return rc;
     } else {
-        if ((rc = eval_sheets(s, s->hcur, CUR_INC_H, s->time - 1))) return rc;
-        if ((rc = eval_sheets(s, s->ecur, CUR_INC_E, s->time))) return rc;
-        rc = s->esz == 8 ? pass_launch_t<double>(s) : pass_launch_t<float>(s);
+        if ((rc = sheets_at(s, s->time, s->time - 1, ahead, &soff))) return rc;
+        rc = s->esz == 8 ? pass_launch_t<double>(s, soff) : pass_launch_t<float>(s, soff);
         if (rc) return rc;
         swap_pass_buffers(s);
     }
@@ -1644,10 +1717,11 @@ static int settle(mpx_solver *s)
 }
 
 // one full step: FDTD_PLRCSolver::stepScheme (src/fdtd_plrc.t:127-168) or the plain/nl/disp
-// stepScheme (src/fdtd_plain.cpp:31-35)
-static int step_once(mpx_solver *s)
+// stepScheme (src/fdtd_plain.cpp:31-35); ahead: steps the call in progress still takes, this one
+// included
+static int step_once(mpx_solver *s, int ahead)
 {
-    int rc;
+    int rc, soff;
     if (!s->plrc) {
         mpx::SimpleArgs a = simple_args(s);
         s->tick(K_SIMPLE_E);
@@ -1678,11 +1752,7 @@ static int step_once(mpx_solver *s)
                 mpx::launch_ref_plasma_current(ae, s->stream);
                 MPX_LAUNCHED("plasma current");
             } else {
-                if ((rc = sheet_time(s, c))) return rc;
-                s->tick(K_SHEET);
-                mpx::launch_sheet_eval(c.ev, s->ft, s->stream);
-                s->tock();
-                MPX_LAUNCHED("sheet E");
+                if ((rc = eval_sheet(s, c, s->time))) return rc;
             }
         }
         if (s->haveJ) {
@@ -1707,11 +1777,7 @@ static int step_once(mpx_solver *s)
                 s->tock();
                 MPX_LAUNCHED("cpml H");
             } else {
-                if ((rc = sheet_time(s, c))) return rc;
-                s->tick(K_SHEET);
-                mpx::launch_sheet_eval(c.ev, s->ft, s->stream);
-                s->tock();
-                MPX_LAUNCHED("sheet H");
+                if ((rc = eval_sheet(s, c, s->time))) return rc;
             }
         }
         if (s->haveM) {
@@ -1729,8 +1795,7 @@ static int step_once(mpx_solver *s)
         MPX_LAUNCHED("stepB");
         if ((rc = wrap_group<double>(s, s->B, K_WRAP_B))) return rc;
     } else if (s->path == MPX_PATH_SWEEP) {
-        if ((rc = eval_sheets(s, s->ecur, CUR_INC_E, s->time))) return rc;
-        if ((rc = eval_sheets(s, s->hcur, CUR_INC_H, s->time))) return rc;
+        if ((rc = sheets_at(s, s->time, s->time, 1, &soff))) return rc;
         s->tick(K_SWEEP);
         if (s->esz == 8)
             mpx::launch_sweep<double>(sweep_args<double>(s), s->np, s->nonlin, s->stream);
@@ -1740,8 +1805,10 @@ static int step_once(mpx_solver *s)
         MPX_LAUNCHED("sweep");
         swap_sweep_buffers(s);
     } else {
-        if ((rc = fused_half(s, false, s->time))) return rc;
-        if ((rc = fused_half(s, true, s->time))) return rc;
+        if ((rc = sheets_at(s, s->time, s->time, ahead, &soff))) return rc;
+        for (int side = 0; side < 2; ++side)
+            if ((rc = s->esz == 8 ? fused_half_t<double>(s, side, soff) : fused_half_t<float>(s, side, soff)))
+                return rc;
     }
     s->time++;
     return record_probes(s);
@@ -1780,8 +1847,9 @@ int mpx_step(mpx_solver *s, int nsteps)
         int rc = settle(s);
         if (rc) return rc;
     }
+    s->win_n = 0;
     for (int n = 0; n < nsteps; ++n) {
-        int rc = pass ? pass_step(s) : step_once(s);
+        int rc = pass ? pass_step(s, nsteps - n) : step_once(s, nsteps - n);
         if (rc) return rc;
     }
     return MPX_OK;
@@ -1831,9 +1899,7 @@ int mpx_step_init(mpx_solver *s)
             mpx::launch_ref_cpml(ah, c.face, true, s->stream);
             MPX_LAUNCHED("cpml H");
         } else {
-            if ((rc = sheet_time(s, c))) return rc;
-            mpx::launch_sheet_eval(c.ev, s->ft, s->stream);
-            MPX_LAUNCHED("sheet H");
+            if ((rc = eval_sheet(s, c, s->time))) return rc;
         }
     }
     return MPX_OK;
@@ -2668,9 +2734,10 @@ struct mpx_batch {
     void *d_pargs[2] = {nullptr, nullptr};  // x-march argument tables per arrangement
     mpx::BatchRun *d_pruns = nullptr;
     int ptotal = 0;
-    mpx::SheetEval *d_sheets = nullptr;
+    mpx::SheetTask *d_sheets = nullptr;  // the components of every run's sheets
     int *d_sheet_first = nullptr;
     int nsheets = 0, sheet_blocks = 0;
+    bool pulses = true;  // every sheet is a short pulse
     int *d_time = nullptr;
     mpx::FaddeevaTables ft{};
     hipGraphExec_t graph[2] = {nullptr, nullptr};
@@ -2849,8 +2916,8 @@ static void batch_fused(mpx_batch *b, int side, int par)
 static void batch_sheets(mpx_batch *b, int j, int hshift, int sides)
 {
     if (b->nsheets)
-        mpx::launch_sheet_eval_batch(b->d_sheets, b->d_sheet_first, b->nsheets, b->sheet_blocks, b->ft, b->d_time, j,
-                                     b->stream, hshift, sides);
+        mpx::launch_sheet_eval_batch(b->d_sheets, b->d_sheet_first, b->nsheets, b->sheet_blocks, b->pulses, b->ft,
+                                     b->d_time, j, b->stream, hshift, sides);
 }
 
 // enqueue step j of a sequence that starts at the device counter, with argument parity par.
@@ -3035,23 +3102,25 @@ int mpx_batch_create(const mpx_desc *descs, int nruns, mpx_batch **out)
         if (s->time != 0) return bail(fail(MPX_ERR_INVALID, "batched runs start at time 0"));
     }
     // source sheets of all runs
-    std::vector<mpx::SheetEval> sheets;
+    std::vector<mpx::SheetTask> sheets;
     std::vector<int> first;
     for (mpx_solver *s : b->runs)
         for (int side = 0; side < 2; ++side)
             for (const Current &c : side ? s->hcur : s->ecur)
-                if (c.type == (side ? CUR_INC_H : CUR_INC_E)) {
-                    first.push_back(b->sheet_blocks);
-                    sheets.push_back(c.ev);
-                    b->sheet_blocks += c.ev.nx2 * ((c.ev.ny2 + 63) / 64);
-                }
+                if (c.type == (side ? CUR_INC_H : CUR_INC_E))
+                    for (int t = 0; t < mpx::sheet_tasks(c.ev); ++t) {
+                        first.push_back(b->sheet_blocks);
+                        sheets.push_back({c.ev, t, mpx::sheet_points(c.ev, t)});
+                        b->sheet_blocks += (sheets.back().points + 63) / 64;
+                        b->pulses = b->pulses && c.ev.kind == 1;
+                    }
     b->nsheets = (int)sheets.size();
     if (b->alloc((void **)&b->d_time, sizeof(int))) return bail(MPX_ERR_NOMEM);
     if (b->nsheets) {
-        if (b->alloc((void **)&b->d_sheets, sheets.size() * sizeof(mpx::SheetEval)) ||
+        if (b->alloc((void **)&b->d_sheets, sheets.size() * sizeof(mpx::SheetTask)) ||
             b->alloc((void **)&b->d_sheet_first, first.size() * sizeof(int)))
             return bail(MPX_ERR_NOMEM);
-        if (hipMemcpyAsync(b->d_sheets, sheets.data(), sheets.size() * sizeof(mpx::SheetEval), hipMemcpyHostToDevice,
+        if (hipMemcpyAsync(b->d_sheets, sheets.data(), sheets.size() * sizeof(mpx::SheetTask), hipMemcpyHostToDevice,
                            b->stream) != hipSuccess ||
             hipMemcpyAsync(b->d_sheet_first, first.data(), first.size() * sizeof(int), hipMemcpyHostToDevice,
                            b->stream) != hipSuccess)
@@ -3323,6 +3392,7 @@ int mpx_adjoint_grad(mpx_solver *s, const mpx_objective *obj, int nsteps, int K,
     double *dJ = mem.get(1, st);
     if (!dJ) return fail(MPX_ERR_NOMEM, "adjoint allocation failed");
     const int t0 = s->time;
+    s->win_n = 0;
     const int nseg = (nsteps + K - 1) / K;
     StateRef cur = state_of(s);
     auto snapshot = [&](std::vector<double *> &dst) -> int {
@@ -3346,7 +3416,7 @@ int mpx_adjoint_grad(mpx_solver *s, const mpx_objective *obj, int nsteps, int K,
     // forward pass: objective after every step, a checkpoint at the start of every segment
     for (int n = 0; n < nsteps; ++n) {
         if (grad && n % K == 0 && (rc = snapshot(ckpt[n / K]))) return rc;
-        if ((rc = step_once(s))) return rc;
+        if ((rc = step_once(s, nsteps - n))) return rc;
         double *E[3] = {(double *)s->E[0], (double *)s->E[1], (double *)s->E[2]};
         mpx::launch_plane_objective(s->g, E, obj->plane_k, obj->weight, dJ, st);
         MPX_LAUNCHED("plane objective");
@@ -3420,6 +3490,7 @@ int mpx_adjoint_grad(mpx_solver *s, const mpx_objective *obj, int nsteps, int K,
         const int len = std::min(K, nsteps - seg * K);
         if ((rc = restore(ckpt[seg]))) return rc;
         s->time = t0 + seg * K;
+        s->win_n = 0;
         auto keepE = [&](int m) -> int {
             for (int c = 0; c < 3; ++c)
                 MPX_HIP(hipMemcpyAsync(hist[m][c], s->E[c], s->cells * 8, hipMemcpyDeviceToDevice, st));
@@ -3427,7 +3498,7 @@ int mpx_adjoint_grad(mpx_solver *s, const mpx_objective *obj, int nsteps, int K,
         };
         if ((rc = keepE(0))) return rc;
         for (int m = 1; m <= len; ++m) {
-            if ((rc = step_once(s))) return rc;
+            if ((rc = step_once(s, len - m + 1))) return rc;
             if ((rc = keepE(m))) return rc;
         }
         for (int m = len - 1; m >= 0; --m) {

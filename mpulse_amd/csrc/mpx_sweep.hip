@@ -146,7 +146,7 @@ __device__ __forceinline__ void sweep_tile(const SweepArgs<T> &a, int tz, int ty
             bcur[r][2] = bz;
             const bool store = own[r] && p <= i1;
             double jx = 0.0, jy = 0.0, jz = 0.0;
-            if (a.sheets_first) add_sheet_planes(a.sheet, a.nsheets, g.py, pp, j, kk, jx, jy, jz);
+            if (a.sheets_first) add_sheet_planes(a.sheet, a.nsheets, g.py, pp, j, kk, 0, jx, jy, jz);
             if (CPML) {
                 // E auxiliaries, list order N,S (y), E,W (x), U,D (z), high face first
 #pragma unroll
@@ -183,7 +183,7 @@ __device__ __forceinline__ void sweep_tile(const SweepArgs<T> &a, int tz, int ty
                     }
                 }
             }
-            if (!a.sheets_first) add_sheet_planes(a.sheet, a.nsheets, g.py, pp, j, kk, jx, jy, jz);
+            if (!a.sheets_first) add_sheet_planes(a.sheet, a.nsheets, g.py, pp, j, kk, 0, jx, jy, jz);
             double ex = (double)ce[r][0], ey = (double)ce[r][1], ez = (double)ce[r][2];
             unsigned fl = 0;
             plrc_e_update_pp<NP, NONLIN, true>(ex, ey, ez, dBz_y, dBy_z, dBx_z, dBz_x, dBy_x, dBx_y,
@@ -222,7 +222,7 @@ __device__ __forceinline__ void sweep_tile(const SweepArgs<T> &a, int tz, int ty
                 const double dEz_x = ecur[r][2] - ez;
                 const double dEy_x = ecur[r][1] - ey;
                 double mx = 0.0, my = 0.0, mz = 0.0;
-                if (a.sheets_first) add_sheet_planes(a.hsheet, a.nhsheets, g.py, pb, j, kk, mx, my, mz);
+                if (a.sheets_first) add_sheet_planes(a.hsheet, a.nhsheets, g.py, pb, j, kk, 0, mx, my, mz);
                 if (CPML) {
 #pragma unroll
                     for (int d = 0; d < 3; ++d) {
@@ -256,7 +256,7 @@ __device__ __forceinline__ void sweep_tile(const SweepArgs<T> &a, int tz, int ty
                         }
                     }
                 }
-                if (!a.sheets_first) add_sheet_planes(a.hsheet, a.nhsheets, g.py, pb, j, kk, mx, my, mz);
+                if (!a.sheets_first) add_sheet_planes(a.hsheet, a.nhsheets, g.py, pb, j, kk, 0, mx, my, mz);
                 const double kdx = a.ikdH[0][pb], kdy = a.ikdH[1][j];
                 a.Bn[0][c] = (T)(bprev[r][0] + a.dt * ((dEy_z * kdz_h - dEz_y * kdy) + mx));
                 a.Bn[1][c] = (T)(bprev[r][1] + a.dt * ((dEz_x * kdx - dEx_z * kdz_h) + my));

@@ -138,6 +138,12 @@ struct SheetEval {
     GaussSheetParams gauss;
 };
 
+// one separately evaluated component of a sheet in a batch's list (mpx_sheet.hip)
+struct SheetTask {
+    SheetEval ev;
+    int task, points;
+};
+
 // PLRC pole constants (PLRCData, src/fdtd_plrc.h:71-78) of the active poles, precomputed on the
 // host with the formulas of src/fdtd_plrc.t:198-216.
 struct PoleConsts {
