@@ -528,21 +528,33 @@ void launch_hbm_copy(const void *src, void *dst, size_t bytes, hipStream_t s)
                        (double2 *)dst, n);
 }
 
+// Coordinate c of dimension d as the grid holds it: where bit d of wrapmask is set, a ghost (0 or
+// N + 1) reads its periodic image (N or 1), which is what the ghost holds once the wrap has run.
+// Reading the image costs the pack kernels nothing; running the wrap first took six launches a
+// group of E or B (twelve with residual words), 36 of them and 0.15 of 0.49 ms for the six fields
+// of a 24^3 grid.
+__device__ __forceinline__ int image(const GridDims &g, int wrapmask, int d, int c)
+{
+    if ((wrapmask >> d) & 1) c = c == 0 ? g.n[d] : (c == g.n[d] + 1 ? 1 : c);
+    return c;
+}
+
 // A grid over the storage box 0..N+1 in the order of the reference's Grid (x fastest), as
 // float64: dst[(k (ny+2) + j) (nx+2) + i] = src(i, j, k), the form FieldDiag hands to its HDF5
 // stream.  A block transposes a 32 (z) x 32 (x) tile of one y row through LDS, so that both
 // the reads (z contiguous) and the writes (x contiguous) are coalesced.
 template <typename T>
 __global__ __launch_bounds__(256) void k_pack_xfast(GridDims g, const T *__restrict__ src, const unsigned *lo, int q,
-                                                    double *__restrict__ dst)
+                                                    int wrapmask, double *__restrict__ dst)
 {
     __shared__ double tile[32][33];
     const int nx2 = g.n[0] + 2, ny2 = g.n[1] + 2, nz2 = g.n[2] + 2;
     const int k0 = blockIdx.x * 32, i0 = blockIdx.y * 32, j = blockIdx.z;
+    const int js = image(g, wrapmask, 1, j);
     for (int r = threadIdx.y; r < 32; r += 8) {
         const int i = i0 + r, k = k0 + threadIdx.x;
         if (i < nx2 && k < nz2) {
-            const size_t c = g.at(i, j, k);
+            const size_t c = g.at(image(g, wrapmask, 0, i), js, image(g, wrapmask, 2, k));
             tile[r][threadIdx.x] = lo ? res_decode((float)src[c], lo[c], q) : (double)src[c];
         }
     }
@@ -554,13 +566,84 @@ __global__ __launch_bounds__(256) void k_pack_xfast(GridDims g, const T *__restr
 }
 
 template <typename T>
-void launch_pack_xfast(const GridDims &g, const T *src, double *dst, hipStream_t s, const unsigned *lo, int q)
+void launch_pack_xfast(const GridDims &g, const T *src, double *dst, hipStream_t s, int wrapmask, const unsigned *lo,
+                       int q)
 {
     dim3 grd((g.n[2] + 2 + 31) / 32, (g.n[0] + 2 + 31) / 32, g.n[1] + 2);
-    hipLaunchKernelGGL(k_pack_xfast<T>, grd, dim3(32, 8), 0, s, g, src, lo, q, dst);
+    hipLaunchKernelGGL(k_pack_xfast<T>, grd, dim3(32, 8), 0, s, g, src, lo, q, wrapmask, dst);
 }
-template void launch_pack_xfast<float>(const GridDims &, const float *, double *, hipStream_t, const unsigned *, int);
-template void launch_pack_xfast<double>(const GridDims &, const double *, double *, hipStream_t, const unsigned *, int);
+template void launch_pack_xfast<float>(const GridDims &, const float *, double *, hipStream_t, int, const unsigned *,
+                                       int);
+template void launch_pack_xfast<double>(const GridDims &, const double *, double *, hipStream_t, int, const unsigned *,
+                                        int);
+
+// Planes i0 .. of the storage box in z-fastest order as float64, the form of mpx_get_field /
+// mpx_set_field: box[((i - i0) (ny+2) + j) (nz+2) + k] <-> the grid's cell (i, j, k).  PSI: the grid is component 0 of a
+// pole's accumulator block shifted to its component (psi_at), and q is the part (0 re, 1 im).
+// Unpacking into float32 + residual storage replaces slot q of the cell's residual word.  The
+// conversion and the padding were a loop over the cells on one host core (0.25 ms of the 0.33 ms
+// of a 50 x 42 x 58 read, 3 s of a 514^3 one); here they run at the copy rate and the host
+// buffer takes one copy.
+template <typename T, bool PSI>
+__global__ __launch_bounds__(256) void k_pack_box(GridDims g, const T *__restrict__ src, const unsigned *lo, int q,
+                                                  int wrapmask, int i0, double *__restrict__ box)
+{
+    const int k = blockIdx.x * 64 + threadIdx.x, j = blockIdx.y * 4 + threadIdx.y, i = i0 + blockIdx.z;
+    if (k > g.n[2] + 1 || j > g.n[1] + 1) return;
+    const size_t c = g.at(image(g, wrapmask, 0, i), image(g, wrapmask, 1, j), image(g, wrapmask, 2, k));
+    double v;
+    if (PSI)
+        v = (double)src[2 * psi_at(c) + q];
+    else
+        v = lo ? res_decode((float)src[c], lo[c], q) : (double)src[c];
+    box[((size_t)blockIdx.z * (g.n[1] + 2) + j) * (g.n[2] + 2) + k] = v;
+}
+
+template <typename T, bool PSI>
+__global__ __launch_bounds__(256) void k_unpack_box(GridDims g, const double *__restrict__ box, T *__restrict__ dst,
+                                                    unsigned *lo, int q, int i0)
+{
+    const int k = blockIdx.x * 64 + threadIdx.x, j = blockIdx.y * 4 + threadIdx.y, i = i0 + blockIdx.z;
+    if (k > g.n[2] + 1 || j > g.n[1] + 1) return;
+    const size_t c = g.at(i, j, k);
+    const double v = box[((size_t)blockIdx.z * (g.n[1] + 2) + j) * (g.n[2] + 2) + k];
+    if (PSI)
+        dst[2 * psi_at(c) + q] = (T)v;
+    else if (lo) {
+        unsigned w = 0;
+        dst[c] = (T)res_encode(v, w, q);
+        lo[c] = (lo[c] & ~(0x3ffu << (10 * q))) | w;
+    } else
+        dst[c] = (T)v;
+}
+
+static dim3 box_grid(const GridDims &g, int ni) { return dim3((g.n[2] + 2 + 63) / 64, (g.n[1] + 2 + 3) / 4, ni); }
+
+template <typename T>
+void launch_pack_box(const GridDims &g, const T *src, double *box, int i0, int ni, hipStream_t s, bool psi, int wrapmask,
+                     const unsigned *lo, int q)
+{
+    if (psi)
+        hipLaunchKernelGGL((k_pack_box<T, true>), box_grid(g, ni), dim3(64, 4), 0, s, g, src, lo, q, wrapmask, i0, box);
+    else
+        hipLaunchKernelGGL((k_pack_box<T, false>), box_grid(g, ni), dim3(64, 4), 0, s, g, src, lo, q, wrapmask, i0, box);
+}
+template <typename T>
+void launch_unpack_box(const GridDims &g, const double *box, T *dst, int i0, int ni, hipStream_t s, bool psi, unsigned *lo, int q)
+{
+    if (psi)
+        hipLaunchKernelGGL((k_unpack_box<T, true>), box_grid(g, ni), dim3(64, 4), 0, s, g, box, dst, lo, q, i0);
+    else
+        hipLaunchKernelGGL((k_unpack_box<T, false>), box_grid(g, ni), dim3(64, 4), 0, s, g, box, dst, lo, q, i0);
+}
+template void launch_pack_box<float>(const GridDims &, const float *, double *, int, int, hipStream_t, bool, int,
+                                     const unsigned *, int);
+template void launch_pack_box<double>(const GridDims &, const double *, double *, int, int, hipStream_t, bool, int,
+                                      const unsigned *, int);
+template void launch_unpack_box<float>(const GridDims &, const double *, float *, int, int, hipStream_t, bool, unsigned *,
+                                       int);
+template void launch_unpack_box<double>(const GridDims &, const double *, double *, int, int, hipStream_t, bool, unsigned *,
+                                        int);
 
 // One record of a sampler: the value at storage cell c (dim < 0) or the len = N[dim] + 2 values
 // of the storage line through c along dim, as float64.  A coordinate of a dimension in
@@ -575,9 +658,7 @@ __global__ __launch_bounds__(256) void k_sample_gather(GridDims g, const T *__re
     if (q >= len) return;
     int c[3] = {c0, c1, c2};
     if (dim >= 0) c[dim] = q;
-    for (int d = 0; d < 3; ++d)
-        if ((wrapmask >> d) & 1) c[d] = c[d] == 0 ? g.n[d] : (c[d] == g.n[d] + 1 ? 1 : c[d]);
-    const size_t at = g.at(c[0], c[1], c[2]);
+    const size_t at = g.at(image(g, wrapmask, 0, c[0]), image(g, wrapmask, 1, c[1]), image(g, wrapmask, 2, c[2]));
     dst[q] = lo ? res_decode((float)src[at], lo[at], qc) : (double)src[at];
 }
 

@@ -103,10 +103,18 @@ template <typename T>
 void launch_probe(const ProbeArgs<T> &a, double *row, hipStream_t s);
 size_t energy_partials(const GridDims &g);
 void launch_hbm_copy(const void *src, void *dst, size_t bytes, hipStream_t s);
-// lo / q: the residual words and slot of a float32 + residual grid (null otherwise)
+// lo / q: the residual words and slot of a float32 + residual grid (null otherwise); wrapmask: the
+// dimensions whose ghosts are read as their periodic images
 template <typename T>
-void launch_pack_xfast(const GridDims &g, const T *src, double *dst, hipStream_t s, const unsigned *lo = nullptr,
-                       int q = 0);
+void launch_pack_xfast(const GridDims &g, const T *src, double *dst, hipStream_t s, int wrapmask,
+                       const unsigned *lo = nullptr, int q = 0);
+// planes i0 .. i0 + ni - 1 of the storage box, z fastest, as float64; psi: an accumulator component, part q (0 re, 1 im)
+template <typename T>
+void launch_pack_box(const GridDims &g, const T *src, double *box, int i0, int ni, hipStream_t s, bool psi, int wrapmask,
+                     const unsigned *lo = nullptr, int q = 0);
+template <typename T>
+void launch_unpack_box(const GridDims &g, const double *box, T *dst, int i0, int ni, hipStream_t s, bool psi,
+                       unsigned *lo = nullptr, int q = 0);
 template <typename T>
 void launch_sample_gather(const GridDims &g, const T *src, int dim, const int *c, int len, int wrapmask, double *dst,
                          hipStream_t s, const unsigned *lo = nullptr, int q = 0);

@@ -173,6 +173,8 @@ struct mpx_solver {
     // 0 = one cell per thread (k_pass)
     // seg 0: 16 planes, fewer where the grid has too few tiles to fill the chip
     int pass_kernel = 1, march_seg = 0, march_rows = 0;  // rows 0: chosen per kernel variant
+    double *d_box = nullptr;       // staging of mpx_get_field / mpx_set_field: box_planes x planes
+    int box_planes = 0;
     double *d_stage = nullptr;     // x-fastest float64 copy of one grid for mpx_fetch_field
     // sweep path: second set of buffers (swapped with the first after every step)
     void *E2[3] = {}, *B2[3] = {};
@@ -1960,6 +1962,62 @@ static const unsigned *res_of(const mpx_solver *s, const void *ptr, int *slot)
     return nullptr;
 }
 
+// the dimensions whose ghosts in grid ptr stand for their periodic images: the periodic ones of E
+// and B on the paths that wrap by index arithmetic
+static int image_mask(const mpx_solver *s, const void *ptr)
+{
+    int mask = 0;
+    if (s->plrc && s->path != MPX_PATH_REFERENCE)
+        for (int q = 0; q < 3; ++q)
+            if (ptr == s->E[q] || ptr == s->B[q])
+                for (int d = 0; d < 3; ++d) mask |= s->periodic[d] ? 1 << d : 0;
+    return mask;
+}
+
+// The storage box of the grid at ptr to `out`, or from `in`, as float64 with z fastest: slabs of x
+// planes go through a device buffer of at most 64 MiB (one plane where that is more), packed or
+// unpacked there.
+static int box_copy(mpx_solver *s, void *ptr, size_t elem, bool isPsi, int part, double *out, const double *in)
+{
+    const GridDims &g = s->g;
+    const size_t plane = (size_t)(g.n[1] + 2) * (g.n[2] + 2);
+    const int nx2 = g.n[0] + 2;
+    if (!s->d_box) {
+        size_t n = std::max<size_t>(1, std::min<size_t>(nx2, ((size_t)1 << 23) / plane));
+        for (;; n = (n + 1) / 2) {
+            if (hipMalloc((void **)&s->d_box, n * plane * 8) == hipSuccess) break;
+            s->d_box = nullptr;
+            (void)hipGetLastError();
+            if (n == 1) return fail(MPX_ERR_NOMEM, "hipMalloc of a staging plane failed");
+        }
+        s->allocs.push_back(s->d_box);
+        s->box_planes = (int)n;
+    }
+    int slot = 0;
+    unsigned *lo = const_cast<unsigned *>(res_of(s, ptr, &slot));
+    const int q = isPsi ? part : slot, wrap = image_mask(s, ptr);
+    for (int i = 0; i < nx2; i += s->box_planes) {
+        const int ni = std::min(s->box_planes, nx2 - i);
+        if (in) {
+            MPX_HIP(hipMemcpyAsync(s->d_box, in + i * plane, ni * plane * 8, hipMemcpyHostToDevice, s->stream));
+            if (isPsi || elem == 8)
+                mpx::launch_unpack_box<double>(g, s->d_box, (double *)ptr, i, ni, s->stream, isPsi, lo, q);
+            else
+                mpx::launch_unpack_box<float>(g, s->d_box, (float *)ptr, i, ni, s->stream, false, lo, q);
+        } else {
+            if (isPsi || elem == 8)
+                mpx::launch_pack_box<double>(g, (const double *)ptr, s->d_box, i, ni, s->stream, isPsi, wrap, lo, q);
+            else
+                mpx::launch_pack_box<float>(g, (const float *)ptr, s->d_box, i, ni, s->stream, false, wrap, lo, q);
+        }
+        MPX_LAUNCHED("field packing");
+        if (out)
+            MPX_HIP(hipMemcpyAsync(out + i * plane, s->d_box, ni * plane * 8, hipMemcpyDeviceToHost, s->stream));
+    }
+    MPX_HIP(hipStreamSynchronize(s->stream));
+    return MPX_OK;
+}
+
 // host copy of a device array of `n` residual words
 static int fetch_words(mpx_solver *s, const unsigned *d, size_t n, std::vector<unsigned> &out)
 {
@@ -2100,29 +2158,7 @@ int mpx_get_field(mpx_solver *s, const char *name, double *host, size_t count)
             std::memset(host, 0, count * sizeof(double));
         return MPX_OK;
     }
-    if ((rc = materialise_ghosts(s))) return rc;
-    // an accumulator component spans its pole's block from its own offset (psi_at)
-    std::vector<unsigned char> buf(isPsi ? (mpx::psi_at(s->cells - 1) + 1) * 16 : s->cells * elem);
-    MPX_HIP(hipMemcpyAsync(buf.data(), ptr, buf.size(), hipMemcpyDeviceToHost, s->stream));
-    MPX_HIP(hipStreamSynchronize(s->stream));
-    int slot = 0;
-    const unsigned *dlo = res_of(s, ptr, &slot);
-    std::vector<unsigned> lo;
-    if (dlo && (rc = fetch_words(s, dlo, s->cells, lo))) return rc;
-    for (size_t i = 0; i < nx2; ++i)
-        for (size_t j = 0; j < ny2; ++j)
-            for (size_t k = 0; k < nz2; ++k) {
-                size_t src = g.at((int)i, (int)j, (int)k);
-                size_t dst = (i * ny2 + j) * nz2 + k;
-                if (isPsi)
-                    host[dst] = ((const double *)buf.data())[2 * mpx::psi_at(src) + part];
-                else if (elem == 8)
-                    host[dst] = ((const double *)buf.data())[src];
-                else if (dlo)
-                    host[dst] = mpx::res_decode(((const float *)buf.data())[src], lo[src], slot);
-                else
-                    host[dst] = ((const float *)buf.data())[src];
-            }
+    if ((rc = box_copy(s, ptr, elem, isPsi, part, host, nullptr))) return rc;
     if (s->path != MPX_PATH_REFERENCE) {
         if (ptr == s->d_rho)
             plasma_ghosts(s, host, 0);
@@ -2171,13 +2207,13 @@ int mpx_fetch_field(mpx_solver *s, const char *name, double *host, size_t count,
     if (!s->d_stage) {
         if (!(s->d_stage = s->dalloc<double>(count, rc))) return rc;
     }
-    if ((rc = materialise_ghosts(s))) return rc;
     int slot = 0;
     const unsigned *dlo = res_of(s, ptr, &slot);
+    const int wrap = image_mask(s, ptr);
     if (elem == 8)
-        mpx::launch_pack_xfast<double>(g, (const double *)ptr, s->d_stage, s->stream);
+        mpx::launch_pack_xfast<double>(g, (const double *)ptr, s->d_stage, s->stream, wrap);
     else
-        mpx::launch_pack_xfast<float>(g, (const float *)ptr, s->d_stage, s->stream, dlo, slot);
+        mpx::launch_pack_xfast<float>(g, (const float *)ptr, s->d_stage, s->stream, wrap, dlo, slot);
     MPX_HIP(hipGetLastError());
     MPX_HIP(hipMemcpyAsync(host, s->d_stage, count * sizeof(double), hipMemcpyDeviceToHost, s->stream));
     mpx_fetch *f = new mpx_fetch;
@@ -2242,34 +2278,7 @@ int mpx_set_field(mpx_solver *s, const char *name, const double *host, size_t co
     int rc = find_grid(s, name, &ptr, &elem, &isPsi, &part);
     if (rc) return fail(rc, std::string("unknown grid ") + name);
     if (!ptr) return fail(MPX_ERR_UNSUPPORTED, std::string("grid ") + name + " is not stored (inactive pole or Sigma)");
-    // an accumulator component spans its pole's block from its own offset (psi_at)
-    std::vector<unsigned char> buf(isPsi ? (mpx::psi_at(s->cells - 1) + 1) * 16 : s->cells * elem);
-    MPX_HIP(hipMemcpyAsync(buf.data(), ptr, buf.size(), hipMemcpyDeviceToHost, s->stream));
-    MPX_HIP(hipStreamSynchronize(s->stream));
-    int slot = 0;
-    unsigned *dlo = const_cast<unsigned *>(res_of(s, ptr, &slot));
-    std::vector<unsigned> lo;
-    if (dlo && (rc = fetch_words(s, dlo, s->cells, lo))) return rc;
-    for (size_t i = 0; i < nx2; ++i)
-        for (size_t j = 0; j < ny2; ++j)
-            for (size_t k = 0; k < nz2; ++k) {
-                size_t dst = g.at((int)i, (int)j, (int)k);
-                size_t src = (i * ny2 + j) * nz2 + k;
-                if (isPsi)
-                    ((double *)buf.data())[2 * mpx::psi_at(dst) + part] = host[src];
-                else if (elem == 8)
-                    ((double *)buf.data())[dst] = host[src];
-                else if (dlo) {
-                    unsigned w = 0;
-                    ((float *)buf.data())[dst] = mpx::res_encode(host[src], w, slot);
-                    lo[dst] = (lo[dst] & ~(0x3ffu << (10 * slot))) | w;
-                } else
-                    ((float *)buf.data())[dst] = (float)host[src];
-            }
-    MPX_HIP(hipMemcpyAsync(ptr, buf.data(), buf.size(), hipMemcpyHostToDevice, s->stream));
-    if (dlo) MPX_HIP(hipMemcpyAsync(dlo, lo.data(), lo.size() * sizeof(unsigned), hipMemcpyHostToDevice, s->stream));
-    MPX_HIP(hipStreamSynchronize(s->stream));
-    return MPX_OK;
+    return box_copy(s, ptr, elem, isPsi, part, nullptr, host);
 }
 
 int mpx_get_layer(mpx_solver *s, const char *name, int dir, double *host, size_t count, int lo[3], int hi[3])
