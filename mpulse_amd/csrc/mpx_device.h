@@ -58,6 +58,30 @@ __device__ __forceinline__ void store_once(T *p, T v)
     __builtin_nontemporal_store(v, (MPX_GLOBAL T *)p);
 }
 
+// Word at byte offset bo (per lane, 32 bits) from the wave-uniform address `base` of a row or of
+// a plane (of (ny + 2) pz words < 2^32 bytes): a scalar base and one offset register for all the
+// grids a lane reads at its cell, instead of a 64-bit address each
+template <typename T>
+__device__ __forceinline__ T ldp(const T *base, unsigned bo)
+{
+    return gld((const T *)((const char *)base + bo));
+}
+template <typename T>
+__device__ __forceinline__ void stp_once(T *base, unsigned bo, T v)
+{
+    store_once((T *)((char *)base + bo), v);
+}
+template <typename T>
+__device__ __forceinline__ T ldp_once(const T *base, unsigned bo)
+{
+    return load_once((const T *)((const char *)base + bo));
+}
+template <typename T>
+__device__ __forceinline__ void stp(T *base, unsigned bo, T v)
+{
+    gst((T *)((char *)base + bo), v);
+}
+
 // The value a neighbouring lane of the wavefront holds, by DPP: lane_prev gives lane l the
 // value of lane l - 1 (wave_shr:1), lane_next that of lane l + 1 (wave_shl:1).  Lanes of a
 // fused-kernel wave hold consecutive z cells of one row, so the z neighbour of a cell is in

@@ -307,31 +307,69 @@ void launch_init_accumulator(const StepArgs<double> &a, int np, hipStream_t s)
 }
 
 // ------------------------------------------------------------------------------------
-// fdtd-plain, fdtd-nl, fdtd-disp (periodic only; no currents)
+// fdtd-plain, fdtd-nl, fdtd-disp (no currents)
 // ------------------------------------------------------------------------------------
+//
+// Memory bound: 12 words a cell and step, fdtd-disp 27 more for its polarisations.  The
+// reference updates E over [1, N+1]^3 and B over [0, N]^3 and exchanges the ghosts after each
+// (src/fdtd_plain.cpp:54-118, src/storage.cpp:194-204); the exchange took six launches of 5 us
+// a step with four-cell rows, 30 of the 160 us of a 120x112x100 step.  Here the B kernel takes
+// E beyond N from the periodic image by index and leaves the images of E and of the new B in
+// the ghosts with the stores of the cells that own them; along a non-periodic z the update
+// covers the reference's range instead.  The ADE solver writes P of the new step over P of the
+// step before last and the host exchanges the two names, 9 words a cell less than moving P to
+// Pp.  Blocks take their tiles in XCD-contiguous slabs (xcd_tile), so the neighbour planes of
+// B and E are read from one L2.
+// Measured, fdtd-disp 120x112x100, us a step: stepD 102, stepB 29, exchange 30 before; 98, 24 and none now
+// (4.1 TB/s in stepD: 18 polarisation streams a lane, each its own pages).
 
 // E loops of FDTD_Plain / FDTD_Nonlinear / FDTD_Dispersion over [1, N+1]^3
-// (src/fdtd_plain.cpp:54-75, src/fdtd_nl.cpp:55-98, src/fdtd_disp.cpp:113-204)
-__global__ __launch_bounds__(256) void k_simple_stepD(SimpleArgs a)
+// (src/fdtd_plain.cpp:54-75, src/fdtd_nl.cpp:55-98, src/fdtd_disp.cpp:113-204); KIND 0, 1, 2.
+// E of a periodic dimension's ghost is left to the B kernel; the threads of those ghosts (all
+// kinds but plain) do what else the reference does there.
+template <int KIND>
+__global__ __launch_bounds__(256) void k_simple_stepD(SimpleArgs a, int nbx, int nby, int nbz)
 {
-    int k = blockIdx.x * 64 + threadIdx.x + 1;
-    int j = blockIdx.y * 4 + threadIdx.y + 1;
-    int i = blockIdx.z + 1;
+    constexpr int LO = KIND == 2 ? 0 : 1;  // the polarisations at coordinate 0 change buffers
+    int bx, by, bz;
+    xcd_tile(nbx, nby, nbz, bx, by, bz);
+    const int k = bx * 64 + threadIdx.x + LO, i = bz + LO;
+    const int j = __builtin_amdgcn_readfirstlane(by * 4 + (int)threadIdx.y + LO);  // one row a wave
     const GridDims &g = a.g;
     if (k > g.n[2] + 1 || j > g.n[1] + 1) return;
-    size_t c = g.at(i, j, k);
-    double *Ex = a.E[0], *Ey = a.E[1], *Ez = a.E[2];
-    const double *Bx = a.B[0], *By = a.B[1], *Bz = a.B[2];
-    double dx = a.dx, dy = a.dy, dz = a.dz, dt = a.dt;
-    double cx = (Bz[c] - Bz[g.at(i, j - 1, k)]) / dy - (By[c] - By[g.at(i, j, k - 1)]) / dz;
-    double cy = (Bx[c] - Bx[g.at(i, j, k - 1)]) / dz - (Bz[c] - Bz[g.at(i - 1, j, k)]) / dx;
-    double cz = (By[c] - By[g.at(i - 1, j, k)]) / dx - (Bx[c] - Bx[g.at(i, j - 1, k)]) / dy;
-    double ex = Ex[c], ey = Ey[c], ez = Ez[c];
-    if (a.kind == 0) {
-        Ex[c] = ex + dt * cx;
-        Ey[c] = ey + dt * cy;
-        Ez[c] = ez + dt * cz;
-    } else if (a.kind == 1) {
+    const bool low = i == 0 || j == 0 || k == 0;
+    const bool ghost = low || i > g.n[0] || j > g.n[1] || (a.zper && k > g.n[2]);
+    const size_t row = g.at(i, j, 0);
+    const unsigned o = 8u * k;
+    const double dx = a.dx, dy = a.dy, dz = a.dz, dt = a.dt;
+    double ex = 0, ey = 0, ez = 0, cx = 0, cy = 0, cz = 0;
+    // every polarisation is read before the first is stored, so that the reads leave together
+    double p1[3][3], p0[3][3];
+    if (KIND == 2) {
+#pragma unroll
+        for (int n = 0; n < 3; ++n)
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {
+                p1[n][d] = ldp_once(a.P[n][d] + row, o);
+                p0[n][d] = ldp_once(a.Pp[n][d] + row, o);
+            }
+    }
+    if (!low) {
+        ex = ldp(a.E[0] + row, o);
+        ey = ldp(a.E[1] + row, o);
+        ez = ldp(a.E[2] + row, o);
+        const double *Bx = a.B[0] + row, *By = a.B[1] + row, *Bz = a.B[2] + row;
+        const double bx0 = ldp(Bx, o), by0 = ldp(By, o), bz0 = ldp(Bz, o);
+        const size_t si = (size_t)g.sx, sj = g.pz;
+        cx = (bz0 - ldp(Bz - sj, o)) / dy - (by0 - ldp(By, o - 8u)) / dz;
+        cy = (bx0 - ldp(Bx, o - 8u)) / dz - (bz0 - ldp(Bz - si, o)) / dx;
+        cz = (by0 - ldp(By - si, o)) / dx - (bx0 - ldp(Bx - sj, o)) / dy;
+    }
+    if (KIND == 0) {
+        ex = ex + dt * cx;
+        ey = ey + dt * cy;
+        ez = ez + dt * cz;
+    } else if (KIND == 1) {
         double E2 = ex * ex + ey * ey + ez * ez;
         double Dx = (a.eps + a.chi * E2) * ex + dt * cx;
         double Dy = (a.eps + a.chi * E2) * ey + dt * cy;
@@ -345,67 +383,137 @@ __global__ __launch_bounds__(256) void k_simple_stepD(SimpleArgs a)
             E2 = E * E;
             E = (2 * a.chi * E2 * E + D) / (3 * a.chi * E2 + a.eps);
         } while (fabs(E - Eold) > 1e-9 && ++it < a.ncap);
-        Ex[c] = E * Dx / D;
-        Ey[c] = E * Dy / D;
-        Ez[c] = E * Dz / D;
+        ex = E * Dx / D;
+        ey = E * Dy / D;
+        ez = E * Dz / D;
         // a zero D gives NaN, as in the reference (src/fdtd_nl.cpp:86-89): reported, not avoided
-        report(a.status, (it >= a.ncap ? 1u : 0u) | finite_flag(Ex[c], Ey[c], Ez[c]));
-        return;
+        report(a.status, (it >= a.ncap ? 1u : 0u) | finite_flag(ex, ey, ez));
     } else {
-        double e[3] = {ex, ey, ez};
+        const double e[3] = {ex, ey, ez};
         double P[3] = {0, 0, 0}, Pp[3] = {0, 0, 0};
-        double dt2 = dt * dt;
+        const double dt2 = dt * dt;
+#pragma unroll
         for (int n = 0; n < 3; ++n) {
-            double aa = dt2 * a.om2[n];
-            double b = aa * a.eps2[n];
+            const double aa = dt2 * a.om2[n];
+            const double b = aa * a.eps2[n];
 #pragma unroll
             for (int d = 0; d < 3; ++d) {
-                double p = a.P[n][d][c], pp = a.Pp[n][d][c];
-                double pn = (2 - aa) * p - pp + b * e[d];
-                a.Pp[n][d][c] = p;
-                a.P[n][d][c] = pn;
+                const double p = p1[n][d], pp = p0[n][d];
+                const double pn = (2 - aa) * p - pp + b * e[d];
+                stp_once(a.Pp[n][d] + row, o, low ? p : pn);
+                if (low) stp(a.P[n][d] + row, o, pp);
                 P[d] += pn;
                 Pp[d] += p;
             }
         }
-        Ex[c] = ex + Pp[0] - P[0] + dt * cx;
-        Ey[c] = ey + Pp[1] - P[1] + dt * cy;
-        Ez[c] = ez + Pp[2] - P[2] + dt * cz;
+        ex = ex + Pp[0] - P[0] + dt * cx;
+        ey = ey + Pp[1] - P[1] + dt * cy;
+        ez = ez + Pp[2] - P[2] + dt * cz;
     }
+    if (ghost) return;
+    stp(a.E[0] + row, o, ex);
+    stp(a.E[1] + row, o, ey);
+    stp(a.E[2] + row, o, ez);
+}
+
+// The cells that hold the value of coordinate c of a periodic dimension: itself and its ghost
+// images (N + 1 for cell 1, 0 for cell N)
+struct Images {
+    int c[3], n;
+};
+__device__ __forceinline__ Images images_of(int c, int N, bool periodic)
+{
+    Images m;
+    m.c[0] = m.c[1] = m.c[2] = c;
+    m.n = 1;
+    if (periodic) {
+        if (c == 1) m.c[m.n++] = N + 1;
+        if (c == N) m.c[m.n++] = 0;
+    }
+    return m;
 }
 
 // stepB shared by the three solvers, including the /dx of both Bz terms
-// (src/fdtd_plain.cpp:97-118)
-__global__ __launch_bounds__(256) void k_simple_stepB(SimpleArgs a)
+// (src/fdtd_plain.cpp:97-118), and the ghosts of B and (EXCH) of E.  Without EXCH
+// (FDTD_Plain::stepSchemeInit, src/fdtd_plain.cpp:26-29) E beyond N is read as stored and left.
+template <bool EXCH>
+__global__ __launch_bounds__(256) void k_simple_stepB(SimpleArgs a, int nbx, int nby, int nbz)
 {
-    int k = blockIdx.x * 64 + threadIdx.x;
-    int j = blockIdx.y * 4 + threadIdx.y;
-    int i = blockIdx.z;
+    int bx, by, bz;
+    xcd_tile(nbx, nby, nbz, bx, by, bz);
     const GridDims &g = a.g;
+    const int k = bx * 64 + threadIdx.x + (a.zper ? 1 : 0), i = bz + 1;
+    const int j = __builtin_amdgcn_readfirstlane(by * 4 + (int)threadIdx.y + 1);
     if (k > g.n[2] || j > g.n[1]) return;
-    size_t c = g.at(i, j, k);
-    const double *Ex = a.E[0], *Ey = a.E[1], *Ez = a.E[2];
+    const size_t row = g.at(i, j, 0);
+    const unsigned o = 8u * k;
+    const size_t ri = EXCH && i == g.n[0] ? g.at(1, j, 0) : row + (size_t)g.sx;
+    const size_t rj = EXCH && j == g.n[1] ? g.at(i, 1, 0) : row + g.pz;
+    const unsigned ok = EXCH && a.zper && k == g.n[2] ? 8u : o + 8u;
     double dx = a.dx, dy = a.dy, dz = a.dz, dt = a.dt;
-    double ex = Ex[c], ey = Ey[c], ez = Ez[c];
-    a.B[0][c] = a.B[0][c] + dt * ((Ey[g.at(i, j, k + 1)] - ey) / dz - (Ez[g.at(i, j + 1, k)] - ez) / dy);
-    a.B[1][c] = a.B[1][c] + dt * ((Ez[g.at(i + 1, j, k)] - ez) / dx - (Ex[g.at(i, j, k + 1)] - ex) / dz);
-    a.B[2][c] = a.B[2][c] + dt * ((Ex[g.at(i, j + 1, k)] - ex) / dx - (Ey[g.at(i + 1, j, k)] - ey) / dx);
+    const double e[3] = {ldp(a.E[0] + row, o), ldp(a.E[1] + row, o), ldp(a.E[2] + row, o)};
+    const double ex = e[0], ey = e[1], ez = e[2];
+    double b[3] = {ldp(a.B[0] + row, o), ldp(a.B[1] + row, o), ldp(a.B[2] + row, o)};
+    b[0] = b[0] + dt * ((ldp(a.E[1] + row, ok) - ey) / dz - (ldp(a.E[2] + rj, o) - ez) / dy);
+    b[1] = b[1] + dt * ((ldp(a.E[2] + ri, o) - ez) / dx - (ldp(a.E[0] + row, ok) - ex) / dz);
+    b[2] = b[2] + dt * ((ldp(a.E[0] + rj, o) - ex) / dx - (ldp(a.E[1] + ri, o) - ey) / dx);
+    for (int d = 0; d < 3; ++d) stp(a.B[d] + row, o, b[d]);
+    if (i > 1 && i < g.n[0] && j > 1 && j < g.n[1]) {  // at most z images: every wave meets a row end
+        if (a.zper && (k == 1 || k == g.n[2])) {
+            const unsigned q = k == 1 ? 8u * (g.n[2] + 1) : 0u;
+            for (int d = 0; d < 3; ++d) {
+                stp(a.B[d] + row, q, b[d]);
+                if (EXCH) stp(a.E[d] + row, q, e[d]);
+            }
+            if (g.n[2] == 1)  // cell 1 is cell N too
+                for (int d = 0; d < 3; ++d) {
+                    stp(a.B[d] + row, 0u, b[d]);
+                    if (EXCH) stp(a.E[d] + row, 0u, e[d]);
+                }
+        }
+        return;
+    }
+    const Images x = images_of(i, g.n[0], true), y = images_of(j, g.n[1], true), z = images_of(k, g.n[2], a.zper);
+    for (int u = 0; u < x.n; ++u)
+        for (int v = 0; v < y.n; ++v)
+            for (int w = 0; w < z.n; ++w) {
+                if (u + v + w == 0) continue;
+                const size_t q = g.at(x.c[u], y.c[v], z.c[w]);
+                for (int d = 0; d < 3; ++d) {
+                    a.B[d][q] = b[d];
+                    if (EXCH) a.E[d][q] = e[d];
+                }
+                if (!a.zper && k == g.n[2])  // the plane above, outside B's range
+                    for (int d = 0; d < 3; ++d) {
+                        a.B[d][q + 1] = a.B[d][row + k + 1];
+                        if (EXCH) a.E[d][q + 1] = a.E[d][row + k + 1];
+                    }
+            }
 }
 
 void launch_simple_stepD(const SimpleArgs &a, hipStream_t s)
 {
     const GridDims &g = a.g;
-    dim3 blk(64, 4);
-    dim3 grd((g.n[2] + 1 + 63) / 64, (g.n[1] + 1 + 3) / 4, g.n[0] + 1);
-    hipLaunchKernelGGL(k_simple_stepD, grd, blk, 0, s, a);
+    const int more = a.kind == 2 ? 2 : (a.kind == 1 ? 1 : 0);  // the ghosts whose threads have work
+    const int nk = g.n[2] + (a.zper || more ? more : 1), nj = g.n[1] + more;
+    const int nbx = (nk + 63) / 64, nby = (nj + 3) / 4, nbz = g.n[0] + more;
+    dim3 blk(64, 4), grd(nbx, nby, nbz);
+    switch (a.kind) {
+    case 0: hipLaunchKernelGGL(k_simple_stepD<0>, grd, blk, 0, s, a, nbx, nby, nbz); break;
+    case 1: hipLaunchKernelGGL(k_simple_stepD<1>, grd, blk, 0, s, a, nbx, nby, nbz); break;
+    default: hipLaunchKernelGGL(k_simple_stepD<2>, grd, blk, 0, s, a, nbx, nby, nbz); break;
+    }
 }
 
-void launch_simple_stepB(const SimpleArgs &a, hipStream_t s)
+void launch_simple_stepB(const SimpleArgs &a, bool exchange, hipStream_t s)
 {
     const GridDims &g = a.g;
-    dim3 blk(64, 4);
-    dim3 grd((g.n[2] + 1 + 63) / 64, (g.n[1] + 1 + 3) / 4, g.n[0] + 1);
-    hipLaunchKernelGGL(k_simple_stepB, grd, blk, 0, s, a);
+    const int nbx = (g.n[2] + (a.zper ? 0 : 1) + 63) / 64, nby = (g.n[1] + 3) / 4, nbz = g.n[0];
+    dim3 blk(64, 4), grd(nbx, nby, nbz);
+    if (exchange)
+        hipLaunchKernelGGL(k_simple_stepB<true>, grd, blk, 0, s, a, nbx, nby, nbz);
+    else
+        hipLaunchKernelGGL(k_simple_stepB<false>, grd, blk, 0, s, a, nbx, nby, nbz);
 }
 
 // ------------------------------------------------------------------------------------

@@ -32,6 +32,7 @@ struct SimpleArgs {
     double eps2[3], om2[3];
     unsigned *status;
     int ncap;
+    int zper;  // z periodic: its ghosts are written as images (x and y always are)
 };
 
 template <typename T>
@@ -98,7 +99,8 @@ void launch_adjoint_step(const AdjArgs &a, hipStream_t s);
 void launch_plane_objective(const GridDims &g, const double *const E[3], int kobj, double w, double *acc,
                             hipStream_t s);
 void launch_simple_stepD(const SimpleArgs &a, hipStream_t s);
-void launch_simple_stepB(const SimpleArgs &a, hipStream_t s);
+// exchange: E beyond N from its periodic image, and the ghosts of E left as images (always B's)
+void launch_simple_stepB(const SimpleArgs &a, bool exchange, hipStream_t s);
 template <typename T>
 void launch_probe(const ProbeArgs<T> &a, double *row, hipStream_t s);
 size_t energy_partials(const GridDims &g);

@@ -425,18 +425,6 @@ struct RowD {
     double a[64], b[64];
 };
 
-// Word at byte offset bo (per lane, 32 bits: a plane holds (ny + 2) pz words < 2^32 bytes)
-// from the plane base `base` (wave-uniform)
-template <typename T>
-__device__ __forceinline__ T ldp(const T *base, unsigned bo)
-{
-    return gld((const T *)((const char *)base + bo));
-}
-template <typename T>
-__device__ __forceinline__ void stp_once(T *base, unsigned bo, T v)
-{
-    store_once((T *)((char *)base + bo), v);
-}
 // A read-only table entry at a wave-uniform address, through the constant address space: a
 // scalar load into SGPRs, counted apart from the vector loads in flight
 __device__ __forceinline__ double kload(const double *p)

@@ -1428,6 +1428,7 @@ static mpx::SimpleArgs simple_args(mpx_solver *s)
     }
     a.status = s->d_status;
     a.ncap = s->ncap;
+    a.zper = s->periodic[2];
     return a;
 }
 
@@ -1730,12 +1731,13 @@ static int step_once(mpx_solver *s, int ahead)
         mpx::launch_simple_stepD(a, s->stream);
         s->tock();
         MPX_LAUNCHED("simple stepD");
-        if ((rc = wrap_group<double>(s, s->E, K_WRAP_E))) return rc;
+        if (s->solver == MPX_SOLVER_DISP)  // the kernel left the new P in Pp's arrays
+            for (int n = 0; n < 3; ++n)
+                for (int c = 0; c < 3; ++c) std::swap(s->P[n][c], s->Pp[n][c]);
         s->tick(K_SIMPLE_B);
-        mpx::launch_simple_stepB(a, s->stream);
+        mpx::launch_simple_stepB(a, true, s->stream);
         s->tock();
         MPX_LAUNCHED("simple stepB");
-        if ((rc = wrap_group<double>(s, s->B, K_WRAP_B))) return rc;
     } else if (s->path == MPX_PATH_REFERENCE) {
         StepArgs<double> ae = step_args<double>(s, false);
         // Sigma := 0 and the E-side OptFields, src/fdtd_plrc.t:129-135
@@ -1868,9 +1870,9 @@ int mpx_step_init(mpx_solver *s)
     if (!s->plrc) {
         mpx::SimpleArgs a = simple_args(s);
         a.dt = 0.5 * s->d.dt;
-        mpx::launch_simple_stepB(a, s->stream);
+        mpx::launch_simple_stepB(a, false, s->stream);
         MPX_LAUNCHED("simple stepB");
-        return wrap_group<double>(s, s->B, K_WRAP_B);
+        return MPX_OK;
     }
     if ((rc = materialise_ghosts(s))) return rc;
     StepArgs<double> ae = step_args<double>(s, false);
