@@ -165,9 +165,9 @@ __device__ __forceinline__ void fused_E_tile(const StepArgs<T> &a, int tbx, int 
         report(a.status, fl | finite_flag(ex, ey, ez));
         unsigned wn = 0;
         const T hx = put<T, RES>(ex, wn, 0), hy = put<T, RES>(ey, wn, 1), hz = put<T, RES>(ez, wn, 2);
-        store_once(&a.E[0][c], hx);
-        store_once(&a.E[1][c], hy);
-        store_once(&a.E[2][c], hz);
+        store_once(&a.En[0][c], hx);
+        store_once(&a.En[1][c], hy);
+        store_once(&a.En[2][c], hz);
         if (RES) store_once(&a.Elo[c], wn);
     }
 }

@@ -611,6 +611,10 @@ void launch_energy(const GridDims &g, T *const e[3], T *const b[3], double *part
     hipLaunchKernelGGL(k_energy_partial<T>, grd, blk, 0, s, g, e[0], e[1], e[2], b[0], b[1], b[2], elo, blo, part);
     hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(256), 0, s, part, energy_partials(g), out, scale);
 }
+void launch_sum_partials(const double *part, size_t n, double *out, double scale, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(256), 0, s, part, n, out, scale);
+}
 template void launch_energy<double>(const GridDims &, double *const[3], double *const[3], double *, double *,
                                     hipStream_t, const unsigned *, const unsigned *, double);
 template void launch_energy<float>(const GridDims &, float *const[3], float *const[3], double *, double *,

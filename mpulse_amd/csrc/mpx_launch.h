@@ -95,9 +95,12 @@ template <typename T>
 void launch_march_batch(const PassArgs<T> *table, const BatchRun *runs, int nruns, int total, int rows, int np,
                         bool nonlin, bool cp, hipStream_t s);
 void launch_advance_time(int *time, int k, hipStream_t s);
-void launch_adjoint_step(const AdjArgs &a, hipStream_t s);
-void launch_plane_objective(const GridDims &g, const double *const E[3], int kobj, double w, double *acc,
-                            hipStream_t s);
+size_t adjoint_waves(const GridDims &g);  // elements of AdjArgs::chiw
+void launch_adjoint_step(const AdjArgs &a, const AdjHistory &h, hipStream_t s);
+// the plane's partial sums, objective_blocks of them
+int objective_blocks(const GridDims &g);
+void launch_plane_objective(const GridDims &g, const double *const E[3], int kobj, double *part, hipStream_t s);
+void launch_sum_partials(const double *part, size_t n, double *out, double scale, hipStream_t s);
 void launch_simple_stepD(const SimpleArgs &a, hipStream_t s);
 // exchange: E beyond N from its periodic image, and the ghosts of E left as images (always B's)
 void launch_simple_stepB(const SimpleArgs &a, bool exchange, hipStream_t s);

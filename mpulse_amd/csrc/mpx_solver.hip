@@ -106,6 +106,90 @@ enum {
 
 }  // namespace
 
+// ---------------------------------------------------------------------------------------
+// device memory
+// ---------------------------------------------------------------------------------------
+//
+// An adjoint call works in gigabytes that it needs for its own length only.  Allocating and
+// freeing them on every call took 60 (250 separate arrays) to 90 ms (one block: the driver clears
+// what it maps) of the 157 ms of a 128x128x256, 100-step gradient, so one block per GPU is kept
+// between calls, whichever solver they are for.  It holds nothing: a call takes the block out of
+// its slot (a second call at the same time finds the slot empty and allocates), uses it on its own
+// stream and puts it back after waiting for that stream.  Bounded to an eighth of the GPU's
+// memory; freed when an allocation of this library fails (which is then tried again) and when the
+// last solver is destroyed.
+namespace {
+struct Spare {
+    void *p = nullptr;
+    size_t bytes = 0;
+};
+std::mutex g_spare_mu;
+std::vector<Spare> g_spare;  // per device id
+int g_solvers = 0;           // solvers alive
+
+// frees the kept blocks; whether there was one
+bool spare_drop()
+{
+    std::vector<Spare> old;
+    {
+        std::lock_guard<std::mutex> lock(g_spare_mu);
+        old.swap(g_spare);
+    }
+    bool any = false;
+    for (const Spare &b : old)
+        if (b.p) any = hipFree(b.p) == hipSuccess || any;
+    return any;
+}
+
+hipError_t dev_malloc(void **p, size_t bytes)
+{
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipErrorOutOfMemory && spare_drop()) {
+        (void)hipGetLastError();
+        e = hipMalloc(p, bytes);
+    }
+    return e;
+}
+
+// a block of at least *bytes (its size returned), the kept one if it is large enough; null on failure
+void *spare_take(int device, size_t *bytes)
+{
+    Spare b;
+    {
+        std::lock_guard<std::mutex> lock(g_spare_mu);
+        if (device < (int)g_spare.size()) std::swap(b, g_spare[device]);
+    }
+    if (b.p && b.bytes >= *bytes) {
+        *bytes = b.bytes;
+        return b.p;
+    }
+    if (b.p) (void)hipFree(b.p);
+    void *p = nullptr;
+    if (dev_malloc(&p, *bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    return p;
+}
+
+// puts a block back (no kernel uses it any more); the slot's older block, or this one past the
+// bound, is freed
+void spare_give(int device, void *p, size_t bytes)
+{
+    if (!p) return;
+    size_t avail = 0, total = 0;
+    Spare b{p, bytes};
+    if (hipMemGetInfo(&avail, &total) == hipSuccess && bytes <= total / 8) {
+        std::lock_guard<std::mutex> lock(g_spare_mu);
+        if (g_solvers > 0) {
+            if ((int)g_spare.size() <= device) g_spare.resize(device + 1);
+            std::swap(b, g_spare[device]);
+        }
+    }
+    if (b.p) (void)hipFree(b.p);
+}
+}  // namespace
+
 struct mpx_solver {
     mpx_desc d{};
     int solver = 0, prec = 0, path = 0;
@@ -201,8 +285,19 @@ struct mpx_solver {
     void *d_pargs[2] = {nullptr, nullptr};
     std::vector<unsigned char> h_pargs[2];
 
+    mpx_solver()
+    {
+        std::lock_guard<std::mutex> lock(g_spare_mu);
+        ++g_solvers;
+    }
     ~mpx_solver()
     {
+        bool last;
+        {
+            std::lock_guard<std::mutex> lock(g_spare_mu);
+            last = --g_solvers == 0;
+        }
+        if (last) (void)spare_drop();
         if (stream) (void)hipStreamSynchronize(stream);
         for (void *p : allocs) (void)hipFree(p);
         for (hipEvent_t e : timer.pool) (void)hipEventDestroy(e);
@@ -214,7 +309,7 @@ struct mpx_solver {
     {
         void *p = nullptr;
         if (count == 0) count = 1;
-        if (hipMalloc(&p, count * sizeof(T)) != hipSuccess) {
+        if (dev_malloc(&p, count * sizeof(T)) != hipSuccess) {
             rc = fail(MPX_ERR_NOMEM, "hipMalloc of " + std::to_string(count * sizeof(T)) + " bytes failed");
             return nullptr;
         }
@@ -1181,7 +1276,7 @@ static StepArgs<T> step_args(mpx_solver *s, bool hside)
         a.kdH[d] = s->d_kdH[d];
         a.ikdE[d] = s->d_ikdE[d];
         a.ikdH[d] = s->d_ikdH[d];
-        a.E[d] = (T *)s->E[d];
+        a.E[d] = a.En[d] = (T *)s->E[d];
         a.B[d] = (T *)s->B[d];
         a.blo[d] = s->periodic[d] ? 1 : 0;
     }
@@ -1510,7 +1605,7 @@ static const StepArgs<T> *dev_args(mpx_solver *s, const StepArgs<T> &a, int side
     std::vector<unsigned char> &h = s->h_fargs[side];
     if (h.size() == sizeof(a) && std::memcmp(h.data(), p, sizeof(a)) == 0) return (const StepArgs<T> *)s->d_fargs[side];
     if (!s->d_fargs[side]) {
-        if (hipMalloc(&s->d_fargs[side], sizeof(StepArgs<double>)) != hipSuccess) {
+        if (dev_malloc(&s->d_fargs[side], sizeof(StepArgs<double>)) != hipSuccess) {
             s->d_fargs[side] = nullptr;
             return nullptr;
         }
@@ -1670,7 +1765,7 @@ static int pass_launch_t(mpx_solver *s, int soff)
     std::vector<unsigned char> &h = s->h_pargs[side];
     if (!(h.size() == sizeof(a) && std::memcmp(h.data(), p, sizeof(a)) == 0)) {
         if (!s->d_pargs[side]) {
-            if (hipMalloc(&s->d_pargs[side], sizeof(mpx::PassArgs<double>)) != hipSuccess) {
+            if (dev_malloc(&s->d_pargs[side], sizeof(mpx::PassArgs<double>)) != hipSuccess) {
                 s->d_pargs[side] = nullptr;
                 return fail(MPX_ERR_NOMEM, "argument block allocation failed");
             }
@@ -1987,7 +2082,7 @@ static int box_copy(mpx_solver *s, void *ptr, size_t elem, bool isPsi, int part,
     if (!s->d_box) {
         size_t n = std::max<size_t>(1, std::min<size_t>(nx2, ((size_t)1 << 23) / plane));
         for (;; n = (n + 1) / 2) {
-            if (hipMalloc((void **)&s->d_box, n * plane * 8) == hipSuccess) break;
+            if (dev_malloc((void **)&s->d_box, n * plane * 8) == hipSuccess) break;
             s->d_box = nullptr;
             (void)hipGetLastError();
             if (n == 1) return fail(MPX_ERR_NOMEM, "hipMalloc of a staging plane failed");
@@ -2407,7 +2502,7 @@ int mpx_sampler_create(mpx_solver *s, const char *name, int dim, const int pos[3
         // the fused and sweep paths of the PLRC solvers leave the ghosts of E and B stale
         if (s->plrc && s->path != MPX_PATH_REFERENCE)
             for (int d = 0; d < 3; ++d) p->wrapmask |= s->periodic[d] ? 1 << d : 0;
-        if (hipMalloc((void **)&p->ring, (size_t)capacity * len * sizeof(double)) != hipSuccess)
+        if (dev_malloc((void **)&p->ring, (size_t)capacity * len * sizeof(double)) != hipSuccess)
             return fail(MPX_ERR_NOMEM, "hipMalloc of the sampler ring failed");
     }
     *out = p.release();
@@ -2635,7 +2730,7 @@ int mpx_copy_probe(size_t bytes, int reps, double *ms_per_copy)
     hipStream_t st;
     hipEvent_t e0, e1;
     MPX_HIP(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
-    if (hipMalloc(&a, bytes) != hipSuccess || hipMalloc(&b, bytes) != hipSuccess) {
+    if (dev_malloc(&a, bytes) != hipSuccess || dev_malloc(&b, bytes) != hipSuccess) {
         (void)hipFree(a);
         (void)hipStreamDestroy(st);
         return fail(MPX_ERR_NOMEM, "copy probe allocation failed");
@@ -2775,7 +2870,7 @@ struct mpx_batch {
     }
     int alloc(void **p, size_t bytes)
     {
-        if (hipMalloc(p, bytes ? bytes : 1) != hipSuccess) return fail(MPX_ERR_NOMEM, "batch table allocation failed");
+        if (dev_malloc(p, bytes ? bytes : 1) != hipSuccess) return fail(MPX_ERR_NOMEM, "batch table allocation failed");
         allocs.push_back(*p);
         return MPX_OK;
     }
@@ -3336,20 +3431,24 @@ namespace {
 
 size_t face_count(const CpmlFace &F) { return (size_t)(F.hi[0] - F.lo[0] + 1) * F.n1 * F.n2; }
 
-// device buffers owned by one adjoint call
-struct DevBufs {
-    std::vector<void *> p;
-    ~DevBufs()
+// The device memory of one adjoint call: one block, sized by a first run of the call's carving
+// (base null) and handed out by the second.
+struct Arena {
+    char *base = nullptr;
+    size_t used = 0, bytes = 0;
+    int device = 0;
+    hipStream_t stream = nullptr;
+    ~Arena()
     {
-        for (void *q : p) (void)hipFree(q);
+        if (base) (void)hipStreamSynchronize(stream);
+        spare_give(device, base, bytes);
     }
-    double *get(size_t count, hipStream_t st)
+    template <typename T>
+    T *get(size_t count)
     {
-        void *q = nullptr;
-        if (hipMalloc(&q, (count ? count : 1) * sizeof(double)) != hipSuccess) return nullptr;
-        p.push_back(q);
-        if (hipMemsetAsync(q, 0, (count ? count : 1) * sizeof(double), st) != hipSuccess) return nullptr;
-        return (double *)q;
+        T *p = base ? (T *)(base + used) : nullptr;
+        used += (count * sizeof(T) + 255) / 256 * 256;
+        return p;
     }
 };
 
@@ -3359,13 +3458,26 @@ struct StateRef {
     std::vector<std::pair<void *, size_t>> arr;  // (device pointer, doubles)
 };
 
+// the CPML face of dimension d on its high (q 0) or low (1) side, E or H currents; null if none
+const CpmlFace *face_of(mpx_solver *s, int hside, int d, int q)
+{
+    for (const Current &c : hside ? s->hcur : s->ecur)
+        if (c.face >= 0 && dim_of(c.dir) == d && is_high(c.dir) == (q == 0))
+            return &(hside ? s->hfaces : s->efaces)[c.face];
+    return nullptr;
+}
+// extent of that face's box along x
+int adj_extent(mpx_solver *s, int hside, int d, int q)
+{
+    const CpmlFace *F = face_of(s, hside, d, q);
+    return F ? F->hi[0] - F->lo[0] + 1 : 0;
+}
+
 StateRef state_of(mpx_solver *s)
 {
     StateRef r;
-    for (int c = 0; c < 3; ++c) {
-        r.arr.push_back({s->E[c], s->cells});
-        r.arr.push_back({s->B[c], s->cells});
-    }
+    for (int c = 0; c < 3; ++c) r.arr.push_back({s->E[c], s->cells});  // E first: entries 0..2
+    for (int c = 0; c < 3; ++c) r.arr.push_back({s->B[c], s->cells});
     for (int p = 0; p < s->np; ++p) r.arr.push_back({s->psi[p][0], mpx::psi_block_elems(s->cells) * 2});
     for (const CpmlFace &F : s->efaces) {
         r.arr.push_back({F.psi0, face_count(F)});
@@ -3399,47 +3511,57 @@ int mpx_adjoint_grad(mpx_solver *s, const mpx_objective *obj, int nsteps, int K,
     if (obj->plane_k < 1 || obj->plane_k > s->g.n[2]) return fail(MPX_ERR_INVALID, "objective plane out of range");
     const bool grad = dJ_deps || dJ_dchi;
     hipStream_t st = s->stream;
-    DevBufs mem;
-    double *dJ = mem.get(1, st);
-    if (!dJ) return fail(MPX_ERR_NOMEM, "adjoint allocation failed");
     const int t0 = s->time;
     s->win_n = 0;
-    const int nseg = (nsteps + K - 1) / K;
+    const int nseg = (nsteps + K - 1) / K, klen = std::min(K, nsteps);
+    const int nobj = mpx::objective_blocks(s->g);
     StateRef cur = state_of(s);
-    auto snapshot = [&](std::vector<double *> &dst) -> int {
-        if (dst.empty())
-            for (auto &a : cur.arr) {
-                double *q = mem.get(a.second, st);
-                if (!q) return fail(MPX_ERR_NOMEM, "checkpoint allocation failed");
-                dst.push_back(q);
-            }
-        for (size_t q = 0; q < cur.arr.size(); ++q)
-            MPX_HIP(hipMemcpyAsync(dst[q], cur.arr[q].first, cur.arr[q].second * 8, hipMemcpyDeviceToDevice, st));
-        return MPX_OK;
-    };
-    auto restore = [&](const std::vector<double *> &src) -> int {
-        for (size_t q = 0; q < cur.arr.size(); ++q)
-            MPX_HIP(hipMemcpyAsync(cur.arr[q].first, src[q], cur.arr[q].second * 8, hipMemcpyDeviceToDevice, st));
-        return MPX_OK;
-    };
-    std::vector<std::vector<double *>> ckpt(grad ? nseg : 0);
-    int rc;
-    // forward pass: objective after every step, a checkpoint at the start of every segment
-    for (int n = 0; n < nsteps; ++n) {
-        if (grad && n % K == 0 && (rc = snapshot(ckpt[n / K]))) return rc;
-        if ((rc = step_once(s, nsteps - n))) return rc;
-        double *E[3] = {(double *)s->E[0], (double *)s->E[1], (double *)s->E[2]};
-        mpx::launch_plane_objective(s->g, E, obj->plane_k, obj->weight, dJ, st);
-        MPX_LAUNCHED("plane objective");
-    }
-    MPX_HIP(hipMemcpyAsync(J, dJ, sizeof(double), hipMemcpyDeviceToHost, st));
-    MPX_HIP(hipStreamSynchronize(st));
-    if (!grad) return MPX_OK;
-    std::vector<double *> fin;
-    if ((rc = snapshot(fin))) return rc;
 
-    // adjoint state, zero after the last step
+    // everything the call needs on the device: `clear` bytes at the front start at zero
+    Arena mem;
+    double *dJ, *part;
+    std::vector<std::vector<double *>> ckpt(grad ? nseg : 0);  // state at the start of every segment
+    std::vector<double *> fin;                                 // and after the last step
+    std::vector<std::array<double *, 3>> hist(grad ? klen + 1 : 0);  // E after steps 1 .. of a segment
+    StepArgs<double> *d_step = nullptr;
     mpx::AdjArgs a{};
+    size_t clear = 0;
+    auto carve = [&]() {
+        mem.used = 0;
+        if (grad) {
+            for (int p = 0; p < s->np; ++p)
+                for (int q = 0; q < 3; ++q) a.lpsi[p][q] = mem.get<double2>(s->cells);
+            for (int d = 0; d < 3; ++d) {
+                a.lE[d] = mem.get<double>(s->cells);
+                a.lB[d] = mem.get<double>(s->cells);
+            }
+            a.epsb = mem.get<double>(s->cells);
+            a.chiw = mem.get<double>(mpx::adjoint_waves(s->g));
+            for (int side = 0; side < 2; ++side)
+                for (int d = 0; d < 3; ++d)
+                    for (int q = 0; q < 2; ++q) {
+                        mpx::AdjFace &f = side ? a.hf[d][q] : a.ef[d][q];
+                        if (f.hi < f.lo) continue;
+                        const size_t n = (size_t)f.s0 * adj_extent(s, side, d, q);
+                        f.A0 = mem.get<double>(n);
+                        f.A1 = mem.get<double>(n);
+                    }
+            clear = mem.used;
+            for (int d = 0; d < 3; ++d) a.rb[d] = mem.get<double>(s->cells);
+            for (int m = 1; m <= klen; ++m)
+                for (int c = 0; c < 3; ++c) hist[m][c] = mem.get<double>(s->cells);
+            fin.clear();
+            for (auto &r : cur.arr) fin.push_back(mem.get<double>(r.second));
+            for (auto &ck : ckpt) {
+                ck.clear();
+                for (auto &r : cur.arr) ck.push_back(mem.get<double>(r.second));
+            }
+            d_step = mem.get<StepArgs<double>>(2 * klen + nseg);
+        }
+        part = mem.get<double>((size_t)nsteps * nobj);
+        dJ = mem.get<double>(1);
+    };
+    // adjoint arguments (the faces' ranges first: carve sizes their arrays)
     a.g = s->g;
     a.dt = s->d.dt;
     a.chi = s->nonlin ? s->d.chi : 0.0;  // the linear core has no Kerr term
@@ -3449,99 +3571,116 @@ int mpx_adjoint_grad(mpx_solver *s, const mpx_objective *obj, int nsteps, int K,
     a.pc = s->pc;
     a.sumChi0 = s->sumChi0;
     a.sumXi0 = s->sumXi0;
-    for (int p = 0; p < s->np; ++p)
-        for (int q = 0; q < 3; ++q) {
-            a.lpsi[p][q] = (double2 *)mem.get(2 * s->cells, st);
-            if (!a.lpsi[p][q]) return fail(MPX_ERR_NOMEM, "adjoint allocation failed");
-        }
+    a.kobj = obj->plane_k;
+    a.wobj = obj->weight;
+    a.band = s->tile_band > 0 ? s->tile_band : auto_band(s->g, nullptr, false);
     for (int d = 0; d < 3; ++d) {
         a.ikdE[d] = s->d_ikdE[d];
         a.ikdH[d] = s->d_ikdH[d];
-        a.lE[d] = mem.get(s->cells, st);
-        a.lB[d] = mem.get(s->cells, st);
+        for (int side = 0; side < 2; ++side)
+            for (int q = 0; q < 2; ++q) {
+                mpx::AdjFace &f = side ? a.hf[d][q] : a.ef[d][q];
+                f.lo = 1;
+                f.hi = 0;
+                const CpmlFace *F = face_of(s, side, d, q);
+                if (!F) continue;
+                f.lo = F->lo[d];
+                f.hi = F->hi[d];
+                f.s0 = F->n1 * F->n2;
+                f.s1 = F->n2;
+                f.off = F->lo[0] * f.s0 + F->lo[1] * f.s1 + F->lo[2];
+                f.b = F->b;
+                f.c = F->c;
+                f.idxn = F->idxn;
+            }
     }
-    for (int q = 0; q < 6; ++q) {
-        a.dEb[q] = mem.get(s->cells, st);
-        a.dBb[q] = mem.get(s->cells, st);
+    carve();
+    mem.device = s->device;
+    mem.stream = st;
+    mem.bytes = mem.used;
+    mem.base = (char *)spare_take(s->device, &mem.bytes);
+    if (!mem.base) return fail(MPX_ERR_NOMEM, "adjoint allocation of " + std::to_string(mem.used) + " bytes failed");
+    carve();
+    if (clear) MPX_HIP(hipMemsetAsync(mem.base, 0, clear, st));
+    auto copy_state = [&](const std::vector<double *> &to, bool back, size_t from) -> int {
+        for (size_t q = from; q < cur.arr.size(); ++q)
+            MPX_HIP(hipMemcpyAsync(back ? cur.arr[q].first : to[q], back ? to[q] : cur.arr[q].first,
+                                   cur.arr[q].second * 8, hipMemcpyDeviceToDevice, st));
+        return MPX_OK;
+    };
+    int rc;
+    // forward pass: objective after every step, a checkpoint at the start of every segment
+    for (int n = 0; n < nsteps; ++n) {
+        if (grad && n % K == 0 && (rc = copy_state(ckpt[n / K], false, 0))) return rc;
+        if ((rc = step_once(s, nsteps - n))) return rc;
+        double *E[3] = {(double *)s->E[0], (double *)s->E[1], (double *)s->E[2]};
+        mpx::launch_plane_objective(s->g, E, obj->plane_k, part + (size_t)n * nobj, st);
+        MPX_LAUNCHED("plane objective");
     }
-    a.epsb = mem.get(s->cells, st);
-    a.chib = mem.get(s->cells, st);
-    a.kobj = obj->plane_k;
-    a.wobj = obj->weight;
-    a.nefaces = (int)s->efaces.size();
-    a.nhfaces = (int)s->hfaces.size();
-    for (int d = 0; d < 3; ++d)
-        for (int q = 0; q < 2; ++q) a.efbd[d][q] = a.hfbd[d][q] = -1;
-    for (size_t f = 0; f < s->efaces.size(); ++f) {
-        a.eface[f] = s->efaces[f];
-        for (int w = 0; w < 2; ++w) a.lpsiE[f][w] = mem.get(face_count(s->efaces[f]), st);
+    mpx::launch_sum_partials(part, (size_t)nsteps * nobj, dJ, obj->weight, st);
+    MPX_LAUNCHED("objective sum");
+    MPX_HIP(hipMemcpyAsync(J, dJ, sizeof(double), hipMemcpyDeviceToHost, st));
+    MPX_HIP(hipStreamSynchronize(st));
+    if (!grad) return MPX_OK;
+    if ((rc = copy_state(fin, false, 0))) return rc;
+
+    // The steps of a segment run again with E written to the history: step m reads E from
+    // hist[m - 1] (the segment's checkpoint for m = 1) and leaves it in hist[m].  Their argument
+    // blocks: nseg of first E halves, then klen - 1 E halves (m >= 2), then klen B halves.
+    std::vector<StepArgs<double>> h_step(2 * klen + nseg);
+    auto e_args = [&](int seg, int m) { return m == 1 ? seg : nseg + m - 2; };
+    auto b_args = [&](int m) { return nseg + klen - 1 + m - 1; };
+    for (int m = 1; m <= klen; ++m) {
+        for (int seg = 0; seg < (m == 1 ? nseg : 1); ++seg) {
+            StepArgs<double> e = step_args<double>(s, false);
+            for (int c = 0; c < 3; ++c) {
+                e.E[c] = m == 1 ? ckpt[seg][c] : hist[m - 1][c];
+                e.En[c] = hist[m][c];
+            }
+            h_step[e_args(seg, m)] = e;
+        }
+        StepArgs<double> b = step_args<double>(s, true);
+        for (int c = 0; c < 3; ++c) b.E[c] = b.En[c] = hist[m][c];
+        h_step[b_args(m)] = b;
     }
-    for (size_t f = 0; f < s->hfaces.size(); ++f) {
-        a.hface[f] = s->hfaces[f];
-        for (int w = 0; w < 2; ++w) a.lpsiH[f][w] = mem.get(face_count(s->hfaces[f]), st);
-    }
-    for (const Current &c : s->ecur)
-        if (c.face >= 0) a.efbd[dim_of(c.dir)][is_high(c.dir) ? 0 : 1] = c.face;
-    for (const Current &c : s->hcur)
-        if (c.face >= 0) a.hfbd[dim_of(c.dir)][is_high(c.dir) ? 0 : 1] = c.face;
-    // forward E of one segment: (K + 1) planes of E
-    std::vector<std::array<double *, 3>> hist(K + 1);
-    for (auto &h : hist)
-        for (int c = 0; c < 3; ++c) h[c] = mem.get(s->cells, st);
-    for (int d = 0; d < 3; ++d)
-        if (!a.lE[d] || !a.lB[d]) return fail(MPX_ERR_NOMEM, "adjoint allocation failed");
-    for (int q = 0; q < 6; ++q)
-        if (!a.dEb[q] || !a.dBb[q]) return fail(MPX_ERR_NOMEM, "adjoint allocation failed");
-    if (!a.epsb || !a.chib) return fail(MPX_ERR_NOMEM, "adjoint allocation failed");
-    for (auto &h : hist)
-        for (int c = 0; c < 3; ++c)
-            if (!h[c]) return fail(MPX_ERR_NOMEM, "adjoint history allocation failed");
+    MPX_HIP(hipMemcpyAsync(d_step, h_step.data(), h_step.size() * sizeof(h_step[0]), hipMemcpyHostToDevice, st));
+    MPX_HIP(hipStreamSynchronize(st));
 
     for (int seg = nseg - 1; seg >= 0; --seg) {
         const int len = std::min(K, nsteps - seg * K);
-        if ((rc = restore(ckpt[seg]))) return rc;
+        if ((rc = copy_state(ckpt[seg], true, 3))) return rc;  // all but E, which is read from the checkpoint
+        for (int c = 0; c < 3; ++c) hist[0][c] = ckpt[seg][c];
         s->time = t0 + seg * K;
         s->win_n = 0;
-        auto keepE = [&](int m) -> int {
-            for (int c = 0; c < 3; ++c)
-                MPX_HIP(hipMemcpyAsync(hist[m][c], s->E[c], s->cells * 8, hipMemcpyDeviceToDevice, st));
-            return MPX_OK;
-        };
-        if ((rc = keepE(0))) return rc;
-        for (int m = 1; m <= len; ++m) {
-            if ((rc = step_once(s, len - m + 1))) return rc;
-            if ((rc = keepE(m))) return rc;
+        for (int m = 1; m <= len; ++m, s->time++) {
+            int soff;
+            if ((rc = sheets_at(s, s->time, s->time, len - m + 1, &soff))) return rc;
+            mpx::launch_fused_E<double>(h_step[e_args(seg, m)], d_step + e_args(seg, m), s->np, s->nonlin, soff, st);
+            MPX_LAUNCHED("fused E");
+            mpx::launch_fused_B<double>(h_step[b_args(m)], d_step + b_args(m), soff, st);
+            MPX_LAUNCHED("fused B");
         }
         for (int m = len - 1; m >= 0; --m) {
+            mpx::AdjHistory h;
             for (int c = 0; c < 3; ++c) {
-                a.E0[c] = hist[m][c];
-                a.E1[c] = hist[m + 1][c];
+                h.E0[c] = hist[m][c];
+                h.E1[c] = hist[m + 1][c];
             }
-            mpx::launch_adjoint_step(a, st);
+            mpx::launch_adjoint_step(a, h, st);
             MPX_LAUNCHED("adjoint step");
         }
     }
-    if ((rc = restore(fin))) return rc;
+    if ((rc = copy_state(fin, true, 0))) return rc;
     s->time = t0 + nsteps;
+    s->win_n = 0;
     // gradients to the host: dJ/dEps in full-storage layout, dJ/dchi summed in a fixed order
-    const GridDims &g = s->g;
-    const size_t nx2 = g.n[0] + 2, ny2 = g.n[1] + 2, nz2 = g.n[2] + 2;
-    std::vector<double> hb(s->cells);
-    if (dJ_deps) {
-        MPX_HIP(hipMemcpyAsync(hb.data(), a.epsb, s->cells * 8, hipMemcpyDeviceToHost, st));
-        MPX_HIP(hipStreamSynchronize(st));
-        for (size_t i = 0; i < nx2; ++i)
-            for (size_t j = 0; j < ny2; ++j)
-                for (size_t k = 0; k < nz2; ++k)
-                    dJ_deps[(i * ny2 + j) * nz2 + k] = hb[g.at((int)i, (int)j, (int)k)];
-    }
+    if (dJ_deps && (rc = box_copy(s, a.epsb, 8, false, 0, dJ_deps, nullptr))) return rc;
     if (dJ_dchi) {
-        MPX_HIP(hipMemcpyAsync(hb.data(), a.chib, s->cells * 8, hipMemcpyDeviceToHost, st));
-        MPX_HIP(hipStreamSynchronize(st));
         double sum = 0.0;
-        for (int i = 1; i <= g.n[0]; ++i)
-            for (int j = 1; j <= g.n[1]; ++j)
-                for (int k = 1; k <= g.n[2]; ++k) sum += hb[g.at(i, j, k)];
+        mpx::launch_sum_partials(a.chiw, mpx::adjoint_waves(s->g), dJ, 1.0, st);
+        MPX_LAUNCHED("chi gradient sum");
+        MPX_HIP(hipMemcpyAsync(&sum, dJ, sizeof(double), hipMemcpyDeviceToHost, st));
+        MPX_HIP(hipStreamSynchronize(st));
         *dJ_dchi = s->nonlin ? sum : 0.0;
     }
     MPX_HIP(hipStreamSynchronize(st));

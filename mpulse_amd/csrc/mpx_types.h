@@ -157,6 +157,7 @@ struct StepArgs {
     GridDims g;
     int periodic[3];
     T *E[3];
+    T *En[3];  // where the E kernel leaves the new E (E itself but for a kept history)
     T *B[3];
     unsigned *Elo, *Blo;  // float32 + residual storage: residual words of E and B, else null
     double2 *psi[3][3];  // [active pole][component]
@@ -271,33 +272,40 @@ struct PassArgs {
     int zper;                     // z periodic (single_periodic); 0: xy-periodic, z ghosts as stored
 };
 
-// Adjoint of one step of the fused float64 PLRC update without Lorentz poles.  The adjoints
-// of the six curl differences of each kernel are kept per cell in the off-diagonal slots
-// [dim][comp] (slot dim*2 + (comp > dim ? comp-1 : comp)): the difference along dim of field
-// component comp.
+// One CPML face of the adjoint: the range of the normal coordinate, the layer index
+// i s0 + j s1 + k - off, and the running adjoints of its two auxiliaries (mpx_adjoint.hip).  A
+// missing face has lo > hi.
+struct AdjFace {
+    int lo, hi;
+    int s0, s1, off;
+    double *A0, *A1;
+    const double *b, *c;
+    double idxn;
+};
+
+// Adjoint of one step of the fused float64 PLRC update; faces by [dimension][0 high, 1 low].
 struct AdjArgs {
     GridDims g;
     double dt, chi, eps;      // eps: uniform permittivity when epsf is null
     const double *epsf;
     const double *ikdE[3], *ikdH[3];
     double *lE[3], *lB[3];    // adjoints of E and B
-    double *dEb[6];           // adjoints of the E differences of the B update
-    double *dBb[6];           // adjoints of the B differences of the E update
-    double *epsb, *chib;      // per-cell gradient accumulators
-    const double *E0[3], *E1[3];  // forward E before and after the step
+    double *rb[3];            // adjoint of the E kernel's curl + current
+    double *epsb, *chiw;      // gradient accumulators: per cell, per wave (adjoint_waves)
     int kobj;                 // objective plane (z index)
     double wobj;
-    int nefaces, nhfaces;
-    CpmlFace eface[kMaxFaces];
-    CpmlFace hface[kMaxFaces];
-    int efbd[3][2], hfbd[3][2];
-    double *lpsiE[kMaxFaces][2], *lpsiH[kMaxFaces][2];  // adjoints of the CPML auxiliaries
+    AdjFace ef[3][2], hf[3][2];
+    int band;                 // rows of a band in the banded tile order
     // Lorentz poles: constants of the active poles and the adjoints of their accumulators,
     // [pole][component] at cell c (storage index)
     int np;
     PoleConsts pc;
     double sumChi0, sumXi0;
     double2 *lpsi[3][3];
+};
+// forward E before and after the step being reversed
+struct AdjHistory {
+    const double *E0[3], *E1[3];
 };
 
 // one run of a batch: its tile grid and the number of its first tile in the batch's list
