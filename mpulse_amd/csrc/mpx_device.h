@@ -82,6 +82,13 @@ __device__ __forceinline__ void stp(T *base, unsigned bo, T v)
     gst((T *)((char *)base + bo), v);
 }
 
+// A read-only table entry at a wave-uniform address, through the constant address space: a
+// scalar load into SGPRs, counted apart from the vector loads in flight
+__device__ __forceinline__ double kload(const double *p)
+{
+    return *(const __attribute__((address_space(4))) double *)p;
+}
+
 // The value a neighbouring lane of the wavefront holds, by DPP: lane_prev gives lane l the
 // value of lane l - 1 (wave_shr:1), lane_next that of lane l + 1 (wave_shl:1).  Lanes of a
 // fused-kernel wave hold consecutive z cells of one row, so the z neighbour of a cell is in
@@ -363,6 +370,123 @@ __device__ __forceinline__ void cpml_face(const CpmlFace &f, int coord, int l, d
     v1 = got<T, RES>(h1, wn, 1);
 }
 
+// ---- CPML by dimension (CpmlDim) ----
+//
+// A cell's auxiliaries are requested with its field words and used after them, those of all
+// three dimensions together: taken face by face, each with its descriptor, coefficients and
+// auxiliaries loaded on the spot, a layer cell paid up to three memory latencies in a row, and
+// a wave with any layer cell paid them whole.
+
+// An opaque use of a loaded value: conversions of it stay behind this point instead of moving up
+// to its load, where they would wait for memory.
+template <typename T>
+__device__ __forceinline__ void hold(T &v)
+{
+    asm volatile("" : "+v"(v));
+}
+
+// the side of the layer that holds coordinate x (0 high, 1 low), -1 outside
+__device__ __forceinline__ int cpml_side(const CpmlDim &D, int x)
+{
+    return x >= D.lo[0] && x <= D.hi[0] ? 0 : (x >= D.lo[1] && x <= D.hi[1] ? 1 : -1);
+}
+__device__ __forceinline__ int cpml_index(const CpmlDim &D, int side, int i, int j, int k)
+{
+    return i * D.s0 + j * D.s1 + k + (side == 0 ? D.off[0] : D.off[1]);
+}
+// the two auxiliaries of a cell as stored
+template <typename T, bool RES>
+struct Aux {
+    T o0, o1;
+    unsigned w;
+};
+template <typename T, bool RES>
+__device__ __forceinline__ Aux<T, RES> cpml_load(const CpmlDim &D, int l)
+{
+    // ordinary loads: a face row covers only part of a cache line (z faces: 16 cells), and the
+    // rest of the line is read by the neighbouring row
+    return {gld((const T *)D.o0 + l), gld((const T *)D.o1 + l), lo_ld<RES>(D.orw, l)};
+}
+// The new auxiliaries from the old (x: loaded from index l), the coordinate and the cell's
+// differences; stored with `store`.  v0, v1: the stored values, which the current sums see.
+// E side: CPMLBorderECurrent::stepScheme, src/cpml_border.cpp:398-425 (psi0 gets -c d1/dx);
+// H side: CPMLBorderHCurrent::stepScheme, src/cpml_border.cpp:499-527 (psi0 gets +c d1/dx).
+template <typename T, bool HSIDE, bool RES>
+__device__ __forceinline__ void cpml_update(const CpmlDim &D, int side, int coord, int l, const Aux<T, RES> &x, double d1,
+                                            double d0, bool store, double &v0, double &v1)
+{
+    const double *line = D.bc + (2 * side * D.len + coord);
+    const double bq = gld(line), cq = gld(line + D.len);
+    T r0 = x.o0, r1 = x.o1;
+    hold(r0);  // decoded here, not where they were requested
+    hold(r1);
+    const double a0 = got<T, RES>(r0, x.w, 0), a1 = got<T, RES>(r1, x.w, 1);
+    double n0, n1;
+    if (HSIDE) {
+        n0 = bq * a0 + cq * d1 * D.idxn;
+        n1 = bq * a1 - cq * d0 * D.idxn;
+    } else {
+        n0 = bq * a0 - cq * d1 * D.idxn;
+        n1 = bq * a1 + cq * d0 * D.idxn;
+    }
+    unsigned wn = 0;
+    const T h0 = put<T, RES>(n0, wn, 0), h1 = put<T, RES>(n1, wn, 1);
+    if (store) {
+        gst((T *)D.p0 + l, h0);
+        gst((T *)D.p1 + l, h1);
+        if (RES) gst(D.rw + l, wn);
+    }
+    v0 = got<T, RES>(h0, wn, 0);
+    v1 = got<T, RES>(h1, wn, 1);
+}
+// A cell's part in the layers of the three dimensions: its sides and what was loaded for them
+template <typename T, bool RES>
+struct CellCpml {
+    int side[3];
+    Aux<T, RES> x[3];
+};
+template <typename T, bool RES>
+__device__ __forceinline__ void cpml_request(const CpmlDim D[3], int i, int j, int k, bool live, CellCpml<T, RES> &s)
+{
+    const int at[3] = {i, j, k};
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        s.side[d] = live ? cpml_side(D[d], at[d]) : -1;
+        // a wave with no cell in these layers skips them; in the others every lane loads, so that no
+        // value is merged and waited for here (lanes outside take the block's first element)
+        if (__ballot(s.side[d] >= 0))
+            s.x[d] = cpml_load<T, RES>(D[d], s.side[d] >= 0 ? cpml_index(D[d], s.side[d], i, j, k) : 0);
+    }
+}
+// The current totals gain the cell's auxiliaries in the reference's list order: faces N,S (y),
+// E,W (x), U,D (z), the high face first.  df[d][0], df[d][1]: the differences along d of the field
+// components d + 1 and d + 2, which feed psi1 and psi0; those feed the currents d + 2 and d + 1.
+template <typename T, bool HSIDE, bool RES>
+__device__ __forceinline__ void cpml_add(const CpmlDim D[3], int i, int j, int k, const CellCpml<T, RES> &s,
+                                         const double df[3][2], bool store, double J[3])
+{
+    const int at[3] = {i, j, k};
+#pragma unroll
+    for (int u = 0; u < 3; ++u) {
+        constexpr int order[3] = {1, 0, 2};
+        const int d = order[u], c0 = (d + 1) % 3, c1 = (d + 2) % 3;
+        if (s.side[d] >= 0) {
+            double v0, v1;
+            cpml_update<T, HSIDE, RES>(D[d], s.side[d], at[d], cpml_index(D[d], s.side[d], i, j, k), s.x[d], df[d][1],
+                                       df[d][0], store, v0, v1);
+            J[c0] += v0;
+            J[c1] += v1;
+            if (D[d].two && s.side[d] == 0 && at[d] >= D[d].lo[1] && at[d] <= D[d].hi[1]) {
+                const int l = cpml_index(D[d], 1, i, j, k);
+                cpml_update<T, HSIDE, RES>(D[d], 1, at[d], l, cpml_load<T, RES>(D[d], l), df[d][1], df[d][0], store, v0,
+                                           v1);
+                J[c0] += v0;
+                J[c1] += v1;
+            }
+        }
+    }
+}
+
 // 32-bit layer index of cell (i, j, k) in a face box
 __device__ __forceinline__ int layer_index(const CpmlFace &f, int i, int j, int k)
 {
@@ -420,6 +544,43 @@ __device__ __forceinline__ void band_tile(int nbx, int nby, int nbz, int R, int 
     rem /= nbx;
     by = b * R + rem % rows;
     bz = rem / rows;
+}
+
+// Block -> tile of the fused kernels from a map made on the host (mpx_types.h): the orders above
+// with multiplications in place of the divisions, which took some 150 instructions and several
+// dependent argument loads at the head of every wave.
+__device__ __forceinline__ unsigned fast_div(unsigned t, const FastDiv &f)
+{
+    return (unsigned)(((unsigned long long)t * f.m) >> f.sh);
+}
+__device__ __forceinline__ void map_tile(const TileMap &M, int &bx, int &by, int &bz)
+{
+    const unsigned lin = blockIdx.x;
+    unsigned t = lin < M.per * 8u ? (lin & 7u) * M.per + (lin >> 3) : lin;
+    if (M.order == 2) {
+        if (M.rev) t = M.total - 1u - t;
+        const unsigned b = fast_div(t, M.full);
+        unsigned rem = t - b * M.full.d;
+        const bool last = (int)b == M.nbands - 1;
+        const unsigned q = fast_div(rem, M.first);
+        bx = rem - q * M.first.d;
+        const unsigned rows = last ? M.rlast.d : M.rband.d;
+        const unsigned z = last ? fast_div(q, M.rlast) : fast_div(q, M.rband);
+        by = b * M.rband.d + (q - z * rows);
+        bz = z;
+    } else {
+        const unsigned q = fast_div(t, M.first), z = fast_div(q, M.second);
+        const int u = t - q * M.first.d, v = q - z * M.second.d;
+        if (M.order == 1) {
+            bz = u;
+            bx = v;
+            by = z;
+        } else {
+            bx = u;
+            by = v;
+            bz = z;
+        }
+    }
 }
 
 __device__ __forceinline__ void fused_tile_of(int order, int band, int rev, int nbx, int nby, int nbz, int &bx,

@@ -16,66 +16,210 @@
 
 namespace mpx {
 
+// A cell's place.  Blocks of 64 z cells x 4 rows: a wave holds cells of one row, so the row's
+// offset is wave-uniform and a lane adds k alone -- one 32-bit offset register for every grid
+// and neighbour row, where an index of its own took a 64-bit address for each.  LIN blocks (256
+// consecutive y-z cells) cross rows and keep a lane's own index.
+template <bool LIN>
+struct At;
+template <>
+struct At<false> {
+    size_t row;  // storage offset of k = 0
+    unsigned k;
+    __device__ __forceinline__ At shift(int d) const { return {row + (long long)d, k}; }  // d: wave-uniform
+    __device__ __forceinline__ At along(int d) const { return {row, k + d}; }
+    template <typename T>
+    __device__ __forceinline__ T ld(const T *p) const
+    {
+        return ldp(p + row, k * (unsigned)sizeof(T));
+    }
+    template <typename T>
+    __device__ __forceinline__ T once(const T *p) const
+    {
+        return ldp_once(p + row, k * (unsigned)sizeof(T));
+    }
+    template <typename T>
+    __device__ __forceinline__ void st(T *p, T v) const
+    {
+        stp(p + row, k * (unsigned)sizeof(T), v);
+    }
+    template <typename T>
+    __device__ __forceinline__ void st_once(T *p, T v) const
+    {
+        stp_once(p + row, k * (unsigned)sizeof(T), v);
+    }
+    // the accumulators (psi_at): the row's chunk is uniform, a lane counts on from it
+    __device__ __forceinline__ size_t psi_row() const { return ((row + PSI_SHIFT) >> 6) * 192; }
+    __device__ __forceinline__ unsigned psi_lane() const
+    {
+        const unsigned t = (unsigned)((row + PSI_SHIFT) & 63) + k;
+        return (t >> 6) * 192 + (t & 63);
+    }
+};
+template <>
+struct At<true> {
+    int c;
+    __device__ __forceinline__ At shift(int d) const { return {c + d}; }
+    __device__ __forceinline__ At along(int d) const { return {c + d}; }
+    template <typename T>
+    __device__ __forceinline__ T ld(const T *p) const
+    {
+        return gld(p + c);
+    }
+    template <typename T>
+    __device__ __forceinline__ T once(const T *p) const
+    {
+        return load_once(p + c);
+    }
+    template <typename T>
+    __device__ __forceinline__ void st(T *p, T v) const
+    {
+        gst(p + c, v);
+    }
+    template <typename T>
+    __device__ __forceinline__ void st_once(T *p, T v) const
+    {
+        store_once(p + c, v);
+    }
+    __device__ __forceinline__ size_t psi_row() const { return 0; }
+    __device__ __forceinline__ unsigned psi_lane() const { return (unsigned)psi_at(c); }
+};
+
+// Two or three components of a cell and its residual word, as stored
+template <typename T, bool RES>
+struct Words {
+    T x, y, z;
+    unsigned w;
+};
+template <bool RES, typename A, typename T>
+__device__ __forceinline__ Words<T, RES> read3(const A &at, const T *const f[3], const unsigned *lo)
+{
+    Words<T, RES> r;
+    r.x = at.ld(f[0]);
+    r.y = at.ld(f[1]);
+    r.z = at.ld(f[2]);
+    r.w = RES ? at.ld(lo) : 0u;
+    return r;
+}
+template <bool RES, typename A, typename T>
+__device__ __forceinline__ Words<T, RES> read3_once(const A &at, const T *const f[3], const unsigned *lo)
+{
+    Words<T, RES> r;
+    r.x = at.once(f[0]);
+    r.y = at.once(f[1]);
+    r.z = at.once(f[2]);
+    r.w = RES ? at.once(lo) : 0u;
+    return r;
+}
+// components p and q only
+template <typename T, bool RES>
+struct Pair {
+    T p, q;
+    unsigned w;
+};
+template <bool RES, typename A, typename T>
+__device__ __forceinline__ Pair<T, RES> read2(const A &at, const T *fp, const T *fq, const unsigned *lo)
+{
+    Pair<T, RES> r;
+    r.p = at.ld(fp);
+    r.q = at.ld(fq);
+    r.w = RES ? at.ld(lo) : 0u;
+    return r;
+}
+
+// accumulators of the active poles at a cell: component q of pole n sits 64 elements after
+// component q - 1
+template <int NP, bool LIN>
+struct PsiCell {
+    double2 *b[NP > 0 ? NP : 1];
+    struct Comp {
+        double2 *p;
+        __device__ double2 &operator[](size_t) const { return *p; }
+    };
+    struct Pole {
+        double2 *p;
+        __device__ Comp operator[](int q) const { return Comp{p + 64 * q}; }
+    };
+    __device__ Pole operator[](int n) const { return Pole{b[n]}; }
+};
+
 // Fused E side of one step.  A thread owns one (j, k) column segment of L cells along x and
 // walks it plane by plane, keeping B of the previous plane in registers for the x difference.
+//
+// Bound by memory latency at the occupancy its registers allow: a wave's life is one round of
+// loads, the update and its stores, so whatever waits for memory before that round is issued
+// adds a latency to every wave.  Every word of a cell -- its own, the three lower neighbours',
+// the accumulators', the CPML auxiliaries' -- is therefore requested unconditionally before the
+// first is used.  The z - 1 neighbour is in the previous lane (DPP) except for the first lane of
+// a wave and the first cell of a row; that word too is loaded by all lanes (at their own cell's
+// address where it is not needed), since under a branch its decoding waited for it at once.
+// Measured against that form (face by face CPML, per-lane 64-bit addresses, tile divisions in
+// the kernel), us for E and B with a 16-cell CPML and one pole: 512^3 float32 + residual 3627 +
+// 1707 -> 3166 + 1345, float32 3184 + 1054 -> 2832 + 1059, float64 4204 + 2187 -> 3764 + 1969;
+// 256^3 float32 + residual 513 + 268 -> 464 + 236; 64^3 float64 14.8 + 14.2 -> 14.4 + 11.3.
 template <typename T, int NP, bool NONLIN, bool CPML, int L, bool LIN = false, bool RES = false>
 __device__ __forceinline__ void fused_E_tile(const StepArgs<T> &a, int tbx, int tby, int tbz, int soff)
 {
-    using V = typename Word<T, RES>::V;
     const GridDims &g = a.g;
     const int one[3] = {1, 1, 1};
     int j, k;
     tile_jk<LIN>(g, one, tbx, tby, j, k);
+    if (!LIN) j = __builtin_amdgcn_readfirstlane(j);
     const int i0 = tbz * L + 1;
     if (k > g.n[2] || j > g.n[1] || i0 > g.n[0]) return;
     const int i1 = min(i0 + L - 1, g.n[0]);
     const int sx = (int)g.sx, pz = g.pz;
     const int ojm = (j == 1 && a.periodic[1]) ? (g.n[1] - 1) * pz : -pz;
     const int okm = (k == 1 && a.periodic[2]) ? (g.n[2] - 1) : -1;
-    int c = i0 * sx + j * pz + k + g.z0;
-    const T *Bx = a.B[0], *By = a.B[1], *Bz = a.B[2];
-    const int cim = (i0 == 1 && a.periodic[0]) ? c + (g.n[0] - 1) * sx : c - sx;
-    const unsigned wim = lo_ld<RES>(a.Blo, cim);
-    double bz_im = (double)rd<T, RES>(Bz, wim, 2, cim), by_im = (double)rd<T, RES>(By, wim, 1, cim);
-    bool iny[2] = {false, false}, inz[2] = {false, false};
-    if (CPML) {
-        in_faces(a.face_by_dim, a.face, 1, j, iny);
-        in_faces(a.face_by_dim, a.face, 2, k, inz);
-    }
-    const double kdy = gld(a.ikdE[1] + j), kdz = gld(a.ikdE[2] + k);
+    const int oim = (i0 == 1 && a.periodic[0]) ? (g.n[0] - 1) * sx : -sx;
+    At<LIN> c;
+    if constexpr (LIN) c = {i0 * sx + j * pz + k + g.z0};
+    else c = {g.at(i0, j, 0), (unsigned)k};
+    const T *const *B = a.B;
+    const bool zload = threadIdx.x == 0 || k == 1;
+    const Pair<T, RES> bim = read2<RES>(c.shift(oim), B[1], B[2], a.Blo);
+    double by_im = 0.0, bz_im = 0.0;
+    const double kdy = LIN ? gld(a.ikdE[1] + j) : kload(a.ikdE[1] + j), kdz = gld(a.ikdE[2] + k);
 #pragma unroll
-    for (int u = 0; u < L; ++u, c += sx) {
+    for (int u = 0; u < L; ++u) {
         const int i = i0 + u;
         if (i > i1) break;
-        // z neighbours: the first lane of a wave and the first cell of a row load them, every
-        // other lane takes them from the previous lane (the loads are issued first, so that one
-        // wait covers them and the cell's own loads)
-        const bool zload = threadIdx.x == 0 || k == 1;
-        V bym = (V)0, bxm = (V)0;
-        if (zload) {
-            const unsigned wm = lo_ld<RES>(a.Blo, c + okm);
-            bym = rd<T, RES>(By, wm, 1, c + okm);
-            bxm = rd<T, RES>(Bx, wm, 0, c + okm);
-        }
-        const unsigned wb = lo_ld<RES>(a.Blo, c);
-        const V bxt = rd<T, RES>(Bx, wb, 0, c), byt = rd<T, RES>(By, wb, 1, c);
-        const double bx = bxt, by = byt, bz = rd<T, RES>(Bz, wb, 2, c);
-        // E and the pole accumulators are read before any store of the cell (the CPML
-        // auxiliaries), so that all its reads leave together
-        const unsigned we = lo_once<RES>(a.Elo, c);
-        double ex = (double)rd_once<T, RES>(a.E[0], we, 0, c), ey = (double)rd_once<T, RES>(a.E[1], we, 1, c);
-        double ez = (double)rd_once<T, RES>(a.E[2], we, 2, c);
+        const Words<T, RES> b = read3<RES>(c, B, a.Blo);
+        const Pair<T, RES> bk = read2<RES>(c.along(zload ? okm : 0), B[0], B[1], a.Blo);
+        const Pair<T, RES> bj = read2<RES>(c.shift(ojm), B[0], B[2], a.Blo);
+        const Words<T, RES> e = read3_once<RES>(c, (const T *const *)a.E, a.Elo);
+        const size_t prow = c.psi_row();
+        const unsigned plane = c.psi_lane();
         PsiRegs<NP> pr;
+        PsiCell<NP, LIN> ps;
 #pragma unroll
-        for (int n = 0; n < NP; ++n)
+        for (int n = 0; n < NP; ++n) {
+            ps.b[n] = a.psi[n][0] + prow + plane;
 #pragma unroll
-            for (int q = 0; q < 3; ++q) pr.v[n][q] = load_once(&a.psi[n][q][psi_at(c)]);
-        const unsigned wj = lo_ld<RES>(a.Blo, c + ojm);
-        const double dBz_y = bz - (double)rd<T, RES>(Bz, wj, 2, c + ojm);
-        const double dBx_y = bx - (double)rd<T, RES>(Bx, wj, 0, c + ojm);
-        const V bys = lane_prev(byt), bxs = lane_prev(bxt);
-        const double dBy_z = by - (double)(zload ? bym : bys);
-        const double dBx_z = bx - (double)(zload ? bxm : bxs);
+            for (int q = 0; q < 3; ++q) pr.v[n][q] = ldp_once(a.psi[n][0] + prow + 64 * q, plane * 16u);
+        }
+        CellCpml<T, RES> cx;
+        if (CPML) cpml_request<T, RES>(a.cd, i, j, k, true, cx);
+        double epsc = 0.0;
+        if (a.epsf) epsc = c.ld(a.epsf);
+        const double bx = got<T, RES>(b.x, b.w, 0), by = got<T, RES>(b.y, b.w, 1), bz = got<T, RES>(b.z, b.w, 2);
+        if (u == 0) {
+            by_im = got<T, RES>(bim.p, bim.w, 1);
+            bz_im = got<T, RES>(bim.q, bim.w, 2);
+        }
+        double ex = got<T, RES>(e.x, e.w, 0), ey = got<T, RES>(e.y, e.w, 1), ez = got<T, RES>(e.z, e.w, 2);
+        const double dBz_y = bz - got<T, RES>(bj.q, bj.w, 2);
+        const double dBx_y = bx - got<T, RES>(bj.p, bj.w, 0);
+        double bxs, bys;
+        if constexpr (RES) {
+            bxs = lane_prev(bx);
+            bys = lane_prev(by);
+        } else {
+            bxs = (double)lane_prev(b.x);
+            bys = (double)lane_prev(b.y);
+        }
+        const double dBx_z = bx - (zload ? got<T, RES>(bk.p, bk.w, 0) : bxs);
+        const double dBy_z = by - (zload ? got<T, RES>(bk.q, bk.w, 1) : bys);
         const double dBz_x = bz - bz_im;
         const double dBy_x = by - by_im;
         bz_im = bz;
@@ -83,223 +227,155 @@ __device__ __forceinline__ void fused_E_tile(const StepArgs<T> &a, int tbx, int 
         // the plasma OptField and the plasma current run before the E update, on E of this step
         double sg = 0.0, jpv[3] = {0.0, 0.0, 0.0};
         if (a.plasma || a.pcur) {
-            double r = gld(a.rho + c);
+            double r = c.ld(a.rho);
+            double jp[3] = {0.0, 0.0, 0.0};
+            if (a.pcur)
+                for (int q = 0; q < 3; ++q) jp[q] = c.ld(a.jp[q]);
             if (a.plasma) {
                 sg = a.pw * plasma_density_cell(ex, ey, ez, r, a.pn, a.pm, a.pk - 1);
-                gst(a.rho + c, r);
-                gst(a.sigma + c, sg);
+                c.st(a.rho, r);
+                c.st(a.sigma, sg);
             }
             if (a.pcur) {
                 const double rt = r + a.rho_bg, ev[3] = {ex, ey, ez};
                 for (int q = 0; q < 3; ++q) {
-                    jpv[q] = plasma_current_comp(gld(a.jp[q] + c), ev[q], rt, a.gdtn, a.gdtd, a.emdt);
-                    gst(a.jp[q] + c, jpv[q]);
+                    jpv[q] = plasma_current_comp(jp[q], ev[q], rt, a.gdtn, a.gdtd, a.emdt);
+                    c.st(a.jp[q], jpv[q]);
                 }
             }
         }
         // current totals in list order: the CPML and sheet groups, the plasma current at its place
-        double jx = 0.0, jy = 0.0, jz = 0.0;
+        double J[3] = {0.0, 0.0, 0.0};
         auto add_cpml = [&]() {
             if (CPML) {
-                // current totals in the reference's list order N,S (y), E,W (x), U,D (z); within a
-                // dimension the high face comes first in that list
-#pragma unroll
-                for (int s = 0; s < 2; ++s)
-                    if (iny[s]) {
-                        const CpmlFace &f = a.face[a.face_by_dim[1][s]];
-                        double v0, v1;
-                        cpml_face<T, false, RES>(f, j, layer_index(f, i, j, k), dBx_y, dBz_y, v0, v1);
-                        jz += v0;
-                        jx += v1;
-                    }
-                bool inx[2];
-                in_faces(a.face_by_dim, a.face, 0, i, inx);
-#pragma unroll
-                for (int s = 0; s < 2; ++s)
-                    if (inx[s]) {
-                        const CpmlFace &f = a.face[a.face_by_dim[0][s]];
-                        double v0, v1;
-                        cpml_face<T, false, RES>(f, i, layer_index(f, i, j, k), dBz_x, dBy_x, v0, v1);
-                        jy += v0;
-                        jz += v1;
-                    }
-#pragma unroll
-                for (int s = 0; s < 2; ++s)
-                    if (inz[s]) {
-                        const CpmlFace &f = a.face[a.face_by_dim[2][s]];
-                        double v0, v1;
-                        cpml_face<T, false, RES>(f, k, layer_index(f, i, j, k), dBy_z, dBx_z, v0, v1);
-                        jx += v0;
-                        jy += v1;
-                    }
+                const double df[3][2] = {{dBy_x, dBz_x}, {dBz_y, dBx_y}, {dBx_z, dBy_z}};
+                cpml_add<T, false, RES>(a.cd, i, j, k, cx, df, true, J);
             }
         };
         auto add_plasma = [&](int pos) {
             if (a.pcur && a.pcur_pos == pos) {
-                jx += jpv[0];
-                jy += jpv[1];
-                jz += jpv[2];
+                J[0] += jpv[0];
+                J[1] += jpv[1];
+                J[2] += jpv[2];
             }
         };
         add_plasma(0);
         if (a.sheets_first)
-            add_sheets(a, i, j, k, soff, jx, jy, jz);
+            add_sheets(a, i, j, k, soff, J[0], J[1], J[2]);
         else
             add_cpml();
         add_plasma(1);
         if (a.sheets_first)
             add_cpml();
         else
-            add_sheets(a, i, j, k, soff, jx, jy, jz);
+            add_sheets(a, i, j, k, soff, J[0], J[1], J[2]);
         add_plasma(2);
         double idenom = a.idenom, numer = a.numer;
-        if (a.epsf || a.plasma) {
-            double denom;
-            cell_eps<NONLIN>(a, (size_t)c, 0.5 * sg * a.dt, denom, numer);
+        if (a.epsf || a.plasma) {  // cell_eps with the permittivity read above and Sigma dt / 2
+            const double ec = a.epsf ? epsc : a.eps, sgh = 0.5 * sg * a.dt;
+            const double denom = NONLIN ? ec + a.sumChi0 - a.sumXi0 + sgh : ec + (a.sumChi0 - a.sumXi0) + sgh;
+            numer = ec - a.sumXi0 - sgh;
             idenom = 1.0 / denom;
         }
         unsigned fl = 0;
-        plrc_e_update_pp<NP, NONLIN, true>(ex, ey, ez, dBz_y, dBy_z, dBx_z, dBz_x, dBy_x, dBx_y, gld(a.ikdE[0] + i), kdy,
-                                           kdz, jx, jy, jz, pr, a.psi, (size_t)c, true, a.pc, a.dt, idenom, numer,
+        plrc_e_update_pp<NP, NONLIN, true>(ex, ey, ez, dBz_y, dBy_z, dBx_z, dBz_x, dBy_x, dBx_y, kload(a.ikdE[0] + i), kdy,
+                                           kdz, J[0], J[1], J[2], pr, ps, (size_t)0, true, a.pc, a.dt, idenom, numer,
                                            a.chi, a.ncap, &fl);
         report(a.status, fl | finite_flag(ex, ey, ez));
         unsigned wn = 0;
         const T hx = put<T, RES>(ex, wn, 0), hy = put<T, RES>(ey, wn, 1), hz = put<T, RES>(ez, wn, 2);
-        store_once(&a.En[0][c], hx);
-        store_once(&a.En[1][c], hy);
-        store_once(&a.En[2][c], hz);
-        if (RES) store_once(&a.Elo[c], wn);
+        c.st_once(a.En[0], hx);
+        c.st_once(a.En[1], hy);
+        c.st_once(a.En[2], hz);
+        if (RES) c.st_once(a.Elo, wn);
+        c = c.shift(sx);
     }
 }
 
-// Fused B side of one step: a thread walks L planes along x keeping E of the next plane in
-// registers as the centre of the following iteration.
+// Fused B side of one step: a thread walks L planes along x keeping E of the next plane as the
+// centre of the following iteration.  Bound and built as the E side: every word of the L planes
+// is requested before the first is used, the z + 1 neighbour by all lanes.
 template <typename T, bool CPML, int L, bool LIN = false, bool RES = false>
 __device__ __forceinline__ void fused_B_tile(const StepArgs<T> &a, int tbx, int tby, int tbz, int soff)
 {
-    using V = typename Word<T, RES>::V;
     const GridDims &g = a.g;
     int j, k;
     tile_jk<LIN>(g, a.blo, tbx, tby, j, k);
+    if (!LIN) j = __builtin_amdgcn_readfirstlane(j);
     const int i0 = tbz * L + a.blo[0];
     if (k > g.n[2] || j > g.n[1] || i0 > g.n[0]) return;
     const int i1 = min(i0 + L - 1, g.n[0]);
     const int sx = (int)g.sx, pz = g.pz;
     const int ojp = (j == g.n[1] && a.periodic[1]) ? -(g.n[1] - 1) * pz : pz;
     const int okp = (k == g.n[2] && a.periodic[2]) ? -(g.n[2] - 1) : 1;
-    int c = i0 * sx + j * pz + k + g.z0;
-    const T *Ex = a.E[0], *Ey = a.E[1], *Ez = a.E[2];
-    T *Bx = a.B[0], *By = a.B[1], *Bz = a.B[2];
-    // z neighbours: the last lane of a wave and the last cell of a row load them, every other
-    // lane takes them from the next lane
+    At<LIN> c;
+    if constexpr (LIN) c = {i0 * sx + j * pz + k + g.z0};
+    else c = {g.at(i0, j, 0), (unsigned)k};
+    const T *const *E = a.E;
     const bool zload = threadIdx.x == 63 || k == g.n[2];
-    V ezl[L][2];
-    if (zload) {
+    // per plane: E of the next plane, E_x and E_z of the next row, E_x and E_y of the next cell, B
+    const Words<T, RES> ec = read3<RES>(c, E, a.Elo);
+    Words<T, RES> en[L], b0[L];
+    Pair<T, RES> ej[L], ek[L];
 #pragma unroll
-        for (int u = 0; u < L; ++u) {
-            const int cu = c + u * sx;
-            ezl[u][0] = ezl[u][1] = (V)0;
-            if (i0 + u <= i1) {
-                const unsigned w = lo_ld<RES>(a.Elo, cu + okp);
-                ezl[u][0] = rd<T, RES>(Ey, w, 1, cu + okp);
-                ezl[u][1] = rd<T, RES>(Ex, w, 0, cu + okp);
-            }
+    for (int u = 0; u < L; ++u) {
+        const int i = i0 + u;
+        if (i > i1) break;
+        const At<LIN> cu = c.shift(u * sx);
+        en[u] = read3<RES>(cu.shift((i == g.n[0] && a.periodic[0]) ? -(g.n[0] - 1) * sx : sx), E, a.Elo);
+        ej[u] = read2<RES>(cu.shift(ojp), E[0], E[2], a.Elo);
+        ek[u] = read2<RES>(cu.along(zload ? okp : 0), E[0], E[1], a.Elo);
+        b0[u] = read3_once<RES>(cu, (const T *const *)a.B, a.Blo);
+    }
+    CellCpml<T, RES> cx;
+    if (CPML) cpml_request<T, RES>(a.cd, i0, j, k, true, cx);
+    const double kdy = LIN ? gld(a.ikdH[1] + j) : kload(a.ikdH[1] + j), kdz = gld(a.ikdH[2] + k);
+    T rx = ec.x, ry = ec.y;  // E_x, E_y of the centre as stored (float32 and float64)
+    double ex = got<T, RES>(ec.x, ec.w, 0), ey = got<T, RES>(ec.y, ec.w, 1), ez = got<T, RES>(ec.z, ec.w, 2);
+#pragma unroll
+    for (int u = 0; u < L; ++u) {
+        const int i = i0 + u;
+        if (i > i1) break;
+        const double ex1 = got<T, RES>(en[u].x, en[u].w, 0), ey1 = got<T, RES>(en[u].y, en[u].w, 1),
+                     ez1 = got<T, RES>(en[u].z, en[u].w, 2);
+        double exs, eys;
+        if constexpr (RES) {
+            exs = lane_next(ex);
+            eys = lane_next(ey);
+        } else {
+            exs = (double)lane_next(rx);
+            eys = (double)lane_next(ry);
         }
-    }
-    const unsigned w0 = lo_ld<RES>(a.Elo, c);
-    const V ex0 = rd<T, RES>(Ex, w0, 0, c), ey0 = rd<T, RES>(Ey, w0, 1, c), ez0 = rd<T, RES>(Ez, w0, 2, c);
-    double ex = ex0, ey = ey0, ez = ez0;
-    bool iny[2] = {false, false}, inz[2] = {false, false};
-    if (CPML) {
-        in_faces(a.face_by_dim, a.face, 1, j, iny);
-        in_faces(a.face_by_dim, a.face, 2, k, inz);
-    }
-    const double kdy = gld(a.ikdH[1] + j), kdz = gld(a.ikdH[2] + k);
-    // the E and B values of all L planes are read before the first store, so that they leave
-    // together (per plane: E at x+1, E_y and E_x at z+1, E_z and E_x at y+1, B)
-    V pe[L][7], pb[L][3];
-#pragma unroll
-    for (int u = 0; u < L; ++u) {
-        const int i = i0 + u;
-        if (i > i1) break;
-        const int cu = c + u * sx;
-        const int cip = (i == g.n[0] && a.periodic[0]) ? cu - (g.n[0] - 1) * sx : cu + sx;
-        const unsigned wx = lo_ld<RES>(a.Elo, cip), wy = lo_ld<RES>(a.Elo, cu + ojp);
-        const unsigned wbu = lo_once<RES>(a.Blo, cu);
-        pe[u][0] = rd<T, RES>(Ex, wx, 0, cip);
-        pe[u][1] = rd<T, RES>(Ey, wx, 1, cip);
-        pe[u][2] = rd<T, RES>(Ez, wx, 2, cip);
-        pe[u][5] = rd<T, RES>(Ez, wy, 2, cu + ojp);
-        pe[u][6] = rd<T, RES>(Ex, wy, 0, cu + ojp);
-        pb[u][0] = rd_once<T, RES>(Bx, wbu, 0, cu);
-        pb[u][1] = rd_once<T, RES>(By, wbu, 1, cu);
-        pb[u][2] = rd_once<T, RES>(Bz, wbu, 2, cu);
-    }
-#pragma unroll
-    for (int u = 0; u < L; ++u) {
-        if (i0 + u > i1) break;
-        // E at z+1: the next lane's centre value of the same plane
-        const V sy = lane_next(u == 0 ? ey0 : pe[u - 1][1]), sx_ = lane_next(u == 0 ? ex0 : pe[u - 1][0]);
-        pe[u][3] = zload ? ezl[u][0] : sy;
-        pe[u][4] = zload ? ezl[u][1] : sx_;
-    }
-#pragma unroll
-    for (int u = 0; u < L; ++u, c += sx) {
-        const int i = i0 + u;
-        if (i > i1) break;
-        const double ex1 = pe[u][0], ey1 = pe[u][1], ez1 = pe[u][2];
-        const double dEy_z = (double)pe[u][3] - ey;
-        const double dEx_z = (double)pe[u][4] - ex;
-        const double dEz_y = (double)pe[u][5] - ez;
-        const double dEx_y = (double)pe[u][6] - ex;
+        const double dEx_z = (zload ? got<T, RES>(ek[u].p, ek[u].w, 0) : exs) - ex;
+        const double dEy_z = (zload ? got<T, RES>(ek[u].q, ek[u].w, 1) : eys) - ey;
+        const double dEx_y = got<T, RES>(ej[u].p, ej[u].w, 0) - ex;
+        const double dEz_y = got<T, RES>(ej[u].q, ej[u].w, 2) - ez;
         const double dEz_x = ez1 - ez;
         const double dEy_x = ey1 - ey;
-        double mx = 0.0, my = 0.0, mz = 0.0;
-        if (a.sheets_first) add_sheets(a, i, j, k, soff, mx, my, mz);
+        double M[3] = {0.0, 0.0, 0.0};
+        if (a.sheets_first) add_sheets(a, i, j, k, soff, M[0], M[1], M[2]);
         if (CPML) {
-#pragma unroll
-            for (int s = 0; s < 2; ++s)
-                if (iny[s]) {
-                    const CpmlFace &f = a.face[a.face_by_dim[1][s]];
-                    double v0, v1;  // psi0 -> Mz from dEx_y, psi1 -> Mx from dEz_y
-                    cpml_face<T, true, RES>(f, j, layer_index(f, i, j, k), dEx_y, dEz_y, v0, v1);
-                    mz += v0;
-                    mx += v1;
-                }
-            bool inx[2];
-            in_faces(a.face_by_dim, a.face, 0, i, inx);
-#pragma unroll
-            for (int s = 0; s < 2; ++s)
-                if (inx[s]) {
-                    const CpmlFace &f = a.face[a.face_by_dim[0][s]];
-                    double v0, v1;  // psi0 -> My from dEz_x, psi1 -> Mz from dEy_x
-                    cpml_face<T, true, RES>(f, i, layer_index(f, i, j, k), dEz_x, dEy_x, v0, v1);
-                    my += v0;
-                    mz += v1;
-                }
-#pragma unroll
-            for (int s = 0; s < 2; ++s)
-                if (inz[s]) {
-                    const CpmlFace &f = a.face[a.face_by_dim[2][s]];
-                    double v0, v1;  // psi0 -> Mx from dEy_z, psi1 -> My from dEx_z
-                    cpml_face<T, true, RES>(f, k, layer_index(f, i, j, k), dEy_z, dEx_z, v0, v1);
-                    mx += v0;
-                    my += v1;
-                }
+            const CellCpml<T, RES> now = cx;
+            if (u + 1 < L && i < i1) cpml_request<T, RES>(a.cd, i + 1, j, k, true, cx);  // the next plane's
+            const double df[3][2] = {{dEy_x, dEz_x}, {dEz_y, dEx_y}, {dEx_z, dEy_z}};
+            cpml_add<T, true, RES>(a.cd, i, j, k, now, df, true, M);
         }
-        if (!a.sheets_first) add_sheets(a, i, j, k, soff, mx, my, mz);
-        const double kdx = gld(a.ikdH[0] + i);
+        if (!a.sheets_first) add_sheets(a, i, j, k, soff, M[0], M[1], M[2]);
+        const double kdx = kload(a.ikdH[0] + i);
         unsigned wn = 0;
-        const T hx = put<T, RES>((double)pb[u][0] + a.dt * ((dEy_z * kdz - dEz_y * kdy) + mx), wn, 0);
-        const T hy = put<T, RES>((double)pb[u][1] + a.dt * ((dEz_x * kdx - dEx_z * kdz) + my), wn, 1);
-        const T hz = put<T, RES>((double)pb[u][2] + a.dt * ((dEx_y * kdy - dEy_x * kdx) + mz), wn, 2);
-        store_once(&Bx[c], hx);
-        store_once(&By[c], hy);
-        store_once(&Bz[c], hz);
-        if (RES) store_once(&a.Blo[c], wn);
+        const T hx = put<T, RES>(got<T, RES>(b0[u].x, b0[u].w, 0) + a.dt * ((dEy_z * kdz - dEz_y * kdy) + M[0]), wn, 0);
+        const T hy = put<T, RES>(got<T, RES>(b0[u].y, b0[u].w, 1) + a.dt * ((dEz_x * kdx - dEx_z * kdz) + M[1]), wn, 1);
+        const T hz = put<T, RES>(got<T, RES>(b0[u].z, b0[u].w, 2) + a.dt * ((dEx_y * kdy - dEy_x * kdx) + M[2]), wn, 2);
+        const At<LIN> cu = c.shift(u * sx);
+        cu.st_once(a.B[0], hx);
+        cu.st_once(a.B[1], hy);
+        cu.st_once(a.B[2], hz);
+        if (RES) cu.st_once(a.Blo, wn);
         ex = ex1;
         ey = ey1;
         ez = ez1;
+        rx = en[u].x;
+        ry = en[u].y;
     }
 }
 
@@ -316,19 +392,18 @@ struct FusedEWaves {
 
 template <typename T, int NP, bool NONLIN, bool CPML, int L, bool RES = false>
 __global__ __attribute__((amdgpu_waves_per_eu(FusedEWaves<T, NP, NONLIN, L, RES>::v))) __launch_bounds__(256) void k_fused_E(
-    const StepArgs<T> *__restrict__ pa, int nbx, int nby, int nbz, int soff)
+    const StepArgs<T> *__restrict__ pa, TileMap map, int soff)
 {
     int tbx, tby, tbz;
-    fused_tile_of(pa->order, pa->band, pa->rev, nbx, nby, nbz, tbx, tby, tbz);
+    map_tile(map, tbx, tby, tbz);
     fused_E_tile<T, NP, NONLIN, CPML, L, false, RES>(*pa, tbx, tby, tbz, soff);
 }
 
 template <typename T, bool CPML, int L, bool RES = false>
-__global__ __launch_bounds__(256) void k_fused_B(const StepArgs<T> *__restrict__ pa, int nbx, int nby, int nbz,
-                                                 int soff)
+__global__ __launch_bounds__(256) void k_fused_B(const StepArgs<T> *__restrict__ pa, TileMap map, int soff)
 {
     int tbx, tby, tbz;
-    fused_tile_of(pa->order, pa->band, pa->rev, nbx, nby, nbz, tbx, tby, tbz);
+    map_tile(map, tbx, tby, tbz);
     fused_B_tile<T, CPML, L, false, RES>(*pa, tbx, tby, tbz, soff);
 }
 
@@ -433,10 +508,10 @@ static void launch_fused_E_L(const StepArgs<T> &a, const StepArgs<T> *dev, int n
 {
     const GridDims &g = a.g;
     int nbx = (g.n[2] + 63) / 64, nby = (g.n[1] + 3) / 4, nbz = (g.n[0] + L - 1) / L;
-    dim3 blk(64, 4);
-    dim3 grd(nbx, nby, nbz);
+    dim3 blk(64, 4), grd((unsigned)nbx * nby * nbz);
+    const TileMap map = tile_map(nbx, nby, nbz, a.order, a.band, a.rev);
     bool cp = a.nfaces > 0;
-#define MPX_FE(NPV, NL, CP) hipLaunchKernelGGL((k_fused_E<T, NPV, NL, CP, L, RES>), grd, blk, 0, s, dev, nbx, nby, nbz, soff)
+#define MPX_FE(NPV, NL, CP) hipLaunchKernelGGL((k_fused_E<T, NPV, NL, CP, L, RES>), grd, blk, 0, s, dev, map, soff)
 #define MPX_FE_NP(NL, CP)            \
     switch (np) {                    \
     case 0: MPX_FE(0, NL, CP); break; \
@@ -476,12 +551,12 @@ static void launch_fused_B_L(const StepArgs<T> &a, const StepArgs<T> *dev, int s
     const GridDims &g = a.g;
     int nk = g.n[2] - a.blo[2] + 1, nj = g.n[1] - a.blo[1] + 1, ni = g.n[0] - a.blo[0] + 1;
     int nbx = (nk + 63) / 64, nby = (nj + 3) / 4, nbz = (ni + L - 1) / L;
-    dim3 blk(64, 4);
-    dim3 grd(nbx, nby, nbz);
+    dim3 blk(64, 4), grd((unsigned)nbx * nby * nbz);
+    const TileMap map = tile_map(nbx, nby, nbz, a.order, a.band, a.rev);
     if (a.nfaces > 0)
-        hipLaunchKernelGGL((k_fused_B<T, true, L, RES>), grd, blk, 0, s, dev, nbx, nby, nbz, soff);
+        hipLaunchKernelGGL((k_fused_B<T, true, L, RES>), grd, blk, 0, s, dev, map, soff);
     else
-        hipLaunchKernelGGL((k_fused_B<T, false, L, RES>), grd, blk, 0, s, dev, nbx, nby, nbz, soff);
+        hipLaunchKernelGGL((k_fused_B<T, false, L, RES>), grd, blk, 0, s, dev, map, soff);
 }
 
 template <typename T>

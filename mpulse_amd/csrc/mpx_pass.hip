@@ -425,12 +425,6 @@ struct RowD {
     double a[64], b[64];
 };
 
-// A read-only table entry at a wave-uniform address, through the constant address space: a
-// scalar load into SGPRs, counted apart from the vector loads in flight
-__device__ __forceinline__ double kload(const double *p)
-{
-    return *(const __attribute__((address_space(4))) double *)p;
-}
 // three components and the residual word of the cell at bo in plane `pl` (storage offset)
 template <typename T, bool RES>
 __device__ __forceinline__ Raw3<T, RES> ldp3(const T *const f[3], const unsigned *lo, size_t pl, unsigned bo)

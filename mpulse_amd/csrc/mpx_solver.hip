@@ -212,6 +212,7 @@ struct mpx_solver {
     int pole_ref[3] = {-1, -1, -1};  // active pole slot -> reference pole index
     std::vector<double> kE[3], kH[3];
     double *d_kdE[3] = {}, *d_kdH[3] = {};
+    double *d_bc[2][3] = {};  // CPML b and c lines of the E / H side per dimension (CpmlDim::bc)
     double *d_ikdE[3] = {}, *d_ikdH[3] = {};  // reciprocals, for the fused and sweep kernels
     double *d_eps = nullptr;                    // per-cell permittivity, once set (full storage)
     // plasma: PlasmaDensity OptField and PlasmaCurrent (float64 grids over the storage box)
@@ -246,9 +247,7 @@ struct mpx_solver {
     unsigned *d_status = nullptr;  // device status (MPX_ERR_NUMERIC bits), read and cleared by mpx_sync
     int ncap = mpx::kNewtonCap;    // Kerr Newton iteration cap
     int time = 0;
-    // x planes per thread in the fused kernels (1, 2 or 4); with the pole accumulators and the
-    // cell's own field streamed nontemporally, E: 1 and B: 2 are fastest in both precisions
-    int march_e = 1, march_b = 2;
+    int march_e = 1, march_b = 1;  // x planes per thread in the fused kernels (1, 2 or 4; B chosen in build)
     int tile_order = 2;            // fused kernels: block order, 0 = z tiles fastest, 1 = x chunks fastest,
                                    // 2 = bands of tile_band rows walked plane by plane (fastest)
     int tile_band = 0;             // 0: chosen from the grid by auto_band
@@ -749,6 +748,30 @@ int mpx_destroy(mpx_solver *s)
 
 }  // extern "C"
 
+// The auxiliaries of the two faces of one dimension and side of the currents, in one block: psi0
+// of the high-side (0) and of the low-side (1) face, psi1 of both, then the residual words of
+// both.  The faces of a dimension have the same extents.
+struct FaceBlock {
+    char *aux = nullptr;
+    unsigned *rw = nullptr;
+    size_t cnt = 0;
+};
+static int face_block(mpx_solver *s, FaceBlock &b, size_t cnt, int side, void *aux[2], unsigned **rw)
+{
+    int rc = MPX_OK;
+    if (!b.aux) {
+        b.cnt = (cnt + 63) / 64 * 64;
+        b.aux = s->esz == 8 ? (char *)s->dalloc<double>(4 * b.cnt, rc) : (char *)s->dalloc<float>(4 * b.cnt, rc);
+        if (rc) return rc;
+        if (s->res) b.rw = s->dalloc<unsigned>(2 * b.cnt, rc);
+        if (rc) return rc;
+    }
+    if (cnt > b.cnt) return fail(MPX_ERR_INVALID, "CPML faces of one dimension differ in size");
+    for (int w = 0; w < 2; ++w) aux[w] = b.aux + (2 * w + side) * b.cnt * s->esz;
+    *rw = b.rw ? b.rw + side * b.cnt : nullptr;
+    return MPX_OK;
+}
+
 static int build(mpx_solver *s, const mpx_desc *desc)
 {
     s->d = *desc;
@@ -761,9 +784,12 @@ static int build(mpx_solver *s, const mpx_desc *desc)
         return fail(MPX_ERR_INVALID, "unknown precision " + std::to_string(s->prec));
     s->res = s->prec == MPX_PREC_FP32_RES;
     s->esz = (s->prec == MPX_PREC_FP64) ? 8 : 4;
-    // the residual B kernel keeps its planes' decoded values in float64 registers: one plane
-    // per thread runs at 8 waves per SIMD against 5 for two (1.72 against 1.82 ms at 512^3)
-    if (s->res) s->march_b = 1;
+    // Planes per thread of the fused B kernel: a second plane saves a read of E but holds its words
+    // in registers and halves the waves.  One is faster in both float32 forms (us, one against two
+    // planes with CPML: 24^3 7.2 / 9.1, 256^3 188 / 205, 512^3 1059 / 1118; with residuals 1348 /
+    // 1573) and for small float64 grids (24^3 7.3 / 9.1, 64^3 11.3 / 12.2); from about 2^21 cells
+    // float64 gains a little from two (131x158x177 74.5 / 73.2, 512^3 2014 / 1969).
+    s->march_b = s->esz == 8 && (double)desc->nx * desc->ny * desc->nz >= (1 << 21) ? 2 : 1;
     s->delta[0] = desc->dx;
     s->delta[1] = desc->dy;
     s->delta[2] = desc->dz;
@@ -906,6 +932,7 @@ static int build(mpx_solver *s, const mpx_desc *desc)
         // coreInitStorage, src/fdtd_plrc.cpp:13-86: layers, coefficients, invalid currents dropped
         auto init_side = [&](std::vector<Current> &list, bool isH) -> int {
             std::vector<Current> kept;
+            FaceBlock blk[3];
             for (Current c : list) {
                 if (c.type == CUR_PLASMA) {  // a grid current over the storage box, no layer
                     kept.push_back(c);
@@ -938,29 +965,43 @@ static int build(mpx_solver *s, const mpx_desc *desc)
                     F.idxn = 1.0 / F.dxn;
                     size_t cnt = s->layers[l0].count();
                     int lc[3] = {l0, l1, l2};
+                    void *aux[2];
+                    if ((rc = face_block(s, blk[dim], cnt, is_high(c.dir) ? 0 : 1, aux, &F.rw))) return rc;
                     for (int w = 0; w < 2; ++w) {
-                        void *p = (s->esz == 8) ? (void *)s->dalloc<double>(cnt, rc) : (void *)s->dalloc<float>(cnt, rc);
-                        if (rc) return rc;
                         int comp = w == 0 ? F.c0 : F.c1;
-                        s->layers[lc[comp]].comp[0] = p;  // each component layer owns one array
-                        if (w == 0) F.psi0 = p; else F.psi1 = p;
+                        s->layers[lc[comp]].comp[0] = aux[w];  // each component layer owns one array
+                        (w == 0 ? F.psi0 : F.psi1) = aux[w];
                     }
                     if (s->res) {
-                        F.rw = s->dalloc<unsigned>(cnt, rc);
-                        if (rc) return rc;
                         s->layers[lc[F.c0]].rw = s->layers[lc[F.c1]].rw = F.rw;
                         s->layers[lc[F.c0]].slot = 0;
                         s->layers[lc[F.c1]].slot = 1;
                     }
                     std::vector<double> bb, cc;
                     cpml_coeff(f, c.dir, isH, F.lo[dim], F.hi[dim], desc->dt, bb, cc);
-                    double *db = s->dalloc<double>(bb.size(), rc);
-                    double *dc = s->dalloc<double>(cc.size(), rc);
-                    if (rc) return rc;
-                    if (upload(s, db, bb.data(), bb.size() * 8) || upload(s, dc, cc.data(), cc.size() * 8))
+                    // lines of b and c over the whole dimension, by side (CpmlDim); the face's own tables
+                    // are the layer's part of them (a layer thicker than the box keeps its own)
+                    const int len = g.n[dim] + 2, own = F.lo[dim] < 0 || F.hi[dim] >= len ? (int)bb.size() : 0;
+                    if (!s->d_bc[isH][dim] && !(s->d_bc[isH][dim] = s->dalloc<double>(4 * (size_t)len, rc))) return rc;
+                    std::vector<double> line(2 * (size_t)len, 0.0);
+                    for (int q = 0; q < (int)bb.size(); ++q)
+                        if (F.lo[dim] + q >= 0 && F.lo[dim] + q < len) {
+                            line[F.lo[dim] + q] = bb[q];
+                            line[len + F.lo[dim] + q] = cc[q];
+                        }
+                    double *dl = s->d_bc[isH][dim] + (is_high(c.dir) ? 0 : 2 * len);
+                    if (upload(s, dl, line.data(), line.size() * 8))
                         return fail(MPX_ERR_HIP, "coefficient upload failed");
-                    F.b = db;
-                    F.c = dc;
+                    F.b = dl + F.lo[dim];
+                    F.c = dl + len + F.lo[dim];
+                    if (own) {
+                        double *dt = s->dalloc<double>(2 * (size_t)own, rc);
+                        if (rc) return rc;
+                        bb.insert(bb.end(), cc.begin(), cc.end());
+                        if (upload(s, dt, bb.data(), bb.size() * 8)) return fail(MPX_ERR_HIP, "coefficient upload failed");
+                        F.b = dt;
+                        F.c = dt + own;
+                    }
                     std::vector<CpmlFace> &faces = isH ? s->hfaces : s->efaces;
                     c.face = (int)faces.size();
                     faces.push_back(F);
@@ -1220,20 +1261,23 @@ static int build(mpx_solver *s, const mpx_desc *desc)
             s->B2lo = s->dalloc<unsigned>(s->cells, rc);
             if (rc) return rc;
         }
+        FaceBlock blk[3];
         for (size_t f = 0; f < s->hfaces.size(); ++f) {
             const CpmlFace &F = s->hfaces[f];
             const size_t cnt = (size_t)(F.hi[0] - F.lo[0] + 1) * F.n1 * F.n2;
+            int side = 1;
+            for (const Current &c : s->hcur)
+                if (c.face == (int)f) side = is_high(c.dir) ? 0 : 1;
+            void *aux[2];
+            unsigned *rw = nullptr;
+            if ((rc = face_block(s, blk[F.dim], cnt, side, aux, &rw))) return rc;
             for (int w = 0; w < 2; ++w) {
-                void *p = (s->esz == 8) ? (void *)s->dalloc<double>(cnt, rc) : (void *)s->dalloc<float>(cnt, rc);
-                if (rc) return rc;
-                s->hpsi2[w].push_back(p);
+                s->hpsi2[w].push_back(aux[w]);
                 int li = -1;
                 for (size_t q = 0; q < s->layers.size(); ++q)
                     if (s->layers[q].comp[0] == (w == 0 ? F.psi0 : F.psi1)) li = (int)q;
                 s->hface_layer[w].push_back(li);
             }
-            unsigned *rw = nullptr;
-            if (s->res && !(rw = s->dalloc<unsigned>(cnt, rc))) return rc;
             s->hrw2.push_back(rw);
         }
     }
@@ -1263,6 +1307,50 @@ static int auto_band(const mpx::GridDims &g, const int *blo, bool hside)
     int band = 1;
     while (band * 2 <= target && band * 2 <= nby) band *= 2;
     return band;
+}
+
+// the index in its side's list of the CPML face of dimension d on its high (q 0) or low (1)
+// side, E or H currents; -1 if none
+static int face_index(const mpx_solver *s, bool hside, int d, int q)
+{
+    for (const Current &c : hside ? s->hcur : s->ecur)
+        if (c.face >= 0 && dim_of(c.dir) == d && is_high(c.dir) == (q == 0)) return c.face;
+    return -1;
+}
+
+// The faces of dimension d as the fused and pass kernels read them.  other: the new auxiliaries
+// go to the pass path's second set (H side), the faces' own hold the old ones.
+static mpx::CpmlDim cpml_dim(const mpx_solver *s, bool hside, int d, bool other)
+{
+    mpx::CpmlDim D{};
+    const std::vector<CpmlFace> &faces = hside ? s->hfaces : s->efaces;
+    const int f[2] = {face_index(s, hside, d, 0), face_index(s, hside, d, 1)};
+    D.lo[0] = D.lo[1] = 1;
+    D.idxn = 1.0 / s->delta[d];
+    D.len = s->g.n[d] + 2;
+    D.bc = s->d_bc[hside][d];
+    const int first = f[0] >= 0 ? f[0] : f[1];
+    if (first < 0) return D;
+    const CpmlFace &A = faces[first];
+    D.o0 = A.psi0;
+    D.o1 = A.psi1;
+    D.orw = A.rw;
+    D.p0 = other ? s->hpsi2[0][first] : A.psi0;
+    D.p1 = other ? s->hpsi2[1][first] : A.psi1;
+    D.rw = other ? s->hrw2[first] : A.rw;
+    D.s0 = A.n1 * A.n2;
+    D.s1 = A.n2;
+    for (int q = 0; q < 2; ++q) {
+        if (f[q] < 0) continue;
+        const CpmlFace &F = faces[f[q]];
+        D.lo[q] = F.lo[d];
+        D.hi[q] = F.hi[d];
+        // both faces' auxiliaries lie in one block per array (face_block)
+        const long long to = ((const char *)F.psi0 - (const char *)A.psi0) / (long long)s->esz;
+        D.off[q] = (int)(to - ((long long)F.lo[0] * D.s0 + (long long)F.lo[1] * D.s1 + F.lo[2]));
+    }
+    D.two = f[0] >= 0 && f[1] >= 0 && D.lo[0] <= D.hi[1] && D.lo[1] <= D.hi[0];
+    return D;
 }
 
 template <typename T>
@@ -1314,14 +1402,9 @@ static StepArgs<T> step_args(mpx_solver *s, bool hside)
     }
     const std::vector<CpmlFace> &faces = hside ? s->hfaces : s->efaces;
     a.nfaces = (int)faces.size();
-    for (int d = 0; d < 3; ++d) a.face_by_dim[d][0] = a.face_by_dim[d][1] = -1;
     const std::vector<Current> &list = hside ? s->hcur : s->ecur;
     for (size_t q = 0; q < faces.size(); ++q) a.face[q] = faces[q];
-    for (const Current &c : list)
-        if (c.face >= 0) {
-            int dim = dim_of(c.dir);
-            a.face_by_dim[dim][is_high(c.dir) ? 0 : 1] = c.face;
-        }
+    for (int d = 0; d < 3; ++d) a.cd[d] = cpml_dim(s, hside, d, false);
     a.nsheets = 0;
     for (const Current &c : list)
         if (c.type == CUR_INC_E || c.type == CUR_INC_H) a.sheet[a.nsheets++] = c.ev.sheet;
@@ -3458,21 +3541,6 @@ struct StateRef {
     std::vector<std::pair<void *, size_t>> arr;  // (device pointer, doubles)
 };
 
-// the CPML face of dimension d on its high (q 0) or low (1) side, E or H currents; null if none
-const CpmlFace *face_of(mpx_solver *s, int hside, int d, int q)
-{
-    for (const Current &c : hside ? s->hcur : s->ecur)
-        if (c.face >= 0 && dim_of(c.dir) == d && is_high(c.dir) == (q == 0))
-            return &(hside ? s->hfaces : s->efaces)[c.face];
-    return nullptr;
-}
-// extent of that face's box along x
-int adj_extent(mpx_solver *s, int hside, int d, int q)
-{
-    const CpmlFace *F = face_of(s, hside, d, q);
-    return F ? F->hi[0] - F->lo[0] + 1 : 0;
-}
-
 StateRef state_of(mpx_solver *s)
 {
     StateRef r;
@@ -3542,7 +3610,7 @@ int mpx_adjoint_grad(mpx_solver *s, const mpx_objective *obj, int nsteps, int K,
                     for (int q = 0; q < 2; ++q) {
                         mpx::AdjFace &f = side ? a.hf[d][q] : a.ef[d][q];
                         if (f.hi < f.lo) continue;
-                        const size_t n = (size_t)f.s0 * adj_extent(s, side, d, q);
+                        const size_t n = face_count((side ? s->hfaces : s->efaces)[face_index(s, side, d, q)]);
                         f.A0 = mem.get<double>(n);
                         f.A1 = mem.get<double>(n);
                     }
@@ -3582,8 +3650,9 @@ int mpx_adjoint_grad(mpx_solver *s, const mpx_objective *obj, int nsteps, int K,
                 mpx::AdjFace &f = side ? a.hf[d][q] : a.ef[d][q];
                 f.lo = 1;
                 f.hi = 0;
-                const CpmlFace *F = face_of(s, side, d, q);
-                if (!F) continue;
+                const int fi = face_index(s, side, d, q);
+                if (fi < 0) continue;
+                const CpmlFace *F = &(side ? s->hfaces : s->efaces)[fi];
                 f.lo = F->lo[d];
                 f.hi = F->hi[d];
                 f.s0 = F->n1 * F->n2;

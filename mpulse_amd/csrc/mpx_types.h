@@ -94,6 +94,22 @@ struct CpmlFace {
     }
 };
 
+// The two CPML faces of one dimension on the E or on the H side, as the fused and pass kernels
+// read them: the auxiliaries of both faces lie in one block (high side first), so that a cell
+// finds its own with one base address and a 32-bit index whichever face holds it.
+struct CpmlDim {
+    int lo[2], hi[2];     // range of the normal coordinate: [0] high side, [1] low side (lo > hi: none)
+    int two;              // the ranges overlap: a cell may lie in both (high side first)
+    int s0, s1, off[2];   // index of cell (i, j, k): i s0 + j s1 + k + off[side]
+    int len;              // n + 2: length of a coefficient line
+    void *p0, *p1;        // auxiliaries psi0, psi1 (CpmlFace)
+    unsigned *rw;         // residual words (float32 + residual storage), else null
+    const void *o0, *o1;  // the auxiliaries of the step before (p0, p1 where updated in place)
+    const unsigned *orw;
+    const double *bc;     // lines of b and c: bc[(2 side + (0 b, 1 c)) len + coordinate]
+    double idxn;          // 1 / spacing
+};
+
 // One incident-source current sheet: a z plane kp of the down face, three float64
 // component planes of (nx+2) x (ny+2), index i*(ny+2)+j.
 struct Sheet {
@@ -144,6 +160,45 @@ struct SheetTask {
     int task, points;
 };
 
+// t / d for t < 2^31 as (t m) >> sh: sh = 31 + ceil(log2 d), m = ceil(2^sh / d) < 2^32
+struct FastDiv {
+    unsigned d, m;
+    int sh;
+};
+inline FastDiv fast_divisor(unsigned d)
+{
+    FastDiv f{d, 0, 31};
+    while ((1ULL << (f.sh - 31)) < d) ++f.sh;
+    f.m = (unsigned)(((1ULL << f.sh) + d - 1) / d);
+    return f;
+}
+
+// Block -> tile of the fused kernels (map_tile): nbx x nby x nbz tiles dealt to the 8 XCDs in
+// contiguous shares of one of three orders
+struct TileMap {
+    unsigned total, per;     // tiles, and tiles per XCD share
+    int order, rev, nbands;  // StepArgs::order, rev
+    FastDiv first, second;   // the order's fastest and second dimension (order 2: nbx)
+    FastDiv full, rband, rlast;  // order 2: tiles of a full band, its rows, the last band's rows
+};
+inline TileMap tile_map(int nbx, int nby, int nbz, int order, int band, int rev)
+{
+    TileMap m{};
+    m.total = (unsigned)nbx * nby * nbz;
+    m.per = m.total / 8u;
+    m.order = order;
+    m.rev = rev;
+    if (band < 1) band = 1;
+    if (band > nby) band = nby;
+    m.nbands = (nby + band - 1) / band;
+    m.first = fast_divisor(order == 1 ? nbz : nbx);
+    m.second = fast_divisor(order == 1 ? nbx : nby);
+    m.full = fast_divisor((unsigned)nbx * band * nbz);
+    m.rband = fast_divisor(band);
+    m.rlast = fast_divisor(nby - (m.nbands - 1) * band);
+    return m;
+}
+
 // PLRC pole constants (PLRCData, src/fdtd_plrc.h:71-78) of the active poles, precomputed on the
 // host with the formulas of src/fdtd_plrc.t:198-216.
 struct PoleConsts {
@@ -180,7 +235,7 @@ struct StepArgs {
     PoleConsts pc;
     int nfaces;
     CpmlFace face[kMaxFaces];   // E-side faces for the E kernel, H-side faces for the B kernel
-    int face_by_dim[3][2];      // per dimension: [0] high-side face (N/E/U, first in the list), [1] low side, or -1
+    CpmlDim cd[3];              // the same faces by dimension
     int nsheets;
     Sheet sheet[kMaxSheets];
     int sheets_first;           // a source factory precedes the CPML factory in the list
