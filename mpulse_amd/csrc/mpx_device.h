@@ -407,37 +407,45 @@ __device__ __forceinline__ Aux<T, RES> cpml_load(const CpmlDim &D, int l)
     // rest of the line is read by the neighbouring row
     return {gld((const T *)D.o0 + l), gld((const T *)D.o1 + l), lo_ld<RES>(D.orw, l)};
 }
-// The new auxiliaries from the old (x: loaded from index l), the coordinate and the cell's
-// differences; stored with `store`.  v0, v1: the stored values, which the current sums see.
+// The new auxiliaries (h0, h1, w: as stored) from the old (x), the coefficients and the cell's
+// differences.  v0, v1: the stored values, which the current sums see.
 // E side: CPMLBorderECurrent::stepScheme, src/cpml_border.cpp:398-425 (psi0 gets -c d1/dx);
 // H side: CPMLBorderHCurrent::stepScheme, src/cpml_border.cpp:499-527 (psi0 gets +c d1/dx).
 template <typename T, bool HSIDE, bool RES>
-__device__ __forceinline__ void cpml_update(const CpmlDim &D, int side, int coord, int l, const Aux<T, RES> &x, double d1,
-                                            double d0, bool store, double &v0, double &v1)
+__device__ __forceinline__ void cpml_next(double idxn, double bq, double cq, const Aux<T, RES> &x, double d1, double d0,
+                                          T &h0, T &h1, unsigned &w, double &v0, double &v1)
 {
-    const double *line = D.bc + (2 * side * D.len + coord);
-    const double bq = gld(line), cq = gld(line + D.len);
     T r0 = x.o0, r1 = x.o1;
     hold(r0);  // decoded here, not where they were requested
     hold(r1);
     const double a0 = got<T, RES>(r0, x.w, 0), a1 = got<T, RES>(r1, x.w, 1);
     double n0, n1;
     if (HSIDE) {
-        n0 = bq * a0 + cq * d1 * D.idxn;
-        n1 = bq * a1 - cq * d0 * D.idxn;
+        n0 = bq * a0 + cq * d1 * idxn;
+        n1 = bq * a1 - cq * d0 * idxn;
     } else {
-        n0 = bq * a0 - cq * d1 * D.idxn;
-        n1 = bq * a1 + cq * d0 * D.idxn;
+        n0 = bq * a0 - cq * d1 * idxn;
+        n1 = bq * a1 + cq * d0 * idxn;
     }
-    unsigned wn = 0;
-    const T h0 = put<T, RES>(n0, wn, 0), h1 = put<T, RES>(n1, wn, 1);
+    w = 0;
+    h0 = put<T, RES>(n0, w, 0);
+    h1 = put<T, RES>(n1, w, 1);
+    v0 = got<T, RES>(h0, w, 0);
+    v1 = got<T, RES>(h1, w, 1);
+}
+// the same, the new auxiliaries stored at index l with `store`
+template <typename T, bool HSIDE, bool RES>
+__device__ __forceinline__ void cpml_update(const CpmlDim &D, double bq, double cq, int l, const Aux<T, RES> &x, double d1,
+                                            double d0, bool store, double &v0, double &v1)
+{
+    T h0, h1;
+    unsigned w;
+    cpml_next<T, HSIDE, RES>(D.idxn, bq, cq, x, d1, d0, h0, h1, w, v0, v1);
     if (store) {
         gst((T *)D.p0 + l, h0);
         gst((T *)D.p1 + l, h1);
-        if (RES) gst(D.rw + l, wn);
+        if (RES) gst(D.rw + l, w);
     }
-    v0 = got<T, RES>(h0, wn, 0);
-    v1 = got<T, RES>(h1, wn, 1);
 }
 // A cell's part in the layers of the three dimensions: its sides and what was loaded for them
 template <typename T, bool RES>
@@ -472,14 +480,16 @@ __device__ __forceinline__ void cpml_add(const CpmlDim D[3], int i, int j, int k
         const int d = order[u], c0 = (d + 1) % 3, c1 = (d + 2) % 3;
         if (s.side[d] >= 0) {
             double v0, v1;
-            cpml_update<T, HSIDE, RES>(D[d], s.side[d], at[d], cpml_index(D[d], s.side[d], i, j, k), s.x[d], df[d][1],
-                                       df[d][0], store, v0, v1);
+            const double *line = D[d].bc + (2 * s.side[d] * D[d].len + at[d]);
+            cpml_update<T, HSIDE, RES>(D[d], gld(line), gld(line + D[d].len), cpml_index(D[d], s.side[d], i, j, k), s.x[d],
+                                       df[d][1], df[d][0], store, v0, v1);
             J[c0] += v0;
             J[c1] += v1;
             if (D[d].two && s.side[d] == 0 && at[d] >= D[d].lo[1] && at[d] <= D[d].hi[1]) {
                 const int l = cpml_index(D[d], 1, i, j, k);
-                cpml_update<T, HSIDE, RES>(D[d], 1, at[d], l, cpml_load<T, RES>(D[d], l), df[d][1], df[d][0], store, v0,
-                                           v1);
+                line = D[d].bc + (2 * D[d].len + at[d]);
+                cpml_update<T, HSIDE, RES>(D[d], gld(line), gld(line + D[d].len), l, cpml_load<T, RES>(D[d], l), df[d][1],
+                                           df[d][0], store, v0, v1);
                 J[c0] += v0;
                 J[c1] += v1;
             }
@@ -581,17 +591,6 @@ __device__ __forceinline__ void map_tile(const TileMap &M, int &bx, int &by, int
             bz = z;
         }
     }
-}
-
-__device__ __forceinline__ void fused_tile_of(int order, int band, int rev, int nbx, int nby, int nbz, int &bx,
-                                              int &by, int &bz)
-{
-    if (order == 2)
-        band_tile(nbx, nby, nbz, band, rev, bx, by, bz);
-    else if (order == 1)
-        xcd_tile(nbz, nbx, nby, bz, bx, by);
-    else
-        xcd_tile(nbx, nby, nbz, bx, by, bz);
 }
 
 // Whether coordinate coord of dimension dim lies in the layer of the high-side ([0]) and

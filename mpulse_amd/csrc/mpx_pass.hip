@@ -24,156 +24,45 @@
 
 namespace mpx {
 
-// One CPML H face at cell l: the old auxiliaries come from the step's old buffers; the new
-// ones go to the face's (new) buffers when the cell is this wave's (store).  Returns the
-// stored values (CPMLBorderHCurrent::stepScheme, src/cpml_border.cpp:499-527).
-template <typename T, bool RES>
-__device__ __forceinline__ void cpml_hface_pp(const CpmlFace &f, const T *o0, const T *o1, const unsigned *orw,
-                                              int coord, int l, double d1, double d0, bool store, double &v0,
-                                              double &v1)
+// The six E differences of a cell (dEy_z, dEx_z, dEz_y, dEx_y, dEz_x, dEy_x) by dimension, as cpml_add
+// takes them
+#define MPX_DIFF_E(d) {{d[5], d[4]}, {d[2], d[3]}, {d[1], d[0]}}
+
+// Magnetic current total at (i, j, k) in the reference's list order: the sheets before or after
+// the CPML faces, which add_faces(M) adds.
+template <typename T, typename F>
+__device__ __forceinline__ void pass_m(const PassArgs<T> &a, int i, int j, int k, double M[3], bool sh, int soff,
+                                       F &&add_faces)
 {
-    const int q = coord - f.lo[f.dim];
-    const double bq = gld(f.b + q), cq = gld(f.c + q);
-    const unsigned w = lo_ld<RES>(orw, l);
-    const double a0 = (double)rd<T, RES>(o0, w, 0, l), a1 = (double)rd<T, RES>(o1, w, 1, l);
-    const double n0 = bq * a0 + cq * d1 * f.idxn;
-    const double n1 = bq * a1 - cq * d0 * f.idxn;
-    unsigned wn = 0;
-    const T h0 = put<T, RES>(n0, wn, 0), h1 = put<T, RES>(n1, wn, 1);
-    if (store) {
-        gst((T *)f.psi0 + l, h0);
-        gst((T *)f.psi1 + l, h1);
-        if (RES) gst(f.rw + l, wn);
-    }
-    v0 = got<T, RES>(h0, wn, 0);
-    v1 = got<T, RES>(h1, wn, 1);
+    M[0] = M[1] = M[2] = 0.0;
+    if (sh && a.sheets_first) add_sheet_planes(a.hsheet, a.nhsheets, a.g.py, i, j, k, soff, M[0], M[1], M[2]);
+    add_faces(M);
+    if (sh && !a.sheets_first) add_sheet_planes(a.hsheet, a.nhsheets, a.g.py, i, j, k, soff, M[0], M[1], M[2]);
 }
 
-// Magnetic current total at (i, j, k) in the reference's list order (sheets before or after
-// the CPML faces; faces N,S (y), E,W (x), U,D (z), high face first), from the six E
-// differences of the cell.
-template <typename T, bool CPML, bool RES>
-__device__ __forceinline__ void pass_m(const PassArgs<T> &a, int i, int j, int k, bool store, double dEy_z,
-                                       double dEx_z, double dEz_y, double dEx_y, double dEz_x, double dEy_x,
-                                       double &mx, double &my, double &mz, bool cp, bool sh, int soff, bool live = true)
+// Electric current total at (i, j, k); the plasma current (jpv) joins it at its place in the
+// list (pcur_pos: before the first group, between the two, after both)
+template <typename T, typename F>
+__device__ __forceinline__ void pass_j(const PassArgs<T> &a, int i, int j, int k, double J[3], bool sh, int soff,
+                                       const double *jpv, F &&add_faces)
 {
-    mx = my = mz = 0.0;
-    if (sh && a.sheets_first) add_sheet_planes(a.hsheet, a.nhsheets, a.g.py, i, j, k, soff, mx, my, mz);
-    if (CPML && cp) {
-        bool in[2];
-        in_faces(a.hfbd, a.hface, 1, j, in);
-        in[0] = in[0] && live;
-        in[1] = in[1] && live;
-#pragma unroll
-        for (int s = 0; s < 2; ++s)
-            if (in[s]) {
-                const int fi = a.hfbd[1][s];
-                const CpmlFace &f = a.hface[fi];
-                double v0, v1;  // psi0 -> Mz from dEx_y, psi1 -> Mx from dEz_y
-                cpml_hface_pp<T, RES>(f, (const T *)a.hold[fi][0], (const T *)a.hold[fi][1], a.hold_rw[fi], j,
-                                      layer_index(f, i, j, k), dEx_y, dEz_y, store, v0, v1);
-                mz += v0;
-                mx += v1;
-            }
-        in_faces(a.hfbd, a.hface, 0, i, in);
-        in[0] = in[0] && live;
-        in[1] = in[1] && live;
-#pragma unroll
-        for (int s = 0; s < 2; ++s)
-            if (in[s]) {
-                const int fi = a.hfbd[0][s];
-                const CpmlFace &f = a.hface[fi];
-                double v0, v1;  // psi0 -> My from dEz_x, psi1 -> Mz from dEy_x
-                cpml_hface_pp<T, RES>(f, (const T *)a.hold[fi][0], (const T *)a.hold[fi][1], a.hold_rw[fi], i,
-                                      layer_index(f, i, j, k), dEz_x, dEy_x, store, v0, v1);
-                my += v0;
-                mz += v1;
-            }
-        in_faces(a.hfbd, a.hface, 2, k, in);
-        in[0] = in[0] && live;
-        in[1] = in[1] && live;
-#pragma unroll
-        for (int s = 0; s < 2; ++s)
-            if (in[s]) {
-                const int fi = a.hfbd[2][s];
-                const CpmlFace &f = a.hface[fi];
-                double v0, v1;  // psi0 -> Mx from dEy_z, psi1 -> My from dEx_z
-                cpml_hface_pp<T, RES>(f, (const T *)a.hold[fi][0], (const T *)a.hold[fi][1], a.hold_rw[fi], k,
-                                      layer_index(f, i, j, k), dEy_z, dEx_z, store, v0, v1);
-                mx += v0;
-                my += v1;
-            }
-    }
-    if (sh && !a.sheets_first) add_sheet_planes(a.hsheet, a.nhsheets, a.g.py, i, j, k, soff, mx, my, mz);
-}
-
-// Electric current total at (i, j, k) (CPML E auxiliaries updated in place; owned cells only).
-template <typename T, bool CPML, bool RES>
-__device__ __forceinline__ void pass_j(const PassArgs<T> &a, int i, int j, int k, double dBz_y, double dBy_z,
-                                       double dBx_z, double dBz_x, double dBy_x, double dBx_y, double &jx,
-                                       double &jy, double &jz, bool cp, bool sh, int soff, bool live = true,
-                                       const double *jpv = nullptr)
-{
-    jx = jy = jz = 0.0;
-    // the plasma current (jpv) joins the totals at its place in the list (pcur_pos: before the
-    // first group, between the two, after both)
+    J[0] = J[1] = J[2] = 0.0;
     auto add_plasma = [&](int pos) {
         if (jpv && a.pcur && a.pcur_pos == pos) {
-            jx += jpv[0];
-            jy += jpv[1];
-            jz += jpv[2];
-        }
-    };
-    auto add_cpml = [&]() {
-        if (CPML && cp) {
-            bool in[2];
-            in_faces(a.efbd, a.eface, 1, j, in);
-            in[0] = in[0] && live;
-            in[1] = in[1] && live;
-#pragma unroll
-            for (int s = 0; s < 2; ++s)
-                if (in[s]) {
-                    const CpmlFace &f = a.eface[a.efbd[1][s]];
-                    double v0, v1;
-                    cpml_face<T, false, RES>(f, j, layer_index(f, i, j, k), dBx_y, dBz_y, v0, v1);
-                    jz += v0;
-                    jx += v1;
-                }
-            in_faces(a.efbd, a.eface, 0, i, in);
-            in[0] = in[0] && live;
-            in[1] = in[1] && live;
-#pragma unroll
-            for (int s = 0; s < 2; ++s)
-                if (in[s]) {
-                    const CpmlFace &f = a.eface[a.efbd[0][s]];
-                    double v0, v1;
-                    cpml_face<T, false, RES>(f, i, layer_index(f, i, j, k), dBz_x, dBy_x, v0, v1);
-                    jy += v0;
-                    jz += v1;
-                }
-            in_faces(a.efbd, a.eface, 2, k, in);
-            in[0] = in[0] && live;
-            in[1] = in[1] && live;
-#pragma unroll
-            for (int s = 0; s < 2; ++s)
-                if (in[s]) {
-                    const CpmlFace &f = a.eface[a.efbd[2][s]];
-                    double v0, v1;
-                    cpml_face<T, false, RES>(f, k, layer_index(f, i, j, k), dBy_z, dBx_z, v0, v1);
-                    jx += v0;
-                    jy += v1;
-                }
+            J[0] += jpv[0];
+            J[1] += jpv[1];
+            J[2] += jpv[2];
         }
     };
     add_plasma(0);
     if (a.sheets_first) {
-        if (sh) add_sheet_planes(a.sheet, a.nsheets, a.g.py, i, j, k, soff, jx, jy, jz);
+        if (sh) add_sheet_planes(a.sheet, a.nsheets, a.g.py, i, j, k, soff, J[0], J[1], J[2]);
         add_plasma(1);
-        add_cpml();
+        add_faces(J);
     } else {
-        add_cpml();
+        add_faces(J);
         add_plasma(1);
-        if (sh) add_sheet_planes(a.sheet, a.nsheets, a.g.py, i, j, k, soff, jx, jy, jz);
+        if (sh) add_sheet_planes(a.sheet, a.nsheets, a.g.py, i, j, k, soff, J[0], J[1], J[2]);
     }
     add_plasma(2);
 }
@@ -206,26 +95,14 @@ __device__ __forceinline__ Cell3<T, RES> ld3(const T *const f[3], const unsigned
     return {rd<T, RES>(f[0], w, 0, c), rd<T, RES>(f[1], w, 1, c), rd<T, RES>(f[2], w, 2, c)};
 }
 
-// B^(n+1) at a cell from its B^n, the six E differences (dEy_z, dEx_z, dEz_y, dEx_y, dEz_x,
-// dEy_x) and its position; the CPML H auxiliaries are written only with store
-// (kdx, kdy, kdz: the reciprocal kappa * delta lines of the H side at i, j, k)
-template <typename T, bool CPML, bool RES>
-__device__ __forceinline__ void b_cell_k(const PassArgs<T> &a, int i, int j, int k, const Cell3<T, RES> &b0,
-                                         const double d[6], bool store, T h[3], unsigned &w, double b[3], bool cp,
-                                         bool sh, int soff, bool live, double kdx, double kdy, double kdz)
+// B^(n+1) at a cell from its B^n, the six E differences and its magnetic current M (kdx, kdy, kdz:
+// the reciprocal kappa * delta lines of the H side at i, j, k)
+template <typename T, bool RES>
+__device__ __forceinline__ void b_cell(const PassArgs<T> &a, const Cell3<T, RES> &b0, const double d[6], const double M[3],
+                                       double kdx, double kdy, double kdz, T h[3], unsigned &w, double b[3])
 {
-    double mx, my, mz;
-    pass_m<T, CPML, RES>(a, i, j, k, store, d[0], d[1], d[2], d[3], d[4], d[5], mx, my, mz, cp, sh, soff, live);
     b_update<T, RES>((double)b0.x, (double)b0.y, (double)b0.z, d[0], d[1], d[2], d[3], d[4], d[5], kdx, kdy, kdz,
-                     a.dt, mx, my, mz, h, w, b);
-}
-template <typename T, bool CPML, bool RES>
-__device__ __forceinline__ void b_cell(const PassArgs<T> &a, int i, int j, int k, const Cell3<T, RES> &b0,
-                                       const double d[6], bool store, T h[3], unsigned &w, double b[3], bool cp,
-                                       bool sh, int soff, bool live = true)
-{
-    b_cell_k<T, CPML, RES>(a, i, j, k, b0, d, store, h, w, b, cp, sh, soff, live, gld(a.ikdH[0] + i), gld(a.ikdH[1] + j),
-                           gld(a.ikdH[2] + k));
+                     a.dt, M[0], M[1], M[2], h, w, b);
 }
 
 // k_pass: one cell per thread, in the fused kernels' banded tile order (64 z cells x 4 rows per
@@ -247,7 +124,7 @@ __global__ __launch_bounds__(256) void k_pass(const PassArgs<T> *__restrict__ pa
     const int Nx = g.n[0], Ny = g.n[1], Nz = g.n[2];
     const int sx = (int)g.sx, pz = g.pz;
     int tbx, tby, tbz;
-    fused_tile_of(2, a.band, 0, nbx, nby, nbz, tbx, tby, tbz);
+    band_tile(nbx, nby, nbz, a.band, 0, tbx, tby, tbz);
     const int lane = threadIdx.x;
     const int k = tbx * 64 + lane + 1, j = tby * 4 + threadIdx.y + 1, i = tbz + 1;
     if (k > Nz || j > Ny || i > Nx) return;
@@ -268,12 +145,10 @@ __global__ __launch_bounds__(256) void k_pass(const PassArgs<T> *__restrict__ pa
         for (int d = 0; d < 3; ++d)
 #pragma unroll
             for (int q = 0; q < 2; ++q) {
-                const int fh = a.hfbd[d][q], fe = a.efbd[d][q];
+                const CpmlDim &H = a.hcd[d], &E = a.ecd[d];
                 // a periodic x - 1 / y - 1 / z - 1 of index 1 is N: both ends are tested
-                if (fh >= 0)
-                    cp |= (lo[d] >= a.hface[fh].lo[d] && lo[d] <= a.hface[fh].hi[d]) ||
-                          (hi[d] >= a.hface[fh].lo[d] && hi[d] <= a.hface[fh].hi[d]);
-                if (fe >= 0) cp |= hi[d] >= a.eface[fe].lo[d] && hi[d] <= a.eface[fe].hi[d];
+                cp |= (lo[d] >= H.lo[q] && lo[d] <= H.hi[q]) || (hi[d] >= H.lo[q] && hi[d] <= H.hi[q]) ||
+                      (hi[d] >= E.lo[q] && hi[d] <= E.hi[q]);
             }
         cp = __ballot(cp) != 0;
     }
@@ -321,25 +196,38 @@ __global__ __launch_bounds__(256) void k_pass(const PassArgs<T> *__restrict__ pa
     const double ex = e0.x, ey = e0.y, ez = e0.z;
     T hh[3];
     unsigned hw;
+    // B^(n+1) at (i, j, k) from its B^n and E differences; its CPML H auxiliaries written with `store`
+    auto bcell = [&](int i, int j, int k, const C3 &b0, const double d[6], bool store, T h[3], unsigned &w, double b[3]) {
+        double M[3];
+        pass_m<T>(a, i, j, k, M, sh, soff, [&](double M[3]) {
+            if (CPML && cp) {
+                CellCpml<T, RES> x;
+                cpml_request<T, RES>(a.hcd, i, j, k, true, x);
+                const double df[3][2] = MPX_DIFF_E(d);
+                cpml_add<T, true, RES>(a.hcd, i, j, k, x, df, store, M);
+            }
+        });
+        b_cell<T, RES>(a, b0, d, M, gld(a.ikdH[0] + i), gld(a.ikdH[1] + j), gld(a.ikdH[2] + k), h, w, b);
+    };
     // B^(n+1) at x - 1 (By, Bz are used), y - 1 (Bx, Bz) and z - 1 (Bx, By): not stored
     double bx_m[3], by_m[3], bz_m[3];
     {
         const double x_ = exm.x, y_ = exm.y, z_ = exm.z;
         const double d[6] = {(double)zx.y - y_, (double)zx.x - x_, (double)exm_yp.z - z_, (double)exm_yp.x - x_,
                              ez - z_, ey - y_};
-        b_cell<T, CPML, RES>(a, im, j, k, bxm, d, false, hh, hw, bx_m, cp, sh, soff);
+        bcell(im, j, k, bxm, d, false, hh, hw, bx_m);
     }
     {
         const double x_ = eym.x, y_ = eym.y, z_ = eym.z;
         const double d[6] = {(double)zy.y - y_, (double)zy.x - x_, ez - z_, ex - x_, (double)eym_xp.z - z_,
                              (double)eym_xp.y - y_};
-        b_cell<T, CPML, RES>(a, i, jm, k, bym, d, false, hh, hw, by_m, cp, sh, soff);
+        bcell(i, jm, k, bym, d, false, hh, hw, by_m);
     }
     {
         const double x_ = ezm.x, y_ = ezm.y, z_ = ezm.z;
         const double d[6] = {ey - y_, ex - x_, (double)ezm_yp.z - z_, (double)ezm_yp.x - x_, (double)ezm_xp.z - z_,
                              (double)ezm_xp.y - y_};
-        b_cell<T, CPML, RES>(a, i, j, km, bzm, d, false, hh, hw, bz_m, cp, sh, soff);
+        bcell(i, j, km, bzm, d, false, hh, hw, bz_m);
     }
     // B^(n+1) at the cell (its CPML H auxiliaries stored)
     T bh[3];
@@ -348,14 +236,21 @@ __global__ __launch_bounds__(256) void k_pass(const PassArgs<T> *__restrict__ pa
     {
         const double d[6] = {(double)z0.y - ey, (double)z0.x - ex, (double)eyp.z - ez, (double)eyp.x - ex,
                              (double)exp_.z - ez, (double)exp_.y - ey};
-        b_cell<T, CPML, RES>(a, i, j, k, b0, d, true, bh, bw, b, cp, sh, soff);
+        bcell(i, j, k, b0, d, true, bh, bw, b);
     }
     // E^(n+2) at the cell
     const double dBz_y = b[2] - by_m[2], dBx_y = b[0] - by_m[0];
     const double dBy_z = b[1] - bz_m[1], dBx_z = b[0] - bz_m[0];
     const double dBz_x = b[2] - bx_m[2], dBy_x = b[1] - bx_m[1];
-    double jx, jy, jz;
-    pass_j<T, CPML, RES>(a, i, j, k, dBz_y, dBy_z, dBx_z, dBz_x, dBy_x, dBx_y, jx, jy, jz, cp, sh, soff);
+    double J[3];
+    pass_j<T>(a, i, j, k, J, sh, soff, nullptr, [&](double J[3]) {
+        if (CPML && cp) {
+            CellCpml<T, RES> x;
+            cpml_request<T, RES>(a.ecd, i, j, k, true, x);
+            const double df[3][2] = {{dBy_x, dBz_x}, {dBz_y, dBx_y}, {dBx_z, dBy_z}};
+            cpml_add<T, false, RES>(a.ecd, i, j, k, x, df, true, J);
+        }
+    });
     double idenom = a.idenom, numer = a.numer;
     if (a.epsf) {
         double denom;
@@ -365,7 +260,7 @@ __global__ __launch_bounds__(256) void k_pass(const PassArgs<T> *__restrict__ pa
     double nex = ex, ney = ey, nez = ez;
     unsigned fl = 0;
     plrc_e_update_pp<NP, NONLIN, true>(nex, ney, nez, dBz_y, dBy_z, dBx_z, dBz_x, dBy_x, dBx_y, gld(a.ikdE[0] + i),
-                                       gld(a.ikdE[1] + j), gld(a.ikdE[2] + k), jx, jy, jz, pr, a.psi, (size_t)c, true,
+                                       gld(a.ikdE[1] + j), gld(a.ikdE[2] + k), J[0], J[1], J[2], pr, a.psi, (size_t)c, true,
                                        a.pc, a.dt, idenom, numer, a.chi, a.ncap, &fl);
     report(a.status, fl | finite_flag(nex, ney, nez));
     unsigned ew = 0;
@@ -432,24 +327,147 @@ __device__ __forceinline__ Raw3<T, RES> ldp3(const T *const f[3], const unsigned
     return {ldp(f[0] + pl, bo), ldp(f[1] + pl, bo), ldp(f[2] + pl, bo), RES ? ldp(lo + pl, bo) : 0u};
 }
 
-// Whether a CPML face of the E side or of the H side holds cell (i, j, k)
-template <typename T>
-__device__ __forceinline__ bool in_cpml(const PassArgs<T> &a, bool eside, int i, int j, int k)
+// ---- CPML in the march ----
+//
+// Vector memory operations return in order, and what a wave may leave in flight at a wait is the
+// count that holds on every path to it.  A load or store that only waves with a layer cell issue
+// is not in that count, so those waves waited for as many of the next plane's prefetched words
+// instead: any layer along z, 4 cells or 20 thick, cost 256^3 a quarter of its time (float32 +
+// residual 579 -> 751 us, float64 692 -> 917).  So the body of a row wave exists once per kind of
+// wave (MODE), each with the same operations on every path: the auxiliaries are read and written
+// through buffer descriptors, which drop the lanes and the dimensions that have no layer there.
+// 256^3 with layers along z 751 -> 681, with all 826 -> 829 (float32 + residual), float64 with all 1011 ->
+// 932, 10 runs of 48^3 to 160^3 in float64 73.5 -> 69.7 ms for 60 steps.  The H auxiliaries of a
+// plane are requested with its field words, the E auxiliaries when the H ones have left their
+// registers.  Coefficients come through other counters: along x and y, where the coordinate is
+// uniform over the wave, from scalar loads, along z from a table in LDS.
+
+// The auxiliaries of one lane's cell at the plane being prefetched
+template <typename T, bool RES>
+struct MarchAux {
+    Aux<T, RES> x[3];
+};
+// Buffer accesses to one array of a face slab from a scalar base.  The hardware drops those at or past
+// `bytes`, so a wave or lane with no cell in the layer issues the same operations as one with,
+// without a branch and without memory traffic.
+constexpr unsigned BUF_OUT = 0x80000000u;  // an offset past the end of every row and slab
+template <typename P>
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buf(P *base, unsigned bytes)
 {
-    const int x[3] = {i, j, k};
-    bool in = false;
+    return __builtin_amdgcn_make_buffer_rsrc((void *)base, 0, (int)bytes, 0x00027000);
+}
+__device__ __forceinline__ void bld(__amdgpu_buffer_rsrc_t r, unsigned o, unsigned &v)
+{
+    v = __builtin_amdgcn_raw_buffer_load_b32(r, o, 0, 0);
+}
+__device__ __forceinline__ void bld(__amdgpu_buffer_rsrc_t r, unsigned o, float &v)
+{
+    v = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, o, 0, 0));
+}
+__device__ __forceinline__ void bld(__amdgpu_buffer_rsrc_t r, unsigned o, double &v)
+{
+    v = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, o, 0, 0));
+}
+__device__ __forceinline__ void bst(__amdgpu_buffer_rsrc_t r, unsigned o, unsigned v)
+{
+    __builtin_amdgcn_raw_buffer_store_b32(v, r, o, 0, 0);
+}
+__device__ __forceinline__ void bst(__amdgpu_buffer_rsrc_t r, unsigned o, float v)
+{
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), r, o, 0, 0);
+}
+__device__ __forceinline__ void bst(__amdgpu_buffer_rsrc_t r, unsigned o, double v)
+{
+    typedef unsigned U2 __attribute__((ext_vector_type(2)));
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(U2, v), r, o, 0, 0);
+}
+template <int V>
+struct Int {
+    static constexpr int v = V;
+};
+// one side's layers as a wave of the march meets them in its row j: sides along y and z are
+// fixed, the side along x is that of the plane
+struct MarchFaces {
+    const CpmlDim *D;
+    int j, k, ys, zs;
+    bool anyz;  // a lane of the wave lies in a z layer
+    __device__ __forceinline__ int side_of(int d, int p) const { return d == 0 ? cpml_side(D[0], p) : ys; }
+    // The row's offset in a slab (elements, scalar), the bytes of its buffer and the lane's offset
+    // in it: along x and y the wave's one side (none: no bytes), along z the lane's own.
+    template <typename T>
+    __device__ __forceinline__ long long at(int d, int p, bool live, unsigned &bytes, unsigned &o) const
+    {
+        const CpmlDim &C = D[d];
+        const long long row = (long long)p * C.s0 + (long long)j * C.s1;
+        if (d == 2) {
+            const int low = min(C.off[0], C.off[1]);
+            bytes = anyz ? BUF_OUT : 0u;
+            o = live && zs >= 0 ? (unsigned)(k + (zs == 0 ? C.off[0] : C.off[1]) - low) * (unsigned)sizeof(T) : BUF_OUT;
+            return row + low;
+        }
+        const int side = side_of(d, p);
+        bytes = side >= 0 ? BUF_OUT : 0u;
+        o = live ? (unsigned)k * (unsigned)sizeof(T) : BUF_OUT;
+        return row + (side == 0 ? C.off[0] : C.off[1]);
+    }
+    // MODE: 1 the layers along z alone, 2 all three
+    template <int MODE, typename T, bool RES>
+    __device__ __forceinline__ void request(int p, MarchAux<T, RES> &m) const
+    {
 #pragma unroll
-    for (int d = 0; d < 3; ++d)
+        for (int d = MODE == 2 ? 0 : 2; d < 3; ++d) {
+            if (MODE == 0) continue;
+            unsigned bytes, o;
+            const long long q = at<T>(d, p, true, bytes, o);
+            bld(buf((const T *)D[d].o0 + q, bytes), o, m.x[d].o0);
+            bld(buf((const T *)D[d].o1 + q, bytes), o, m.x[d].o1);
+            if (RES) bld(buf(D[d].orw + q, bytes), o, m.x[d].w);
+        }
+    }
+    // The current totals gain the auxiliaries of plane p in the list order y, x, z (cpml_add).
+    // live: this lane's cell is the wave's to store; zb, zc: its z coefficients
+    template <int MODE, typename T, bool HSIDE, bool STORE, bool RES>
+    __device__ __forceinline__ void add(int p, const MarchAux<T, RES> &m, const double df[3][2], bool live, double zb,
+                                        double zc, double J[3]) const
+    {
 #pragma unroll
-        for (int q = 0; q < 2; ++q) {
-            const int f = eside ? a.efbd[d][q] : a.hfbd[d][q];
-            if (f >= 0) {
-                const CpmlFace &F = eside ? a.eface[f] : a.hface[f];
-                in |= x[d] >= F.lo[d] && x[d] <= F.hi[d];
+        for (int u = MODE == 2 ? 0 : 2; u < 3; ++u) {
+            constexpr int order[3] = {1, 0, 2};
+            const int d = order[u], side = d == 2 ? zs : side_of(d, p), coord = d == 0 ? p : (d == 1 ? j : k);
+            if (MODE == 0) continue;
+            const CpmlDim &C = D[d];
+            T h0{}, h1{};
+            unsigned w = 0;
+            if (side >= 0) {
+                double bq = zb, cq = zc, v0, v1;
+                if (d != 2) {
+                    const double *line = C.bc + (2 * side * C.len + coord);
+                    bq = kload(line);
+                    cq = kload(line + C.len);
+                }
+                cpml_next<T, HSIDE, RES>(C.idxn, bq, cq, m.x[d], df[d][1], df[d][0], h0, h1, w, v0, v1);
+                J[(d + 1) % 3] += v0;
+                J[(d + 2) % 3] += v1;
+                // layers that overlap (a box shorter than two of them): the low face too, loaded on the spot
+                if (MODE == 2 && C.two && side == 0 && coord >= C.lo[1] && coord <= C.hi[1]) {
+                    const double *line = C.bc + (2 * C.len + coord);
+                    const int l = cpml_index(C, 1, p, j, k);
+                    cpml_update<T, HSIDE, RES>(C, gld(line), gld(line + C.len), l, cpml_load<T, RES>(C, l), df[d][1],
+                                               df[d][0], STORE && live, v0, v1);
+                    J[(d + 1) % 3] += v0;
+                    J[(d + 2) % 3] += v1;
+                }
+            }
+            if (STORE) {
+                unsigned bytes, o;
+                const long long q = at<T>(d, p, live, bytes, o);
+                bst(buf((T *)C.p0 + q, bytes), o, h0);
+                bst(buf((T *)C.p1 + q, bytes), o, h1);
+                if (RES) bst(buf(C.rw + q, bytes), o, w);
             }
         }
-    return in;
-}
+    }
+};
 
 // accumulators of the active poles through one base pointer per pole: component q of a pole
 // sits 64 elements after component q - 1 (psi_at), so a lane needs one address per pole
@@ -490,6 +508,7 @@ __device__ __forceinline__ void march_tile(const PassArgs<T> &a, int tz, int ty,
     // brow[b][s]: B^(n+1) (x, z) of slot s; bcol[b][l]: B^(n+1) (x, y) of the column k0 - 1 of
     // tile row l; ecol[b][l]: E (x, y) of the right-end neighbour of tile row l
     __shared__ RowD erow[2][R + 2], brow[2][R + 1], bcol[2], ecol[2];
+    __shared__ RowD ztab[2];  // b (a) and c (b) of the z layers at the tile's 64 z cells, H and E side
 
     const int lane = threadIdx.x;
     const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.y);  // wave-uniform role
@@ -532,6 +551,35 @@ __device__ __forceinline__ void march_tile(const PassArgs<T> &a, int tz, int ty,
         sh = __ballot(sh) != 0;
         const double khy = kload(a.ikdH[1] + j), khz = gld(a.ikdH[2] + k);
         const double khyc = gld(a.ikdH[1] + (col ? jc : j)), khzc = kload(a.ikdH[2] + kc);
+        // the layers of the halo row, as a row wave has them, and of the column (sides along x and z
+        // uniform, along y the lane's own, with its coefficients)
+        MarchFaces F{a.hcd, j, k, -1, -1, false};
+        int cys = -1;
+        double cyb = 0.0, cyc = 0.0;
+        if (CPML) {
+            const int ze = cpml_side(a.ecd[2], k);
+            F.ys = cpml_side(a.hcd[1], j);
+            F.zs = cpml_side(a.hcd[2], k);
+            F.anyz = __ballot(F.zs >= 0) != 0;
+            const double *lh = a.hcd[2].bc + (2 * (F.zs < 0 ? 0 : F.zs) * a.hcd[2].len + k);
+            const double *le = a.ecd[2].bc + (2 * (ze < 0 ? 0 : ze) * a.ecd[2].len + k);
+            if (F.zs >= 0) {
+                ztab[0].a[lane] = gld(lh);
+                ztab[0].b[lane] = gld(lh + a.hcd[2].len);
+            }
+            if (ze >= 0) {
+                ztab[1].a[lane] = gld(le);
+                ztab[1].b[lane] = gld(le + a.ecd[2].len);
+            }
+            if (col) cys = cpml_side(a.hcd[1], jc);
+            if (cys >= 0) {
+                const double *line = a.hcd[1].bc + (2 * cys * a.hcd[1].len + jc);
+                cyb = gld(line);
+                cyc = gld(line + a.hcd[1].len);
+            }
+        }
+        const int czs = CPML ? cpml_side(a.hcd[2], kc) : -1;
+        const bool anycy = CPML && __ballot(cys >= 0) != 0;
         // E of the row above the tile and of the right-end cells at plane p, into buffer b
         auto provide = [&](int p, int b) {
             const size_t bp = (size_t)p * sx;
@@ -558,28 +606,81 @@ __device__ __forceinline__ void march_tile(const PassArgs<T> &a, int tz, int ty,
             const RW ce0 = ldp3<T, RES>(a.Eo, a.Eolo, bp, oc * SZ), cb0 = ldp3<T, RES>(a.Bo, a.Bolo, bp, oc * SZ);
             const RW cez = ldp3<T, RES>(a.Eo, a.Eolo, bp, ocz * SZ), ceu = ldp3<T, RES>(a.Eo, a.Eolo, bp, ocy * SZ);
             const RW cen = ldp3<T, RES>(a.Eo, a.Eolo, bn, oc * SZ);
-            bool cp = false;
-            if (CPML) cp = __ballot((ok && in_cpml(a, false, p, j, k)) || (col && in_cpml(a, false, p, jc, kc))) != 0;
+            MarchAux<T, RES> ma;  // and the row's auxiliaries
+            if (CPML) F.template request<2, T, RES>(p, ma);
             {  // the halo row; E of its y + 1 row is the tile's first row (slot 1)
                 const C3 e = cell_of(e0), n = cell_of(en), z = cell_of(ez);
                 const double d[6] = {(double)z.y - e.y, (double)z.x - e.x, erow[be][1].b[lane] - e.z,
                                      erow[be][1].a[lane] - e.x, (double)n.z - e.z, (double)n.y - e.y};
                 T h[3];
                 unsigned hw;
-                double b[3];
-                b_cell_k<T, CPML, RES>(a, p, j, k, cell_of(b0), d, false, h, hw, b, cp, sh, soff, ok, kxh, khy, khz);
+                double b[3], M[3];
+                pass_m<T>(a, p, j, k, M, sh, soff, [&](double M[3]) {
+                    if (CPML) {
+                        const double df[3][2] = MPX_DIFF_E(d);
+                        F.template add<2, T, true, false, RES>(p, ma, df, false, ztab[0].a[lane], ztab[0].b[lane], M);
+                    }
+                });
+                b_cell<T, RES>(a, cell_of(b0), d, M, kxh, khy, khz, h, hw, b);
                 brow[bb][0].a[lane] = b[0];
                 brow[bb][0].b[lane] = b[2];
             }
-            {  // the column
+            {  // the column; its auxiliaries are requested here, where the row's have left their registers
+                const int xs = CPML ? cpml_side(a.hcd[0], p) : -1, jl = col ? jc : j;
+                MarchAux<T, RES> ca;
+                if (xs >= 0) ca.x[0] = cpml_load<T, RES>(a.hcd[0], cpml_index(a.hcd[0], xs, p, jl, kc));
+                if (anycy) ca.x[1] = cpml_load<T, RES>(a.hcd[1], cys >= 0 ? cpml_index(a.hcd[1], cys, p, jl, kc) : 0);
+                if (czs >= 0) ca.x[2] = cpml_load<T, RES>(a.hcd[2], cpml_index(a.hcd[2], czs, p, jl, kc));
                 const C3 e = cell_of(ce0), z = cell_of(cez), u = cell_of(ceu), n = cell_of(cen);
                 const double d[6] = {(double)z.y - e.y, (double)z.x - e.x, (double)u.z - e.z, (double)u.x - e.x,
                                      (double)n.z - e.z, (double)n.y - e.y};
                 T h[3];
                 unsigned hw;
-                double b[3];
-                b_cell_k<T, CPML, RES>(a, p, col ? jc : j, col ? kc : k, cell_of(cb0), d, kzero, h, hw, b, cp, sh,
-                                       soff, col, kxh, khyc, khzc);
+                double b[3], M[3];
+                pass_m<T>(a, p, jl, kc, M, sh, soff, [&](double M[3]) {
+                    if (CPML) {
+                        const double df[3][2] = MPX_DIFF_E(d);
+                        const bool st = kzero && col;
+                        double v0, v1;
+                        auto second = [&](int d, int coord) {  // overlapping layers
+                            const CpmlDim &C = a.hcd[d];
+                            if (C.two && coord <= C.hi[0] && coord >= C.lo[0] && coord >= C.lo[1] && coord <= C.hi[1]) {
+                                const double *line = C.bc + (2 * C.len + coord);
+                                const int l = cpml_index(C, 1, p, jl, kc);
+                                cpml_update<T, true, RES>(C, gld(line), gld(line + C.len), l, cpml_load<T, RES>(C, l),
+                                                          df[d][1], df[d][0], st, v0, v1);
+                                M[(d + 1) % 3] += v0;
+                                M[(d + 2) % 3] += v1;
+                            }
+                        };
+                        if (anycy && cys >= 0) {
+                            cpml_update<T, true, RES>(a.hcd[1], cyb, cyc, cpml_index(a.hcd[1], cys, p, jl, kc), ca.x[1],
+                                                      df[1][1], df[1][0], st, v0, v1);
+                            M[2] += v0;
+                            M[0] += v1;
+                            second(1, jl);
+                        }
+                        if (xs >= 0) {
+                            const double *line = a.hcd[0].bc + (2 * xs * a.hcd[0].len + p);
+                            cpml_update<T, true, RES>(a.hcd[0], kload(line), kload(line + a.hcd[0].len),
+                                                      cpml_index(a.hcd[0], xs, p, jl, kc), ca.x[0], df[0][1], df[0][0],
+                                                      st, v0, v1);
+                            M[1] += v0;
+                            M[2] += v1;
+                            second(0, p);
+                        }
+                        if (czs >= 0) {
+                            const double *line = a.hcd[2].bc + (2 * czs * a.hcd[2].len + kc);
+                            cpml_update<T, true, RES>(a.hcd[2], kload(line), kload(line + a.hcd[2].len),
+                                                      cpml_index(a.hcd[2], czs, p, jl, kc), ca.x[2], df[2][1], df[2][0],
+                                                      st, v0, v1);
+                            M[0] += v0;
+                            M[1] += v1;
+                            second(2, kc);
+                        }
+                    }
+                });
+                b_cell<T, RES>(a, cell_of(cb0), d, M, kxh, khyc, khzc, h, hw, b);
                 bcol[bb].a[lane] = b[0];
                 bcol[bb].b[lane] = b[1];
                 if (kzero && col) {
@@ -629,6 +730,36 @@ __device__ __forceinline__ void march_tile(const PassArgs<T> &a, int tz, int ty,
         for (int n = 0; n < NP; ++n) psb.b[n] = a.psi[n][0];
         const double khy = kload(a.ikdH[1] + j), khz = gld(a.ikdH[2] + k);
         const double key = kload(a.ikdE[1] + j), kez = gld(a.ikdE[2] + k);
+        MarchFaces FH{a.hcd, j, k, -1, -1, false}, FE{a.ecd, j, k, -1, -1, false};
+        if (CPML) {
+            FH.ys = cpml_side(a.hcd[1], j);
+            FH.zs = cpml_side(a.hcd[2], k);
+            FH.anyz = __ballot(FH.zs >= 0) != 0;
+            FE.ys = cpml_side(a.ecd[1], j);
+            FE.zs = cpml_side(a.ecd[2], k);
+            FE.anyz = __ballot(FE.zs >= 0) != 0;
+        }
+        // Which layers the wave's cells meet in this segment: none, those along z, or others.  Each has a
+        // body of its own, so that within it every wave issues the same memory operations on every path.
+        int mode = 0;
+        if (CPML) {
+            auto meets = [&](const CpmlDim *D) {
+                bool x = D[0].two || D[1].two || D[2].two;
+                for (int q = 0; q < 2; ++q) x |= (D[0].lo[q] <= min(D[0].hi[q], i1) && D[0].hi[q] >= i0) || (D[0].lo[q] <= pm && pm <= D[0].hi[q]);
+                return x;
+            };
+            mode = FH.ys >= 0 || FE.ys >= 0 || meets(a.hcd) || meets(a.ecd) ? 2 : (FH.anyz || FE.anyz ? 1 : 0);
+            mode = __builtin_amdgcn_readfirstlane(mode);
+        }
+        auto rows = [&](auto mode, int lane, int k, unsigned o, unsigned os) {
+        constexpr int MODE = decltype(mode)::v;
+        // opaque copies: what the body derives from them is not formed, and kept, ahead of all three
+        hold(lane);
+        hold(k);
+        hold(o);
+        hold(os);
+        FH.k = FE.k = k;
+        MarchAux<T, RES> mh, me;  // this plane's auxiliaries, H and E side
         // E^(n+1) of the row at p + 1 and B^n at p (real: at the lane's cell, else at the
         // padding position 0), the cell's permittivity
         struct Stage {
@@ -652,7 +783,7 @@ __device__ __forceinline__ void march_tile(const PassArgs<T> &a, int tz, int ty,
         };
         // B^(n+1) of the row at plane p from E^(n+1) at p (e, decoded), at p + 1 (n) and the
         // E rows above and to the right (LDS buffer be); CPML H auxiliaries stored with `store`
-        auto bstep = [&](int p, int be, const C3 &e, const C3 &n, const RW &b0w, bool store, bool cp, double kxh,
+        auto bstep = [&](auto store, int p, int be, const C3 &e, const C3 &n, const RW &b0w, double kxh,
                          T h[3], unsigned &hw, double b[3]) {
             double zx = lane_next((double)e.x), zy = lane_next((double)e.y);
             if (lane == lr) {
@@ -661,23 +792,31 @@ __device__ __forceinline__ void march_tile(const PassArgs<T> &a, int tz, int ty,
             }
             const double d[6] = {zy - e.y, zx - e.x, erow[be][w + 1].b[lane] - e.z, erow[be][w + 1].a[lane] - e.x,
                                  (double)n.z - e.z, (double)n.y - e.y};
-            b_cell_k<T, CPML, RES>(a, p, j, k, cell_of(b0w), d, store, h, hw, b, cp, sh, soff, ok, kxh, khy, khz);
+            double M[3];
+            pass_m<T>(a, p, j, k, M, sh, soff, [&](double M[3]) {
+                if (CPML) {
+                    const double df[3][2] = MPX_DIFF_E(d);
+                    FH.template add<MODE, T, true, decltype(store)::v != 0, RES>(p, mh, df, ok, ztab[0].a[lane],
+                                                                                ztab[0].b[lane], M);
+                }
+            });
+            b_cell<T, RES>(a, cell_of(b0w), d, M, kxh, khy, khz, h, hw, b);
         };
         Stage cur;
         C3 e = cell_of(ldp3<T, RES>(a.Eo, a.Eolo, (size_t)pm * sx, o * SZ));  // E^(n+1) at plane pm
         load(pm, true, cur);
+        if (CPML) FH.template request<MODE, T, RES>(pm, mh);
         erow[0][w].a[lane] = e.x;
         erow[0][w].b[lane] = e.z;
         lds_barrier();
         // the segment's x - 1 plane: B^(n+1) recomputed there (not stored), for the first plane's E
         double bp1, bp2;  // By, Bz of B^(n+1) at plane p - 1
         {
-            const bool cp = CPML && __ballot(ok && in_cpml(a, false, pm, j, k)) != 0;
             const C3 n = cell_of(cur.en);
             T h[3];
             unsigned hw;
             double b[3];
-            bstep(pm, 0, e, n, cur.b0, false, cp, kload(a.ikdH[0] + pm), h, hw, b);
+            bstep(Int<0>{}, pm, 0, e, n, cur.b0, kload(a.ikdH[0] + pm), h, hw, b);
             bp1 = b[1];
             bp2 = b[2];
             e = n;
@@ -685,6 +824,7 @@ __device__ __forceinline__ void march_tile(const PassArgs<T> &a, int tz, int ty,
             erow[1][w].b[lane] = e.z;
         }
         load(i0, true, cur);
+        if (CPML) FH.template request<MODE, T, RES>(i0, mh);
         PsiRegs<NP> pr;
         load_psi(i0, true, pr);
         lds_barrier();
@@ -694,15 +834,15 @@ __device__ __forceinline__ void march_tile(const PassArgs<T> &a, int tz, int ty,
             const size_t bp = (size_t)p * sx;
             const unsigned ob = os * SZ;
             const double kxh = kload(a.ikdH[0] + p), kxe = kload(a.ikdE[0] + p);
-            const bool cp = CPML && __ballot(ok && (in_cpml(a, false, p, j, k) || in_cpml(a, true, p, j, k))) != 0;
             const C3 n = cell_of(cur.en);  // E^(n+1) at p + 1
             const double ee = cur.eps;
             T bh[3];
             unsigned bw;
             double b[3];
-            bstep(p, be, e, n, cur.b0, true, cp, kxh, bh, bw, b);
+            bstep(Int<1>{}, p, be, e, n, cur.b0, kxh, bh, bw, b);
             // the next plane's words, once this plane's are consumed
             load(last ? p : p + 1, !last, cur);
+            FE.template request<MODE, T, RES>(p, me);
             stp_once(a.Bn[0] + bp, ob, bh[0]);
             stp_once(a.Bn[1] + bp, ob, bh[1]);
             stp_once(a.Bn[2] + bp, ob, bh[2]);
@@ -743,9 +883,13 @@ __device__ __forceinline__ void march_tile(const PassArgs<T> &a, int tz, int ty,
                     }
                 }
             }
-            double jx, jy, jz;
-            pass_j<T, CPML, RES>(a, p, j, k, dBz_y, dBy_z, dBx_z, dBz_x, dBy_x, dBx_y, jx, jy, jz, cp, sh, soff, ok,
-                                 PL ? jpv : nullptr);
+            double J[3];
+            pass_j<T>(a, p, j, k, J, sh, soff, PL ? jpv : nullptr, [&](double J[3]) {
+                if (CPML) {
+                    const double df[3][2] = {{dBy_x, dBz_x}, {dBz_y, dBx_y}, {dBx_z, dBy_z}};
+                    FE.template add<MODE, T, false, true, RES>(p, me, df, ok, ztab[1].a[lane], ztab[1].b[lane], J);
+                }
+            });
             double idenom = a.idenom, numer = a.numer;
             if (a.epsf || (PL && a.plasma)) {  // cell_eps with the prefetched permittivity and Sigma dt / 2
                 const double e0 = a.epsf ? ee : a.eps, sgh = 0.5 * sg * a.dt;
@@ -756,7 +900,7 @@ __device__ __forceinline__ void march_tile(const PassArgs<T> &a, int tz, int ty,
             double nex = e.x, ney = e.y, nez = e.z;
             unsigned lf = 0;
             plrc_e_update_pp<NP, NONLIN, true>(nex, ney, nez, dBz_y, dBy_z, dBx_z, dBz_x, dBy_x, dBx_y, kxe, key,
-                                               kez, jx, jy, jz, pr, psb, bp + os, true, a.pc, a.dt, idenom, numer,
+                                               kez, J[0], J[1], J[2], pr, psb, bp + os, true, a.pc, a.dt, idenom, numer,
                                                a.chi, a.ncap, &lf);
             lf |= finite_flag(nex, ney, nez);
             fl |= ok ? lf : 0u;
@@ -767,10 +911,15 @@ __device__ __forceinline__ void march_tile(const PassArgs<T> &a, int tz, int ty,
             stp_once(a.En[2] + bp, ob, hz);
             if (RES) stp_once(a.Enlo + bp, ob, ew);
             load_psi(last ? p : p + 1, !last, pr);
+            FH.template request<MODE, T, RES>(last ? p : p + 1, mh);
             bp1 = b[1];
             bp2 = b[2];
             e = n;
         }
+        };
+        if (!CPML || mode == 0) rows(Int<0>{}, lane, k, o, os);
+        else if (mode == 1) rows(Int<CPML ? 1 : 0>{}, lane, k, o, os);
+        else rows(Int<CPML ? 2 : 0>{}, lane, k, o, os);
     }
     report(a.status, fl);
 }
@@ -784,9 +933,20 @@ __device__ __forceinline__ unsigned xcd_share(unsigned lin, unsigned total)
     return (lin < per * 8u) ? xcd * per + idx : lin;
 }
 
+// Waves per SIMD the registers are held to: four (128 VGPRs, so two 8-wave blocks fit a CU) for the
+// variants with layers that come within a few registers of it (float64 without poles 129, with one
+// 131, with two 142; two poles with residuals 137): the words that two poles spill cost less than a
+// third of the waves (131x158x177 with two poles 376 -> 352 us in float64).  Plain float32 fits by
+// itself and is faster left alone (10 runs of 48^3 to 160^3 55.6 with, 52.8 ms without for 60 steps);
+// three poles (162 and more) and the plasma variants keep their registers.
+template <typename T, int NP, bool CPML, bool RES, bool PL>
+struct MarchWaves {
+    static constexpr int v = CPML && !PL && NP <= 2 && (sizeof(T) == 8 || RES) ? 4 : 1;
+};
+
 // one grid: tiles in the order z tiles fastest, then tile rows, then x segments
 template <typename T, int NP, bool NONLIN, bool CPML, bool RES, int R, bool PL>
-__global__ __launch_bounds__(64 * (R + 1)) void k_march(const PassArgs<T> *__restrict__ pa, int nbz, int nby,
+__global__ __attribute__((amdgpu_waves_per_eu(MarchWaves<T, NP, CPML, RES, PL>::v))) __launch_bounds__(64 * (R + 1)) void k_march(const PassArgs<T> *__restrict__ pa, int nbz, int nby,
                                                         int nseg, int soff)
 {
     unsigned t = xcd_share(blockIdx.x, (unsigned)nbz * nby * nseg);
@@ -798,7 +958,7 @@ __global__ __launch_bounds__(64 * (R + 1)) void k_march(const PassArgs<T> *__res
 // Independent runs in one launch: run r owns the tiles runs[r].first .. runs[r+1].first - 1
 // of the list, in its own grid's order; its argument block is pa[r].
 template <typename T, int NP, bool NONLIN, bool CPML, bool RES, int R, bool PL>
-__global__ __launch_bounds__(64 * (R + 1)) void k_march_batch(const PassArgs<T> *__restrict__ pa,
+__global__ __attribute__((amdgpu_waves_per_eu(MarchWaves<T, NP, CPML, RES, PL>::v))) __launch_bounds__(64 * (R + 1)) void k_march_batch(const PassArgs<T> *__restrict__ pa,
                                                               const BatchRun *__restrict__ runs, int nruns,
                                                               int total)
 {

@@ -1773,22 +1773,10 @@ static mpx::PassArgs<T> pass_args(mpx_solver *s)
     a.pc = s->pc;
     a.nefaces = (int)s->efaces.size();
     a.nhfaces = (int)s->hfaces.size();
-    for (int d = 0; d < 3; ++d)
-        for (int q = 0; q < 2; ++q) a.efbd[d][q] = a.hfbd[d][q] = -1;
-    for (size_t f = 0; f < s->efaces.size(); ++f) a.eface[f] = s->efaces[f];
-    for (size_t f = 0; f < s->hfaces.size(); ++f) {
-        a.hface[f] = s->hfaces[f];
-        a.hface[f].psi0 = s->hpsi2[0][f];
-        a.hface[f].psi1 = s->hpsi2[1][f];
-        a.hface[f].rw = s->hrw2[f];
-        a.hold[f][0] = s->hfaces[f].psi0;
-        a.hold[f][1] = s->hfaces[f].psi1;
-        a.hold_rw[f] = s->hfaces[f].rw;
+    for (int d = 0; d < 3; ++d) {
+        a.ecd[d] = cpml_dim(s, false, d, false);
+        a.hcd[d] = cpml_dim(s, true, d, true);
     }
-    for (const Current &c : s->ecur)
-        if (c.face >= 0) a.efbd[dim_of(c.dir)][is_high(c.dir) ? 0 : 1] = c.face;
-    for (const Current &c : s->hcur)
-        if (c.face >= 0) a.hfbd[dim_of(c.dir)][is_high(c.dir) ? 0 : 1] = c.face;
     for (const Current &c : s->ecur)
         if (c.type == CUR_INC_E) a.sheet[a.nsheets++] = c.ev.sheet;
     for (const Current &c : s->hcur)
@@ -1866,6 +1854,22 @@ static int pass_launch_t(mpx_solver *s, int soff)
     return MPX_OK;
 }
 
+// Whether the march kernel can address the layers of s: its buffer offsets reach 2 GiB, the distance
+// of the two faces along z within one array (a face of more bytes has 2^28 cells or more).
+static bool march_fits(const mpx_solver *s)
+{
+    for (int h = 0; h < 2; ++h) {
+        const mpx::CpmlDim D = cpml_dim(s, h, 2, false);
+        const long long apart = (long long)D.off[0] - D.off[1];
+        if (((apart < 0 ? -apart : apart) + s->g.n[2] + 2) * (long long)s->esz >= (1LL << 31)) return false;
+    }
+    return true;
+}
+
+// Whether a pending B half and the next E half run as one pass (pass_launch_t) or as the two fused
+// kernels, which give the same bits
+static bool pass_in_one(const mpx_solver *s) { return s->pass_kernel != 1 || march_fits(s); }
+
 // One step on the pass path.  Settled state at time t (E^t, B^t): the E half of step t.
 // Pending state at time t (E^t, B^(t-1)): one pass, the B half of step t - 1 (H-side sheets
 // at t - 1) and the E half of step t (E-side sheets at t).  Either way the state is pending at
@@ -1877,9 +1881,14 @@ static int pass_step(mpx_solver *s, int ahead)
         if ((rc = fused_half(s, false, s->time))) return rc;
     } else {
         if ((rc = sheets_at(s, s->time, s->time - 1, ahead, &soff))) return rc;
-        rc = s->esz == 8 ? pass_launch_t<double>(s, soff) : pass_launch_t<float>(s, soff);
-        if (rc) return rc;
-        swap_pass_buffers(s);
+        if (pass_in_one(s)) {
+            rc = s->esz == 8 ? pass_launch_t<double>(s, soff) : pass_launch_t<float>(s, soff);
+            if (rc) return rc;
+            swap_pass_buffers(s);
+        } else
+            for (int side = 1; side >= 0; --side)
+                if ((rc = s->esz == 8 ? fused_half_t<double>(s, side, soff) : fused_half_t<float>(s, side, soff)))
+                    return rc;
     }
     s->pending = true;
     s->time++;
@@ -2907,6 +2916,7 @@ struct mpx_batch {
     int variant = 2, seg = 32, blocks_per_cu = 2, graph_steps = 50;  // sweep tiling
     int march_b = 4, fused_bpc = 8;  // fused B planes per thread, fused blocks per CU
     int pass_seg = 16, pass_rows = 0;  // x-march: planes per block, rows per tile (0: per variant)
+    bool march_ok = true;              // the march kernel takes every run (march_fits)
     int prows = 7;                     // x-march rows in use
     int cus = 256;
     int time = 0;
@@ -3289,6 +3299,7 @@ int mpx_batch_create(const mpx_desc *descs, int nruns, mpx_batch **out)
                              "batched runs must share precision, solver, active pole count and CPML presence"));
         }
         if (s->time != 0) return bail(fail(MPX_ERR_INVALID, "batched runs start at time 0"));
+        b->march_ok = b->march_ok && march_fits(s);
     }
     // source sheets of all runs
     std::vector<mpx::SheetTask> sheets;
@@ -3371,7 +3382,7 @@ int mpx_batch_set_tuning(mpx_batch *b, const char *key, int value)
     if (!std::strcmp(key, "structure")) {
         if (value < 0 || value > 2)
             return fail(MPX_ERR_INVALID, "structure must be 0 (fused), 1 (sweep) or 2 (x-march pass)");
-        b->structure = value;
+        b->structure = value == 2 && !b->march_ok ? 0 : value;  // the same bits
     } else if (!std::strcmp(key, "pass_seg")) {
         if (value < 1) return fail(MPX_ERR_INVALID, "pass_seg must be >= 1");
         b->pass_seg = value;
@@ -3443,7 +3454,8 @@ int mpx_batch_autotune(mpx_batch *b, int steps_per_trial, int result[4], double 
         for (int sg : {8, 16, 32})
             for (int bpc : {1, 2}) cands.push_back({1, v, sg, bpc});
     for (int sg : {8, 16, 32})
-        for (int rows : {3, 7}) cands.push_back({2, sg, rows, 0});
+        for (int rows : {3, 7})
+            if (b->march_ok) cands.push_back({2, sg, rows, 0});
     auto apply = [&](const Cand &c) {
         b->structure = c.structure;
         if (c.structure == 0) {

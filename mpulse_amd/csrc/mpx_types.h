@@ -308,12 +308,8 @@ struct PassArgs {
     double *rho, *jp[3], *sigma;
     PoleConsts pc;
     int nefaces, nhfaces;
-    CpmlFace eface[kMaxFaces];    // E auxiliaries, in place
-    int efbd[3][2];
-    CpmlFace hface[kMaxFaces];    // psi0 / psi1 / rw: the new H auxiliaries
-    const void *hold[kMaxFaces][2];   // the old H auxiliaries
-    const unsigned *hold_rw[kMaxFaces];
-    int hfbd[3][2];
+    CpmlDim ecd[3];               // E faces by dimension, updated in place
+    CpmlDim hcd[3];               // H faces: old auxiliaries read, the new ones written to the other set
     int nsheets, nhsheets;
     Sheet sheet[kMaxSheets];      // E-side sheets (J of step n + 1)
     Sheet hsheet[kMaxSheets];     // H-side sheets (M of step n)
