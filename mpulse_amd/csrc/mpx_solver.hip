@@ -256,6 +256,7 @@ struct mpx_solver {
     // 0 = one cell per thread (k_pass)
     // seg 0: 16 planes, fewer where the grid has too few tiles to fill the chip
     int pass_kernel = 1, march_seg = 0, march_rows = 0;  // rows 0: chosen per kernel variant
+    bool pass_set = false;         // one of the three was set: the pass runs at every size (pass_in_one)
     double *d_box = nullptr;       // staging of mpx_get_field / mpx_set_field: box_planes x planes
     int box_planes = 0;
     double *d_stage = nullptr;     // x-fastest float64 copy of one grid for mpx_fetch_field
@@ -1867,8 +1868,26 @@ static bool march_fits(const mpx_solver *s)
 }
 
 // Whether a pending B half and the next E half run as one pass (pass_launch_t) or as the two fused
-// kernels, which give the same bits
-static bool pass_in_one(const mpx_solver *s) { return s->pass_kernel != 1 || march_fits(s); }
+// kernels, which give the same bits.  A pass launches one kernel less and moves fewer bytes (E and B
+// cross memory once); the fused kernels hold more waves a SIMD and have no halo to recompute.
+// Measured (us a step, pass / two halves, one pole, layers of 4 to 16 cells):
+//   24^3 23.1 / 26.0 (float64), 64^3 34.1 / 36.9 (with residuals 37.4 / 34.2, 56^3 30.3 / 32.0): the
+//   launch decides; 96^3 97 / 83, 256^3 965 / 924,
+//   with residuals 256^3 829 / 748; float64 from about 2^25 cells on: 320^3 1570 / 1696, 512^3
+//   6138 / 6480; float32 with and without residuals draw level there (512^3 5061 / 5059).
+// Without layers the pass has no auxiliaries to wait for: float64 24^3 18.7 / 24.1, 128^3 98 / 107,
+// 256^3 698 / 734; float32 128^3 78 / 84, 256^3 520 / 488.
+// A pass_kernel, march_seg or march_rows set by the user asks for the pass.
+static bool pass_in_one(const mpx_solver *s)
+{
+    if (s->pass_kernel == 1 && !march_fits(s)) return false;
+    if (s->pass_set) return true;
+    const double cells = (double)s->g.n[0] * s->g.n[1] * s->g.n[2];
+    const bool layers = !s->efaces.empty() || !s->hfaces.empty();
+    if (cells <= (s->res ? 3 << 16 : 1 << 18)) return true;
+    if (layers || s->plasma || s->pcur) return s->esz == 8 && !s->plasma && !s->pcur && cells >= (1 << 25);
+    return s->esz == 8 || cells <= (1 << 22);
+}
 
 // One step on the pass path.  Settled state at time t (E^t, B^t): the E half of step t.
 // Pending state at time t (E^t, B^(t-1)): one pass, the B half of step t - 1 (H-side sheets
@@ -2875,13 +2894,16 @@ int mpx_set_tuning(mpx_solver *s, const char *key, int value)
     } else if (!std::strcmp(key, "pass_kernel")) {
         if (value != 0 && value != 1) return fail(MPX_ERR_INVALID, "pass_kernel must be 0 or 1");
         s->pass_kernel = value;
+        s->pass_set = true;
     } else if (!std::strcmp(key, "march_seg")) {
         if (value < 0) return fail(MPX_ERR_INVALID, "march_seg must be >= 1 (0: chosen from the grid)");
         s->march_seg = value;
+        s->pass_set |= value > 0;
     } else if (!std::strcmp(key, "march_rows")) {
         if (value != 0 && value != 3 && value != 7)
             return fail(MPX_ERR_INVALID, "march_rows must be 3 or 7 (0: chosen from the kernel's registers)");
         s->march_rows = value;
+        s->pass_set |= value > 0;
     } else if (!std::strcmp(key, "sweep_variant")) {
         if (value < 0 || value > 2) return fail(MPX_ERR_INVALID, "sweep_variant must be 0, 1 or 2");
         s->sweep_variant = value;
@@ -2915,7 +2937,7 @@ struct mpx_batch {
     int structure = 0;
     int variant = 2, seg = 32, blocks_per_cu = 2, graph_steps = 50;  // sweep tiling
     int march_b = 4, fused_bpc = 8;  // fused B planes per thread, fused blocks per CU
-    int pass_seg = 16, pass_rows = 0;  // x-march: planes per block, rows per tile (0: per variant)
+    int pass_seg = 16, pass_rows = 0;  // x-march: planes per block (at creation as in pass_args), rows per tile (0: per variant)
     bool march_ok = true;              // the march kernel takes every run (march_fits)
     int prows = 7;                     // x-march rows in use
     int cus = 256;
@@ -3301,6 +3323,16 @@ int mpx_batch_create(const mpx_desc *descs, int nruns, mpx_batch **out)
         if (s->time != 0) return bail(fail(MPX_ERR_INVALID, "batched runs start at time 0"));
         b->march_ok = b->march_ok && march_fits(s);
     }
+    // shorter x-march segments while 16 planes a block would give fewer than 2048 blocks (pass_args);
+    // 8 runs of 40^3 to 60^3 took 130 us a step with 16 planes throughout
+    for (auto blocks = [&] {
+             long long t = 0;
+             for (const mpx_solver *s : b->runs)
+                 t += (long long)((s->g.n[2] + 63) / 64) * ((s->g.n[1] + 2) / 3) * ((s->g.n[0] + b->pass_seg - 1) / b->pass_seg);
+             return t;
+         };
+         b->pass_seg > 2 && blocks() < 2048;)
+        b->pass_seg /= 2;
     // source sheets of all runs
     std::vector<mpx::SheetTask> sheets;
     std::vector<int> first;
