@@ -563,10 +563,11 @@ __device__ __forceinline__ unsigned fast_div(unsigned t, const FastDiv &f)
 {
     return (unsigned)(((unsigned long long)t * f.m) >> f.sh);
 }
-__device__ __forceinline__ void map_tile(const TileMap &M, int &bx, int &by, int &bz)
+__device__ __forceinline__ bool map_tile(const TileMap &M, int &bx, int &by, int &bz)
 {
-    const unsigned lin = blockIdx.x;
-    unsigned t = lin < M.per * 8u ? (lin & 7u) * M.per + (lin >> 3) : lin;
+    const unsigned x = blockIdx.x & 7u;
+    unsigned t = M.at[x] + (blockIdx.x >> 3);
+    if (t >= M.at[x + 1]) return false;
     if (M.order == 2) {
         if (M.rev) t = M.total - 1u - t;
         const unsigned b = fast_div(t, M.full);
@@ -591,6 +592,7 @@ __device__ __forceinline__ void map_tile(const TileMap &M, int &bx, int &by, int
             bz = z;
         }
     }
+    return true;
 }
 
 // Whether coordinate coord of dimension dim lies in the layer of the high-side ([0]) and

@@ -395,7 +395,7 @@ __global__ __attribute__((amdgpu_waves_per_eu(FusedEWaves<T, NP, NONLIN, L, RES>
     const StepArgs<T> *__restrict__ pa, TileMap map, int soff)
 {
     int tbx, tby, tbz;
-    map_tile(map, tbx, tby, tbz);
+    if (!map_tile(map, tbx, tby, tbz)) return;
     fused_E_tile<T, NP, NONLIN, CPML, L, false, RES>(*pa, tbx, tby, tbz, soff);
 }
 
@@ -403,7 +403,7 @@ template <typename T, bool CPML, int L, bool RES = false>
 __global__ __launch_bounds__(256) void k_fused_B(const StepArgs<T> *__restrict__ pa, TileMap map, int soff)
 {
     int tbx, tby, tbz;
-    map_tile(map, tbx, tby, tbz);
+    if (!map_tile(map, tbx, tby, tbz)) return;
     fused_B_tile<T, CPML, L, false, RES>(*pa, tbx, tby, tbz, soff);
 }
 
@@ -502,14 +502,28 @@ template void launch_fused_B_batch<float>(const StepArgs<float> *, const BatchRu
                                           hipStream_t);
 #endif
 
+// The block order of a launch.  bytes: what a cell without layers reads and writes; a layer adds the
+// reads and writes of two auxiliaries (and their residual word).  Shares of equal work from 2048 tiles
+// on (eight blocks a CU), where the XCDs run long enough to end at different times; equal / balanced, us
+// a step with layers of 6 to 16 cells: 96x88x120 84.4 / 82.2, 131x158x177 211.5 / 207.6 (float32 +
+// residual 179.4 / 175.0), 256^3 925 / 899 (748 / 726; float32 615 / 607), 512^3 4998 / 4980.
+template <typename T>
+static TileMap fused_map(const StepArgs<T> &a, int nbx, int nby, int nbz, int L, int j0, int i0, double bytes)
+{
+    TileMap m = tile_map(nbx, nby, nbz, a.order, a.band, a.rev);
+    if (a.order == 2 && a.nfaces > 0 && m.total >= 2048)
+        balance_shares(m, nbx, nby, nbz, L, j0, i0, a.cd, (4.0 * sizeof(T) + (a.Elo ? 8 : 0)) / bytes);
+    return m;
+}
+
 template <typename T, int L, bool RES = false>
 static void launch_fused_E_L(const StepArgs<T> &a, const StepArgs<T> *dev, int np, bool nonlin, int soff,
                              hipStream_t s)
 {
     const GridDims &g = a.g;
     int nbx = (g.n[2] + 63) / 64, nby = (g.n[1] + 3) / 4, nbz = (g.n[0] + L - 1) / L;
-    dim3 blk(64, 4), grd((unsigned)nbx * nby * nbz);
-    const TileMap map = tile_map(nbx, nby, nbz, a.order, a.band, a.rev);
+    const TileMap map = fused_map<T>(a, nbx, nby, nbz, L, 1, 1, (3 * 3 * sizeof(T) + (RES ? 3 * 4 : 0)) + 96.0 * np);
+    dim3 blk(64, 4), grd(tile_blocks(map));
     bool cp = a.nfaces > 0;
 #define MPX_FE(NPV, NL, CP) hipLaunchKernelGGL((k_fused_E<T, NPV, NL, CP, L, RES>), grd, blk, 0, s, dev, map, soff)
 #define MPX_FE_NP(NL, CP)            \
@@ -551,8 +565,8 @@ static void launch_fused_B_L(const StepArgs<T> &a, const StepArgs<T> *dev, int s
     const GridDims &g = a.g;
     int nk = g.n[2] - a.blo[2] + 1, nj = g.n[1] - a.blo[1] + 1, ni = g.n[0] - a.blo[0] + 1;
     int nbx = (nk + 63) / 64, nby = (nj + 3) / 4, nbz = (ni + L - 1) / L;
-    dim3 blk(64, 4), grd((unsigned)nbx * nby * nbz);
-    const TileMap map = tile_map(nbx, nby, nbz, a.order, a.band, a.rev);
+    const TileMap map = fused_map<T>(a, nbx, nby, nbz, L, a.blo[1], a.blo[0], 3 * 3 * sizeof(T) + (RES ? 3 * 4 : 0));
+    dim3 blk(64, 4), grd(tile_blocks(map));
     if (a.nfaces > 0)
         hipLaunchKernelGGL((k_fused_B<T, true, L, RES>), grd, blk, 0, s, dev, map, soff);
     else

@@ -1872,9 +1872,9 @@ static bool march_fits(const mpx_solver *s)
 // cross memory once); the fused kernels hold more waves a SIMD and have no halo to recompute.
 // Measured (us a step, pass / two halves, one pole, layers of 4 to 16 cells):
 //   24^3 23.1 / 26.0 (float64), 64^3 34.1 / 36.9 (with residuals 37.4 / 34.2, 56^3 30.3 / 32.0): the
-//   launch decides; 96^3 97 / 83, 256^3 965 / 924,
-//   with residuals 256^3 829 / 748; float64 from about 2^25 cells on: 320^3 1570 / 1696, 512^3
-//   6138 / 6480; float32 with and without residuals draw level there (512^3 5061 / 5059).
+//   launch decides; 96^3 97 / 83, 256^3 932 / 899, with residuals 256^3 829 / 726; float64 from
+//   about 2^25 cells on: 320^3 1598 / 1696, 512^3 6138 / 6480; float32 with and without residuals
+//   draws level there (512^3 5061 / 5059 with).
 // Without layers the pass has no auxiliaries to wait for: float64 24^3 18.7 / 24.1, 128^3 98 / 107,
 // 256^3 698 / 734; float32 128^3 78 / 84, 256^3 520 / 488.
 // A pass_kernel, march_seg or march_rows set by the user asks for the pass.

@@ -176,7 +176,7 @@ inline FastDiv fast_divisor(unsigned d)
 // Block -> tile of the fused kernels (map_tile): nbx x nby x nbz tiles dealt to the 8 XCDs in
 // contiguous shares of one of three orders
 struct TileMap {
-    unsigned total, per;     // tiles, and tiles per XCD share
+    unsigned total, at[9];   // tiles; XCD x takes at[x] .. at[x + 1] - 1 of the order
     int order, rev, nbands;  // StepArgs::order, rev
     FastDiv first, second;   // the order's fastest and second dimension (order 2: nbx)
     FastDiv full, rband, rlast;  // order 2: tiles of a full band, its rows, the last band's rows
@@ -185,7 +185,7 @@ inline TileMap tile_map(int nbx, int nby, int nbz, int order, int band, int rev)
 {
     TileMap m{};
     m.total = (unsigned)nbx * nby * nbz;
-    m.per = m.total / 8u;
+    for (unsigned x = 0; x <= 8; ++x) m.at[x] = (unsigned)((unsigned long long)m.total * x / 8);
     m.order = order;
     m.rev = rev;
     if (band < 1) band = 1;
@@ -197,6 +197,48 @@ inline TileMap tile_map(int nbx, int nby, int nbz, int order, int band, int rev)
     m.rband = fast_divisor(band);
     m.rlast = fast_divisor(nby - (m.nbands - 1) * band);
     return m;
+}
+// Shares of equal work instead of equal tiles, in the banded order: tile (by, bz) holds rows 4 by + j0
+// .. and planes L bz + i0 .., and a cell in a layer of y or x (D) costs `extra` of a cell more, the bytes
+// of its auxiliaries over those of its words.  The order starts and ends in layers, so the first and
+// the last XCD's equal shares held most of them and the other six waited (z layers spread evenly).
+inline void balance_shares(TileMap &m, int nbx, int nby, int nbz, int L, int j0, int i0, const CpmlDim D[3], double extra)
+{
+    const int band = (int)m.rband.d;
+    auto in_layers = [](const CpmlDim &d, int lo, int n) {  // of the cells lo .. lo + n - 1
+        int c = 0;
+        for (int x = lo; x < lo + n; ++x) c += (x >= d.lo[0] && x <= d.hi[0]) || (x >= d.lo[1] && x <= d.hi[1]);
+        return (double)c / n;
+    };
+    double sx = 0, sy = 0;
+    for (int i = 0; i < nbz; ++i) sx += in_layers(D[0], i0 + L * i, L);
+    for (int j = 0; j < nby; ++j) sy += in_layers(D[1], j0 + 4 * j, 4);
+    const double all = nbx * ((double)nby * nbz + extra * (sx * nby + sy * nbz));
+    double sum = 0;
+    unsigned t = 0, at[9] = {0};
+    int x = 1;
+    for (int b = 0; b < m.nbands; ++b) {
+        const int r0 = b * band, rows = b == m.nbands - 1 ? (int)m.rlast.d : band;
+        double ly = 0;
+        for (int j = r0; j < r0 + rows; ++j) ly += in_layers(D[1], j0 + 4 * j, 4);
+        for (int i = 0; i < nbz; ++i) {
+            const unsigned n = (unsigned)nbx * rows;
+            const double c = nbx * (rows * (1 + extra * in_layers(D[0], i0 + L * i, L)) + extra * ly);
+            for (; x < 8 && sum + c >= all * x / 8; ++x) at[x] = t + (unsigned)(n * ((all * x / 8 - sum) / c));
+            sum += c;
+            t += n;
+        }
+    }
+    for (; x <= 8; ++x) at[x] = m.total;
+    for (x = 0; x <= 8; ++x) m.at[x] = m.rev ? m.total - at[8 - x] : at[x];
+}
+// blocks to launch: every XCD gets as many, those past its share leave at once
+inline unsigned tile_blocks(const TileMap &m)
+{
+    unsigned most = 0;
+    for (int x = 0; x < 8; ++x)
+        if (m.at[x + 1] - m.at[x] > most) most = m.at[x + 1] - m.at[x];
+    return 8 * most;
 }
 
 // PLRC pole constants (PLRCData, src/fdtd_plrc.h:71-78) of the active poles, precomputed on the
