@@ -336,41 +336,10 @@ struct PsiRegs {
 };
 
 
-// CPML auxiliaries of one face updated inside the fused kernels.  The face map is
-// x: (psi0 -> Jy from dBz, psi1 -> Jz from dBy), y: (psi0 -> Jz from dBx, psi1 -> Jx from dBz),
-// z: (psi0 -> Jx from dBy, psi1 -> Jy from dBx) (src/cpml_border.cpp:357-386, 456-485).
-// E side: CPMLBorderECurrent::stepScheme, src/cpml_border.cpp:398-425 (psi0 gets -c d1/dx);
-// H side: CPMLBorderHCurrent::stepScheme, src/cpml_border.cpp:499-527 (psi0 gets +c d1/dx).
-template <typename T, bool HSIDE, bool RES = false>
-__device__ __forceinline__ void cpml_face(const CpmlFace &f, int coord, int l, double d1, double d0, double &v0,
-                                          double &v1)
-{
-    int q = coord - f.lo[f.dim];
-    T *p0 = (T *)f.psi0, *p1 = (T *)f.psi1;
-    double bq = gld(f.b + q), cq = gld(f.c + q);
-    // ordinary loads: a face row covers only part of a cache line (z faces: 16 cells), and the
-    // rest of the line is read by the neighbouring row
-    const unsigned w = lo_ld<RES>(f.rw, l);
-    const double o0 = (double)rd<T, RES>(p0, w, 0, l), o1 = (double)rd<T, RES>(p1, w, 1, l);
-    double n0, n1;
-    if (HSIDE) {
-        n0 = bq * o0 + cq * d1 * f.idxn;
-        n1 = bq * o1 - cq * d0 * f.idxn;
-    } else {
-        n0 = bq * o0 - cq * d1 * f.idxn;
-        n1 = bq * o1 + cq * d0 * f.idxn;
-    }
-    // the current sums see the stored values
-    unsigned wn = 0;
-    const T h0 = put<T, RES>(n0, wn, 0), h1 = put<T, RES>(n1, wn, 1);
-    gst(p0 + l, h0);
-    gst(p1 + l, h1);
-    if (RES) gst(f.rw + l, wn);
-    v0 = got<T, RES>(h0, wn, 0);
-    v1 = got<T, RES>(h1, wn, 1);
-}
-
 // ---- CPML by dimension (CpmlDim) ----
+//
+// The face map is x: (psi0 -> Jy from dBz, psi1 -> Jz from dBy), y: (psi0 -> Jz from dBx, psi1 -> Jx
+// from dBz), z: (psi0 -> Jx from dBy, psi1 -> Jy from dBx) (src/cpml_border.cpp:357-386, 456-485).
 //
 // A cell's auxiliaries are requested with its field words and used after them, those of all
 // three dimensions together: taken face by face, each with its descriptor, coefficients and
@@ -593,18 +562,6 @@ __device__ __forceinline__ bool map_tile(const TileMap &M, int &bx, int &by, int
         }
     }
     return true;
-}
-
-// Whether coordinate coord of dimension dim lies in the layer of the high-side ([0]) and
-// low-side ([1]) CPML face of that dimension.  The face index itself stays uniform across
-// the wave (fbd[dim][s]), so the face descriptors are read with scalar loads.
-__device__ __forceinline__ void in_faces(const int fbd[3][2], const CpmlFace *faces, int dim, int coord, bool out[2])
-{
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {
-        int f = fbd[dim][s];
-        out[s] = f >= 0 && coord >= faces[f].lo[dim] && coord <= faces[f].hi[dim];
-    }
 }
 
 // (j, k) of this thread in a tile of the fused kernels: 64 z cells x 4 y rows, or (LIN) 256 consecutive cells of
