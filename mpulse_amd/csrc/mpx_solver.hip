@@ -2936,7 +2936,7 @@ struct mpx_batch {
     // and E of the next per launch; the fused E kernel opens a call, the fused B kernel closes it)
     int structure = 0;
     int variant = 2, seg = 32, blocks_per_cu = 2, graph_steps = 50;  // sweep tiling
-    int march_b = 4, fused_bpc = 8;  // fused B planes per thread, fused blocks per CU
+    int march_b = 2, fused_bpc = 8;  // fused B planes per thread (chosen at creation), fused blocks per CU
     int pass_seg = 16, pass_rows = 0;  // x-march: planes per block (at creation as in pass_args), rows per tile (0: per variant)
     bool march_ok = true;              // the march kernel takes every run (march_fits)
     int prows = 7;                     // x-march rows in use
@@ -3323,6 +3323,9 @@ int mpx_batch_create(const mpx_desc *descs, int nruns, mpx_batch **out)
         if (s->time != 0) return bail(fail(MPX_ERR_INVALID, "batched runs start at time 0"));
         b->march_ok = b->march_ok && march_fits(s);
     }
+    // B planes per thread, ms for 60 steps with 1 / 2 / 4: float64 10 runs of 48^3 to 160^3 76.0 / 74.1 /
+    // 76.2, 4 of 30^3 to 60^3 2.97 / 2.84 / 3.08; float32 55.5 / 56.8 / 57.0 and 2.20 / 2.28 / 2.58
+    b->march_b = b->esz == 8 ? 2 : 1;
     // shorter x-march segments while 16 planes a block would give fewer than 2048 blocks (pass_args);
     // 8 runs of 40^3 to 60^3 took 130 us a step with 16 planes throughout
     for (auto blocks = [&] {
