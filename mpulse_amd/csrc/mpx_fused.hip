@@ -49,12 +49,8 @@ struct At<false> {
         stp_once(p + row, k * (unsigned)sizeof(T), v);
     }
     // the accumulators (psi_at): the row's chunk is uniform, a lane counts on from it
-    __device__ __forceinline__ size_t psi_row() const { return ((row + PSI_SHIFT) >> 6) * 192; }
-    __device__ __forceinline__ unsigned psi_lane() const
-    {
-        const unsigned t = (unsigned)((row + PSI_SHIFT) & 63) + k;
-        return (t >> 6) * 192 + (t & 63);
-    }
+    __device__ __forceinline__ size_t psi_row() const { return psi_base(row); }
+    __device__ __forceinline__ unsigned psi_lane() const { return psi_ahead(row, k); }
 };
 template <>
 struct At<true> {
@@ -81,8 +77,11 @@ struct At<true> {
     {
         store_once(p + c, v);
     }
-    __device__ __forceinline__ size_t psi_row() const { return 0; }
-    __device__ __forceinline__ unsigned psi_lane() const { return (unsigned)psi_at(c); }
+    // the accumulators count on from the wave's first cell, its lowest: psi_at itself as a 32-bit lane
+    // offset wrapped at 4 GiB, storage cell 89478464 (a cube of 431^3)
+    __device__ __forceinline__ unsigned first() const { return (unsigned)__builtin_amdgcn_readfirstlane(c); }
+    __device__ __forceinline__ size_t psi_row() const { return psi_base(first()); }
+    __device__ __forceinline__ unsigned psi_lane() const { return psi_ahead(first(), (unsigned)c - first()); }
 };
 
 // Two or three components of a cell and its residual word, as stored

@@ -36,6 +36,14 @@ __host__ __device__ __forceinline__ size_t psi_at(size_t c)
 {
     return ((c + PSI_SHIFT) >> 6) * 192 + ((c + PSI_SHIFT) & 63);
 }
+// psi_at(c) in two parts for the cells of a wave, c0 being the lowest of them: psi_base(c0), the
+// same for all, and psi_ahead, 3 (c - c0) to within a chunk: small however large the block is
+__host__ __device__ __forceinline__ size_t psi_base(size_t c0) { return ((c0 + PSI_SHIFT) >> 6) * 192; }
+__host__ __device__ __forceinline__ unsigned psi_ahead(size_t c0, unsigned ahead)
+{
+    const unsigned t = (unsigned)((c0 + PSI_SHIFT) & 63) + ahead;
+    return (t >> 6) * 192 + (t & 63);
+}
 // double2 elements of one pole's block over `cells` storage cells
 inline size_t psi_block_elems(size_t cells) { return (((cells - 1 + PSI_SHIFT) >> 6) + 1) * 192; }
 
