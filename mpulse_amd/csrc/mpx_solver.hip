@@ -773,6 +773,32 @@ static int face_block(mpx_solver *s, FaceBlock &b, size_t cnt, int side, void *a
     return MPX_OK;
 }
 
+// The second set of one side's face auxiliaries: laid out as the first (CpmlDim takes one base and one
+// offset for both faces of a dimension, whichever set is in force), and the layers that show a face.
+static int second_faces(mpx_solver *s, const std::vector<CpmlFace> &faces, const std::vector<Current> &list,
+                        std::vector<void *> psi2[2], std::vector<int> layer[2], std::vector<unsigned *> *rw2)
+{
+    FaceBlock blk[3];
+    for (size_t f = 0; f < faces.size(); ++f) {
+        const CpmlFace &F = faces[f];
+        int side = 1;
+        for (const Current &c : list)
+            if (c.face == (int)f) side = is_high(c.dir) ? 0 : 1;
+        void *aux[2];
+        unsigned *rw = nullptr;
+        if (int rc = face_block(s, blk[F.dim], (size_t)(F.hi[0] - F.lo[0] + 1) * F.n1 * F.n2, side, aux, &rw)) return rc;
+        for (int w = 0; w < 2; ++w) {
+            psi2[w].push_back(aux[w]);
+            int li = -1;
+            for (size_t q = 0; q < s->layers.size(); ++q)
+                if (s->layers[q].comp[0] == (w == 0 ? F.psi0 : F.psi1)) li = (int)q;
+            layer[w].push_back(li);
+        }
+        if (rw2) rw2->push_back(rw);
+    }
+    return MPX_OK;
+}
+
 static int build(mpx_solver *s, const mpx_desc *desc)
 {
     s->d = *desc;
@@ -1229,19 +1255,7 @@ static int build(mpx_solver *s, const mpx_desc *desc)
                 if (rc) return rc;
                 for (int c = 0; c < 3; ++c) s->psi2[a][c] = base + 64 * c;
             }
-            for (size_t f = 0; f < s->efaces.size(); ++f) {
-                const CpmlFace &F = s->efaces[f];
-                size_t cnt = (size_t)(F.hi[0] - F.lo[0] + 1) * F.n1 * F.n2;
-                for (int w = 0; w < 2; ++w) {
-                    void *p = (s->esz == 8) ? (void *)s->dalloc<double>(cnt, rc) : (void *)s->dalloc<float>(cnt, rc);
-                    if (rc) return rc;
-                    s->epsi2[w].push_back(p);
-                    int li = -1;
-                    for (size_t q = 0; q < s->layers.size(); ++q)
-                        if (s->layers[q].comp[0] == (w == 0 ? F.psi0 : F.psi1)) li = (int)q;
-                    s->eface_layer[w].push_back(li);
-                }
-            }
+            if ((rc = second_faces(s, s->efaces, s->ecur, s->epsi2, s->eface_layer, nullptr))) return rc;
         }
     }
     // the pass path's second set; the sweep path (whose E2 and B2 are already there) takes the
@@ -1262,25 +1276,7 @@ static int build(mpx_solver *s, const mpx_desc *desc)
             s->B2lo = s->dalloc<unsigned>(s->cells, rc);
             if (rc) return rc;
         }
-        FaceBlock blk[3];
-        for (size_t f = 0; f < s->hfaces.size(); ++f) {
-            const CpmlFace &F = s->hfaces[f];
-            const size_t cnt = (size_t)(F.hi[0] - F.lo[0] + 1) * F.n1 * F.n2;
-            int side = 1;
-            for (const Current &c : s->hcur)
-                if (c.face == (int)f) side = is_high(c.dir) ? 0 : 1;
-            void *aux[2];
-            unsigned *rw = nullptr;
-            if ((rc = face_block(s, blk[F.dim], cnt, side, aux, &rw))) return rc;
-            for (int w = 0; w < 2; ++w) {
-                s->hpsi2[w].push_back(aux[w]);
-                int li = -1;
-                for (size_t q = 0; q < s->layers.size(); ++q)
-                    if (s->layers[q].comp[0] == (w == 0 ? F.psi0 : F.psi1)) li = (int)q;
-                s->hface_layer[w].push_back(li);
-            }
-            s->hrw2.push_back(rw);
-        }
+        if ((rc = second_faces(s, s->hfaces, s->hcur, s->hpsi2, s->hface_layer, &s->hrw2))) return rc;
     }
     s->d_status = s->dalloc<unsigned>(1, rc);
     if (rc) return rc;
