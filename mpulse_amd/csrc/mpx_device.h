@@ -359,10 +359,6 @@ __device__ __forceinline__ int cpml_side(const CpmlDim &D, int x)
 {
     return x >= D.lo[0] && x <= D.hi[0] ? 0 : (x >= D.lo[1] && x <= D.hi[1] ? 1 : -1);
 }
-__device__ __forceinline__ int cpml_index(const CpmlDim &D, int side, int i, int j, int k)
-{
-    return i * D.s0 + j * D.s1 + k + (side == 0 ? D.off[0] : D.off[1]);
-}
 // the two auxiliaries of a cell as stored
 template <typename T, bool RES>
 struct Aux {
@@ -370,7 +366,7 @@ struct Aux {
     unsigned w;
 };
 template <typename T, bool RES>
-__device__ __forceinline__ Aux<T, RES> cpml_load(const CpmlDim &D, int l)
+__device__ __forceinline__ Aux<T, RES> cpml_load(const CpmlDim &D, unsigned l)
 {
     // ordinary loads: a face row covers only part of a cache line (z faces: 16 cells), and the
     // rest of the line is read by the neighbouring row
@@ -404,7 +400,7 @@ __device__ __forceinline__ void cpml_next(double idxn, double bq, double cq, con
 }
 // the same, the new auxiliaries stored at index l with `store`
 template <typename T, bool HSIDE, bool RES>
-__device__ __forceinline__ void cpml_update(const CpmlDim &D, double bq, double cq, int l, const Aux<T, RES> &x, double d1,
+__device__ __forceinline__ void cpml_update(const CpmlDim &D, double bq, double cq, unsigned l, const Aux<T, RES> &x, double d1,
                                             double d0, bool store, double &v0, double &v1)
 {
     T h0, h1;
@@ -432,7 +428,7 @@ __device__ __forceinline__ void cpml_request(const CpmlDim D[3], int i, int j, i
         // a wave with no cell in these layers skips them; in the others every lane loads, so that no
         // value is merged and waited for here (lanes outside take the block's first element)
         if (__ballot(s.side[d] >= 0))
-            s.x[d] = cpml_load<T, RES>(D[d], s.side[d] >= 0 ? cpml_index(D[d], s.side[d], i, j, k) : 0);
+            s.x[d] = cpml_load<T, RES>(D[d], s.side[d] >= 0 ? cpml_index(D[d], s.side[d], i, j, k) : 0u);
     }
 }
 // The current totals gain the cell's auxiliaries in the reference's list order: faces N,S (y),
@@ -455,7 +451,7 @@ __device__ __forceinline__ void cpml_add(const CpmlDim D[3], int i, int j, int k
             J[c0] += v0;
             J[c1] += v1;
             if (D[d].two && s.side[d] == 0 && at[d] >= D[d].lo[1] && at[d] <= D[d].hi[1]) {
-                const int l = cpml_index(D[d], 1, i, j, k);
+                const unsigned l = cpml_index(D[d], 1, i, j, k);
                 line = D[d].bc + (2 * D[d].len + at[d]);
                 cpml_update<T, HSIDE, RES>(D[d], gld(line), gld(line + D[d].len), l, cpml_load<T, RES>(D[d], l), df[d][1],
                                            df[d][0], store, v0, v1);

@@ -400,15 +400,15 @@ struct MarchFaces {
         const CpmlDim &C = D[d];
         const long long row = (long long)p * C.s0 + (long long)j * C.s1;
         if (d == 2) {
-            const int low = min(C.off[0], C.off[1]);
+            const long long low = min(C.at0[0], C.at0[1]);
             bytes = anyz ? BUF_OUT : 0u;
-            o = live && zs >= 0 ? (unsigned)(k + (zs == 0 ? C.off[0] : C.off[1]) - low) * (unsigned)sizeof(T) : BUF_OUT;
+            o = live && zs >= 0 ? (unsigned)(k + (zs == 0 ? C.at0[0] : C.at0[1]) - low) * (unsigned)sizeof(T) : BUF_OUT;
             return row + low;
         }
         const int side = side_of(d, p);
         bytes = side >= 0 ? BUF_OUT : 0u;
         o = live ? (unsigned)k * (unsigned)sizeof(T) : BUF_OUT;
-        return row + (side == 0 ? C.off[0] : C.off[1]);
+        return row + (side == 0 ? C.at0[0] : C.at0[1]);
     }
     // MODE: 1 the layers along z alone, 2 all three
     template <int MODE, typename T, bool RES>
@@ -451,7 +451,7 @@ struct MarchFaces {
                 // layers that overlap (a box shorter than two of them): the low face too, loaded on the spot
                 if (MODE == 2 && C.two && side == 0 && coord >= C.lo[1] && coord <= C.hi[1]) {
                     const double *line = C.bc + (2 * C.len + coord);
-                    const int l = cpml_index(C, 1, p, j, k);
+                    const unsigned l = cpml_index(C, 1, p, j, k);
                     cpml_update<T, HSIDE, RES>(C, gld(line), gld(line + C.len), l, cpml_load<T, RES>(C, l), df[d][1],
                                                df[d][0], STORE && live, v0, v1);
                     J[(d + 1) % 3] += v0;
@@ -629,7 +629,7 @@ __device__ __forceinline__ void march_tile(const PassArgs<T> &a, int tz, int ty,
                 const int xs = CPML ? cpml_side(a.hcd[0], p) : -1, jl = col ? jc : j;
                 MarchAux<T, RES> ca;
                 if (xs >= 0) ca.x[0] = cpml_load<T, RES>(a.hcd[0], cpml_index(a.hcd[0], xs, p, jl, kc));
-                if (anycy) ca.x[1] = cpml_load<T, RES>(a.hcd[1], cys >= 0 ? cpml_index(a.hcd[1], cys, p, jl, kc) : 0);
+                if (anycy) ca.x[1] = cpml_load<T, RES>(a.hcd[1], cys >= 0 ? cpml_index(a.hcd[1], cys, p, jl, kc) : 0u);
                 if (czs >= 0) ca.x[2] = cpml_load<T, RES>(a.hcd[2], cpml_index(a.hcd[2], czs, p, jl, kc));
                 const C3 e = cell_of(ce0), z = cell_of(cez), u = cell_of(ceu), n = cell_of(cen);
                 const double d[6] = {(double)z.y - e.y, (double)z.x - e.x, (double)u.z - e.z, (double)u.x - e.x,
@@ -646,7 +646,7 @@ __device__ __forceinline__ void march_tile(const PassArgs<T> &a, int tz, int ty,
                             const CpmlDim &C = a.hcd[d];
                             if (C.two && coord <= C.hi[0] && coord >= C.lo[0] && coord >= C.lo[1] && coord <= C.hi[1]) {
                                 const double *line = C.bc + (2 * C.len + coord);
-                                const int l = cpml_index(C, 1, p, jl, kc);
+                                const unsigned l = cpml_index(C, 1, p, jl, kc);
                                 cpml_update<T, true, RES>(C, gld(line), gld(line + C.len), l, cpml_load<T, RES>(C, l),
                                                           df[d][1], df[d][0], st, v0, v1);
                                 M[(d + 1) % 3] += v0;

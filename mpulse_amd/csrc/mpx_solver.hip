@@ -1340,11 +1340,8 @@ static mpx::CpmlDim cpml_dim(const mpx_solver *s, bool hside, int d, bool other)
     for (int q = 0; q < 2; ++q) {
         if (f[q] < 0) continue;
         const CpmlFace &F = faces[f[q]];
-        D.lo[q] = F.lo[d];
-        D.hi[q] = F.hi[d];
         // both faces' auxiliaries lie in one block per array (face_block)
-        const long long to = ((const char *)F.psi0 - (const char *)A.psi0) / (long long)s->esz;
-        D.off[q] = (int)(to - ((long long)F.lo[0] * D.s0 + (long long)F.lo[1] * D.s1 + F.lo[2]));
+        mpx::set_face(D, q, F, ((const char *)F.psi0 - (const char *)A.psi0) / (long long)s->esz);
     }
     D.two = f[0] >= 0 && f[1] >= 0 && D.lo[0] <= D.hi[1] && D.lo[1] <= D.hi[0];
     return D;
@@ -1857,7 +1854,7 @@ static bool march_fits(const mpx_solver *s)
 {
     for (int h = 0; h < 2; ++h) {
         const mpx::CpmlDim D = cpml_dim(s, h, 2, false);
-        const long long apart = (long long)D.off[0] - D.off[1];
+        const long long apart = D.at0[0] - D.at0[1];
         if (((apart < 0 ? -apart : apart) + s->g.n[2] + 2) * (long long)s->esz >= (1LL << 31)) return false;
     }
     return true;

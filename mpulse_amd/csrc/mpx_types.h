@@ -108,8 +108,10 @@ struct CpmlFace {
 struct CpmlDim {
     int lo[2], hi[2];     // range of the normal coordinate: [0] high side, [1] low side (lo > hi: none)
     int two;              // the ranges overlap: a cell may lie in both (high side first)
-    int s0, s1, off[2];   // index of cell (i, j, k): i s0 + j s1 + k + off[side]
     int len;              // n + 2: length of a coefficient line
+    int s0, s1;           // index of cell (i, j, k): i s0 + j s1 + k + off[side]
+    unsigned off[2];      // modulo 2^32 (cpml_index)
+    long long at0[2];     // off itself
     void *p0, *p1;        // auxiliaries psi0, psi1 (CpmlFace)
     unsigned *rw;         // residual words (float32 + residual storage), else null
     const void *o0, *o1;  // the auxiliaries of the step before (p0, p1 where updated in place)
@@ -117,6 +119,22 @@ struct CpmlDim {
     const double *bc;     // lines of b and c: bc[(2 side + (0 b, 1 c)) len + coordinate]
     double idxn;          // 1 / spacing
 };
+
+// Face F (q 0: high side, 1: low side), whose auxiliaries begin `to` elements into the block
+inline void set_face(CpmlDim &D, int q, const CpmlFace &F, long long to)
+{
+    D.lo[q] = F.lo[F.dim];
+    D.hi[q] = F.hi[F.dim];
+    D.at0[q] = to - ((long long)F.lo[0] * D.s0 + (long long)F.lo[1] * D.s1 + F.lo[2]);
+    D.off[q] = (unsigned)D.at0[q];
+}
+// Index of a cell of the layer on `side`.  Modulo 2^32 and without sign: a face has fewer than 2^31
+// cells (a grid has), the block of both up to twice as many.
+__host__ __device__ __forceinline__ unsigned cpml_index(const CpmlDim &D, int side, int i, int j, int k)
+{
+    return (unsigned)i * (unsigned)D.s0 + (unsigned)j * (unsigned)D.s1 + (unsigned)k +
+           (side == 0 ? D.off[0] : D.off[1]);
+}
 
 // One incident-source current sheet: a z plane kp of the down face, three float64
 // component planes of (nx+2) x (ny+2), index i*(ny+2)+j.

@@ -50,3 +50,51 @@ int main()
 
 def test_accumulator_address_of_a_wave(tmp_path):
     assert compile_and_run(tmp_path, PSI) == "ok\n"
+
+
+LAYERS = """
+// the first and last cells of both faces of one dimension, by 64-bit arithmetic and by cpml_index
+static int faces(int dim, const int n[3], int d)
+{
+    CpmlFace F[2]{};
+    CpmlDim D{};
+    for (int q = 0; q < 2; ++q) {  // 0: high side, 1: low
+        F[q].dim = dim;
+        for (int a = 0; a < 3; ++a) F[q].hi[a] = n[a] + 1;
+        F[q].lo[dim] = q ? 1 : n[dim] + 1 - d;
+        F[q].hi[dim] = F[q].lo[dim] + d - 1;
+        F[q].n1 = F[q].hi[1] - F[q].lo[1] + 1;
+        F[q].n2 = F[q].hi[2] - F[q].lo[2] + 1;
+    }
+    const long long cnt = (long long)(F[0].hi[0] - F[0].lo[0] + 1) * F[0].n1 * F[0].n2, block = (cnt + 63) / 64 * 64;
+    if (cnt >= 1LL << 31) return 0;
+    D.s0 = F[0].n1 * F[0].n2;
+    D.s1 = F[0].n2;
+    for (int q = 0; q < 2; ++q) set_face(D, q, F[q], q * block);
+    for (int q = 0; q < 2; ++q)
+        for (int corner = 0; corner < 8; ++corner) {
+            int at[3];
+            for (int a = 0; a < 3; ++a) at[a] = corner >> a & 1 ? F[q].hi[a] : F[q].lo[a];
+            const long long want = q * block + ((long long)(at[0] - F[q].lo[0]) * F[q].n1 + at[1] - F[q].lo[1]) * F[q].n2 +
+                                   at[2] - F[q].lo[2];
+            if ((long long)cpml_index(D, q, at[0], at[1], at[2]) != want) return 0;
+        }
+    return 1;
+}
+int main()
+{
+    const int grids[][4] = {{24, 20, 28, 6}, {8, 8, 8, 8}, {512, 512, 512, 16}, {13, 11600, 11500, 8}, {13, 11500, 11600, 9},
+                            {11600, 13, 11000, 8}, {11600, 11000, 13, 8}, {1, 30000, 20000, 1}, {1288, 1288, 1288, 700}};
+    for (auto &g : grids)
+        for (int dim = 0; dim < 3; ++dim)
+            if (g[dim] >= g[3] && !faces(dim, g, g[3])) {
+                std::printf("%d x %d x %d dim %d layers %d\\n", g[0], g[1], g[2], dim, g[3]);
+                return 0;
+            }
+    std::printf("ok\\n");
+}
+"""
+
+
+def test_layer_index_up_to_the_largest_faces(tmp_path):
+    assert compile_and_run(tmp_path, LAYERS) == "ok\n"
