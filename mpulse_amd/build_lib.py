@@ -9,7 +9,8 @@ LIB = os.path.join(HERE, "libmpulse_hip.so")
 # (source, storage form): the template-heavy units are compiled once per form, in parallel
 SOURCES = [("mpx_pass.hip", 0), ("mpx_pass.hip", 1), ("mpx_pass.hip", 2), ("mpx_fused.hip", 0), ("mpx_fused.hip", 1),
            ("mpx_sweep.hip", 0), ("mpx_sweep.hip", 1), ("mpx_kernels.hip", None), ("mpx_sheet.hip", None),
-           ("mpx_adjoint.hip", None), ("mpx_gauss.hip", None), ("mpx_solver.hip", None)]
+           ("mpx_adjoint.hip", None), ("mpx_gauss.hip", None), ("mpx_memory.hip", None),
+           ("mpx_solver.hip", None)]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
     "--offload-arch=gfx950",

@@ -14,6 +14,7 @@
 #include <cmath>
 
 #include "mpx_gauss.h"
+#include "mpx_memory.h"
 
 namespace mpx {
 
@@ -117,7 +118,9 @@ unsigned blocks_for(size_t n) { return (unsigned)((n + 255) / 256); }
 bool plan1d(hipfftHandle *p, int n, int batch, hipStream_t s)
 {
     int len = n;
-    if (hipfftPlanMany(p, 1, &len, nullptr, 1, n, nullptr, 1, n, HIPFFT_Z2Z, batch) != HIPFFT_SUCCESS) return false;
+    auto plan = [&] { return hipfftPlanMany(p, 1, &len, nullptr, 1, n, nullptr, 1, n, HIPFFT_Z2Z, batch) == HIPFFT_SUCCESS; };
+    // a plan allocates its own work area: where that fails, once more without the kept blocks
+    if (!plan() && !(spare_drop() && plan())) return false;
     return hipfftSetStream(*p, s) == HIPFFT_SUCCESS;
 }
 
@@ -163,9 +166,9 @@ int GaussInjectDev::setup(const mpx_factory &f, int isH_, int nx, int ny, double
     const size_t row = (size_t)SizeY * SizeT * sizeof(double2);
     slab = (int)std::max<size_t>(1, std::min<size_t>((size_t)SizeX, ((size_t)1 << 30) / row));
     const size_t nF = (size_t)Nt * SizeX * SizeY;
-    if (hipMalloc(&F1, nF * sizeof(double)) != hipSuccess || hipMalloc(&F2, nF * sizeof(double)) != hipSuccess ||
-        hipMalloc(&S, (size_t)slab * row) != hipSuccess || hipMalloc(&P, nF * sizeof(double2)) != hipSuccess ||
-        hipMalloc(&Q, nF * sizeof(double2)) != hipSuccess)
+    if (dev_malloc(&F1, nF * sizeof(double)) != hipSuccess || dev_malloc(&F2, nF * sizeof(double)) != hipSuccess ||
+        dev_malloc(&S, (size_t)slab * row) != hipSuccess || dev_malloc(&P, nF * sizeof(double2)) != hipSuccess ||
+        dev_malloc(&Q, nF * sizeof(double2)) != hipSuccess)
         return 1;
     if (hipMemsetAsync(F1, 0, nF * sizeof(double), s) != hipSuccess ||
         hipMemsetAsync(F2, 0, nF * sizeof(double), s) != hipSuccess)

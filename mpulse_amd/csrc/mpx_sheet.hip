@@ -22,6 +22,7 @@
 #include <hip/hip_runtime.h>
 
 #include "mpx_launch.h"
+#include "mpx_memory.h"
 
 namespace mpx {
 
@@ -299,7 +300,7 @@ __global__ void k_pulse_norm(PulseParams P, FaddeevaTables ft, double *out)
 double pulse_norm_device(const PulseParams &P, const FaddeevaTables &ft, hipStream_t s)
 {
     double *d = nullptr, h = 0;
-    if (hipMalloc(&d, sizeof(double)) != hipSuccess) return NAN;
+    if (dev_malloc(&d, sizeof(double)) != hipSuccess) return NAN;
     hipLaunchKernelGGL(k_pulse_norm, dim3(1), dim3(64), 0, s, P, ft, d);
     if (hipMemcpyAsync(&h, d, sizeof(double), hipMemcpyDeviceToHost, s) != hipSuccess) h = NAN;
     if (hipStreamSynchronize(s) != hipSuccess) h = NAN;

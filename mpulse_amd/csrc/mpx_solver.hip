@@ -17,8 +17,10 @@
 #include "../../include/mpulse_hip.h"
 #include "mpx_gauss.h"
 #include "mpx_launch.h"
+#include "mpx_memory.h"
 
 using mpx::CpmlFace;
+using mpx::dev_malloc;
 using mpx::GridDims;
 using mpx::StepArgs;
 
@@ -104,90 +106,6 @@ enum {
     K_FUSED_E, K_FUSED_B, K_SIMPLE_E, K_SIMPLE_B, K_PROBE, K_SWEEP, K_PASS, K_NCLASSES
 };
 
-}  // namespace
-
-// ---------------------------------------------------------------------------------------
-// device memory
-// ---------------------------------------------------------------------------------------
-//
-// An adjoint call works in gigabytes that it needs for its own length only.  Allocating and
-// freeing them on every call took 60 (250 separate arrays) to 90 ms (one block: the driver clears
-// what it maps) of the 157 ms of a 128x128x256, 100-step gradient, so one block per GPU is kept
-// between calls, whichever solver they are for.  It holds nothing: a call takes the block out of
-// its slot (a second call at the same time finds the slot empty and allocates), uses it on its own
-// stream and puts it back after waiting for that stream.  Bounded to an eighth of the GPU's
-// memory; freed when an allocation of this library fails (which is then tried again) and when the
-// last solver is destroyed.
-namespace {
-struct Spare {
-    void *p = nullptr;
-    size_t bytes = 0;
-};
-std::mutex g_spare_mu;
-std::vector<Spare> g_spare;  // per device id
-int g_solvers = 0;           // solvers alive
-
-// frees the kept blocks; whether there was one
-bool spare_drop()
-{
-    std::vector<Spare> old;
-    {
-        std::lock_guard<std::mutex> lock(g_spare_mu);
-        old.swap(g_spare);
-    }
-    bool any = false;
-    for (const Spare &b : old)
-        if (b.p) any = hipFree(b.p) == hipSuccess || any;
-    return any;
-}
-
-hipError_t dev_malloc(void **p, size_t bytes)
-{
-    hipError_t e = hipMalloc(p, bytes);
-    if (e == hipErrorOutOfMemory && spare_drop()) {
-        (void)hipGetLastError();
-        e = hipMalloc(p, bytes);
-    }
-    return e;
-}
-
-// a block of at least *bytes (its size returned), the kept one if it is large enough; null on failure
-void *spare_take(int device, size_t *bytes)
-{
-    Spare b;
-    {
-        std::lock_guard<std::mutex> lock(g_spare_mu);
-        if (device < (int)g_spare.size()) std::swap(b, g_spare[device]);
-    }
-    if (b.p && b.bytes >= *bytes) {
-        *bytes = b.bytes;
-        return b.p;
-    }
-    if (b.p) (void)hipFree(b.p);
-    void *p = nullptr;
-    if (dev_malloc(&p, *bytes) != hipSuccess) {
-        (void)hipGetLastError();
-        return nullptr;
-    }
-    return p;
-}
-
-// puts a block back (no kernel uses it any more); the slot's older block, or this one past the
-// bound, is freed
-void spare_give(int device, void *p, size_t bytes)
-{
-    if (!p) return;
-    size_t avail = 0, total = 0;
-    Spare b{p, bytes};
-    if (hipMemGetInfo(&avail, &total) == hipSuccess && bytes <= total / 8) {
-        std::lock_guard<std::mutex> lock(g_spare_mu);
-        if (g_solvers > 0) {
-            if ((int)g_spare.size() <= device) g_spare.resize(device + 1);
-            std::swap(b, g_spare[device]);
-        }
-    }
-    if (b.p) (void)hipFree(b.p);
-}
 }  // namespace
 
 struct mpx_solver {
@@ -285,19 +203,10 @@ struct mpx_solver {
     void *d_pargs[2] = {nullptr, nullptr};
     std::vector<unsigned char> h_pargs[2];
 
-    mpx_solver()
-    {
-        std::lock_guard<std::mutex> lock(g_spare_mu);
-        ++g_solvers;
-    }
+    mpx_solver() { mpx::spare_solvers(1); }
     ~mpx_solver()
     {
-        bool last;
-        {
-            std::lock_guard<std::mutex> lock(g_spare_mu);
-            last = --g_solvers == 0;
-        }
-        if (last) (void)spare_drop();
+        mpx::spare_solvers(-1);
         if (stream) (void)hipStreamSynchronize(stream);
         for (void *p : allocs) (void)hipFree(p);
         for (hipEvent_t e : timer.pool) (void)hipEventDestroy(e);
@@ -3564,7 +3473,7 @@ struct Arena {
     ~Arena()
     {
         if (base) (void)hipStreamSynchronize(stream);
-        spare_give(device, base, bytes);
+        mpx::spare_give(device, base, bytes);
     }
     template <typename T>
     T *get(size_t count)
@@ -3707,7 +3616,7 @@ int mpx_adjoint_grad(mpx_solver *s, const mpx_objective *obj, int nsteps, int K,
     mem.device = s->device;
     mem.stream = st;
     mem.bytes = mem.used;
-    mem.base = (char *)spare_take(s->device, &mem.bytes);
+    mem.base = (char *)mpx::spare_take(s->device, &mem.bytes);
     if (!mem.base) return fail(MPX_ERR_NOMEM, "adjoint allocation of " + std::to_string(mem.used) + " bytes failed");
     carve();
     if (clear) MPX_HIP(hipMemsetAsync(mem.base, 0, clear, st));
