@@ -341,7 +341,8 @@ int  mpx_batch_time_steps(mpx_batch *b, int nsteps, double *ms_per_step);
    update (fused float64 kernels), recomputing the forward E of each segment of
    checkpoint_every steps from a stored checkpoint.  Gradients: dJ/dEps(x) for every interior
    cell (full-storage layout, zero in the ghosts) and dJ/dchi (0 for the linear core).  The
-   solver ends at the final forward state.  Scope: FDTD_PLRC solvers (Kerr or linear core,
+   solver ends at the final forward state.  The call's working memory stays allocated for the next
+   one: see mpx_release_memory.  Scope: FDTD_PLRC solvers (Kerr or linear core,
    with or without Lorentz poles), float64, fused path, periodic boundary (CPML and current
    sheets allowed; no plasma, no gauss_inject).  With dJ_deps and dJ_dchi both NULL only the
    forward objective is computed. */
@@ -351,6 +352,13 @@ typedef struct mpx_objective {
 } mpx_objective;
 int  mpx_adjoint_grad(mpx_solver *s, const mpx_objective *obj, int nsteps, int checkpoint_every, double *J,
                       double *dJ_deps, double *dJ_dchi);
+
+/* Frees the device memory the library keeps between calls: one block per GPU, the working memory of
+   the last mpx_adjoint_grad there, at most an eighth of the GPU's memory.  The next call allocates
+   it again (90 ms for 8 GB).  It goes by itself when an allocation of this library finds the GPU
+   full and when the last solver of the process is destroyed; other allocators in the process see it
+   as used, so call this before they need the space.  May be called at any time, from any thread. */
+int mpx_release_memory(void);
 
 /* The value a field word holds once stored in `precision` (MPX_PREC_*): x itself (float64),
    its float32 rounding, or the float32 word plus residual; what mpx_set_field stores for x.

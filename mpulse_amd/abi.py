@@ -176,6 +176,7 @@ def load():
         "mpx_batch_time_steps": (C.c_int, [P, C.c_int, C.POINTER(C.c_double)]),
         "mpx_adjoint_grad": (C.c_int, [P, C.POINTER(Objective), C.c_int, C.c_int, C.POINTER(C.c_double),
                                        C.POINTER(C.c_double), C.POINTER(C.c_double)]),
+        "mpx_release_memory": (C.c_int, []),
         "mpx_last_error": (C.c_char_p, []),
         "mpx_store_round": (C.c_double, [C.c_double, C.c_int]),
         "mpx_abi_version": (C.c_int, []),
@@ -529,6 +530,12 @@ class Batch:
         ms = C.c_double()
         self._check(self.lib.mpx_batch_time_steps(self.h, nsteps, C.byref(ms)))
         return ms.value
+
+
+def release_memory():
+    """Free the working memory that adjoint_grad leaves allocated for its next call, so that other
+    allocators of the process (torch) can have it."""
+    load().mpx_release_memory()
 
 
 def copy_probe(nbytes, reps=20):

@@ -4,8 +4,8 @@
 // between calls, whichever solver they are for.  It holds nothing: a call takes the block out of
 // its slot (a second call at the same time finds the slot empty and allocates), uses it on its own
 // stream and puts it back after waiting for that stream.  Bounded to an eighth of the GPU's
-// memory; freed with the last solver, and when an allocation of this library (hipFFT's plans
-// included) finds the GPU full, which is then tried again.
+// memory; freed by mpx_release_memory, with the last solver, and when an allocation of this library
+// (hipFFT's plans included) finds the GPU full, which is then tried again.
 #include "mpx_memory.h"
 
 #include <mutex>

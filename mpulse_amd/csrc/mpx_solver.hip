@@ -649,6 +649,12 @@ int mpx_create(const mpx_desc *desc, mpx_solver **out)
     return MPX_OK;
 }
 
+int mpx_release_memory(void)
+{
+    (void)mpx::spare_drop();
+    return MPX_OK;
+}
+
 int mpx_destroy(mpx_solver *s)
 {
     MPX_NOT_IN_BATCH(s);

@@ -1,11 +1,12 @@
 """The block of device memory kept between adjoint calls: its bookkeeping on the CPU (the unit compiled
-against a HIP stand-in with a fixed amount of memory), and on the GPU that it serves
+against a HIP stand-in with a fixed amount of memory), and on the GPU that it is given back, serves
 grids of different sizes one after the other and calls from two threads."""
 import os
 import re
 import shutil
 import subprocess
 import threading
+import time
 
 import numpy as np
 import pytest
@@ -87,7 +88,7 @@ int main()
     n = 700;
     a = spare_take(0, &n);
     spare_give(0, a, n);
-    CHECK(spare_drop() && held() == 0 && !spare_drop());
+    CHECK(spare_drop() && held() == 0 && !spare_drop());  // the release call
     n = 700;
     a = spare_take(0, &n);
     spare_give(0, a, n);
@@ -138,6 +139,25 @@ def gradient(n, nz, seed=3, keep=None):
 
 def same(a, b):
     return a[0] == b[0] and np.array_equal(a[1], b[1]) and a[2] == b[2]
+
+
+@pytest.mark.gpu
+def test_release_gives_the_block_back():
+    torch = pytest.importorskip("torch")
+    print("case: kept adjoint block, release", flush=True)
+    keep = []
+    gradient(24, 24, keep=keep)
+    abi.release_memory()
+    before = torch.cuda.mem_get_info()[0]
+    keep[0].adjoint_grad(20, 1.0, 200, checkpoint_every=100)  # over 100 states of 0.4 MB each
+    kept = before - torch.cuda.mem_get_info()[0]
+    abi.release_memory()
+    assert kept >= 1 << 25
+    end = time.monotonic() + 20  # the driver reports freed memory up to a second late
+    while torch.cuda.mem_get_info()[0] < before and time.monotonic() < end:
+        time.sleep(0.1)
+    assert torch.cuda.mem_get_info()[0] >= before
+    keep[0].close()
 
 
 @pytest.mark.gpu
