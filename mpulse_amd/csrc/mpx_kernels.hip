@@ -17,13 +17,13 @@ namespace mpx {
 // ------------------------------------------------------------------------------------
 
 // CPMLBorderECurrent::stepScheme, src/cpml_border.cpp:398-425
-__global__ __launch_bounds__(256) void k_ref_cpml_E(StepArgs<double> a, int fi)
+__global__ __launch_bounds__(256) void k_ref_cpml_E(StepArgs<double> a, int fi, FaceCells at)
 {
     const CpmlFace &f = a.face[fi];
-    int k = f.lo[2] + blockIdx.x * 64 + threadIdx.x;
-    int j = f.lo[1] + blockIdx.y * 4 + threadIdx.y;
-    int i = f.lo[0] + blockIdx.z;
-    if (k > f.hi[2] || j > f.hi[1]) return;
+    int k = at.lo[2] + blockIdx.x * 64 + threadIdx.x;
+    int j = at.lo[1] + blockIdx.y * 4 + threadIdx.y;
+    int i = at.lo[0] + blockIdx.z;
+    if (k > at.hi[2] || j > at.hi[1]) return;
     int ind[3] = {i, j, k};
     int m[3] = {i, j, k};
     m[f.dim] -= 1;
@@ -38,13 +38,13 @@ __global__ __launch_bounds__(256) void k_ref_cpml_E(StepArgs<double> a, int fi)
 }
 
 // CPMLBorderHCurrent::stepScheme, src/cpml_border.cpp:499-527
-__global__ __launch_bounds__(256) void k_ref_cpml_H(StepArgs<double> a, int fi)
+__global__ __launch_bounds__(256) void k_ref_cpml_H(StepArgs<double> a, int fi, FaceCells at)
 {
     const CpmlFace &f = a.face[fi];
-    int k = f.lo[2] + blockIdx.x * 64 + threadIdx.x;
-    int j = f.lo[1] + blockIdx.y * 4 + threadIdx.y;
-    int i = f.lo[0] + blockIdx.z;
-    if (k > f.hi[2] || j > f.hi[1]) return;
+    int k = at.lo[2] + blockIdx.x * 64 + threadIdx.x;
+    int j = at.lo[1] + blockIdx.y * 4 + threadIdx.y;
+    int i = at.lo[0] + blockIdx.z;
+    if (k > at.hi[2] || j > at.hi[1]) return;
     int ind[3] = {i, j, k};
     int p[3] = {i, j, k};
     p[f.dim] += 1;
@@ -62,11 +62,12 @@ void launch_ref_cpml(const StepArgs<double> &a, int fi, bool isH, hipStream_t s)
 {
     const CpmlFace &f = a.face[fi];
     dim3 blk(64, 4);
-    dim3 grd((f.hi[2] - f.lo[2] + 64) / 64, (f.hi[1] - f.lo[1] + 4) / 4, f.hi[0] - f.lo[0] + 1);
+    const FaceCells c = face_cells(f, a.g.n, isH);
+    dim3 grd((c.hi[2] - c.lo[2] + 64) / 64, (c.hi[1] - c.lo[1] + 4) / 4, c.hi[0] - c.lo[0] + 1);
     if (isH)
-        hipLaunchKernelGGL(k_ref_cpml_H, grd, blk, 0, s, a, fi);
+        hipLaunchKernelGGL(k_ref_cpml_H, grd, blk, 0, s, a, fi, c);
     else
-        hipLaunchKernelGGL(k_ref_cpml_E, grd, blk, 0, s, a, fi);
+        hipLaunchKernelGGL(k_ref_cpml_E, grd, blk, 0, s, a, fi, c);
 }
 
 // FDTD_PLRCSolver::sumCurrents / sumMagCurrents, src/fdtd_plrc.t:342-409: totals := 0, then

@@ -102,6 +102,22 @@ struct CpmlFace {
     }
 };
 
+// The cells of a face whose stencil lies in the storage box 0 .. n + 1: the layer itself unless it is
+// thicker than the box.  H differences reach one cell up, E differences one cell down.
+struct FaceCells {
+    int lo[3], hi[3];
+};
+inline FaceCells face_cells(const CpmlFace &f, const int n[3], bool isH)
+{
+    FaceCells c;
+    for (int d = 0; d < 3; ++d) {
+        const int first = d == f.dim && !isH ? 1 : 0, last = d == f.dim && isH ? n[d] : n[d] + 1;
+        c.lo[d] = f.lo[d] > first ? f.lo[d] : first;
+        c.hi[d] = f.hi[d] < last ? f.hi[d] : last;
+    }
+    return c;
+}
+
 // The two CPML faces of one dimension on the E or on the H side, as the fused and pass kernels
 // read them: the auxiliaries of both faces lie in one block (high side first), so that a cell
 // finds its own with one base address and a 32-bit index whichever face holds it.

@@ -98,3 +98,44 @@ int main()
 
 def test_layer_index_up_to_the_largest_faces(tmp_path):
     assert compile_and_run(tmp_path, LAYERS) == "ok\n"
+
+
+STENCIL = """
+int main()
+{
+    for (int n = 1; n <= 9; ++n)
+        for (int d = 1; d <= 12; ++d)
+            for (int dim = 0; dim < 3; ++dim)
+                for (int isH = 0; isH < 2; ++isH)
+                    for (int high = 0; high < 2; ++high) {
+                        // the layer as border_extent places it: distance 1 from either end, the low H face 0
+                        int N[3] = {5, 5, 5};
+                        N[dim] = n;
+                        CpmlFace f{};
+                        f.dim = dim;
+                        for (int a = 0; a < 3; ++a) f.hi[a] = N[a] + 1;
+                        f.lo[dim] = high ? n + 1 - d : (isH ? 0 : 1);
+                        f.hi[dim] = f.lo[dim] + d - 1;
+                        const FaceCells c = face_cells(f, N, isH);
+                        const int below = isH ? 0 : 1, above = isH ? 1 : 0;
+                        bool good = c.lo[dim] <= c.hi[dim] && c.lo[dim] >= f.lo[dim] && c.hi[dim] <= f.hi[dim];
+                        for (int a = 0; a < 3; ++a) {
+                            good = good && c.lo[a] - (a == dim ? below : 0) >= 0 && c.hi[a] + (a == dim ? above : 0) <= N[a] + 1;
+                            if (d <= n) good = good && c.lo[a] == f.lo[a] && c.hi[a] == f.hi[a];
+                            // every cell the updates use (1 .. n; H from 0) that lies in the layer is kept
+                            const int first = f.lo[a] > (isH ? 0 : 1) ? f.lo[a] : (isH ? 0 : 1);
+                            const int last = f.hi[a] < N[a] ? f.hi[a] : N[a];
+                            good = good && c.lo[a] <= first && c.hi[a] >= last;
+                        }
+                        if (!good) {
+                            std::printf("n %d d %d dim %d H %d high %d\\n", n, d, dim, isH, high);
+                            return 0;
+                        }
+                    }
+    std::printf("ok\\n");
+}
+"""
+
+
+def test_layer_thicker_than_the_box_keeps_its_stencil_inside(tmp_path):
+    assert compile_and_run(tmp_path, STENCIL) == "ok\n"
