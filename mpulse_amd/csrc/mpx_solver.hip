@@ -1778,23 +1778,54 @@ static bool march_fits(const mpx_solver *s)
 // Whether a pending B half and the next E half run as one pass (pass_launch_t) or as the two fused
 // kernels, which give the same bits.  A pass launches one kernel less and moves fewer bytes (E and B
 // cross memory once); the fused kernels hold more waves a SIMD and have no halo to recompute.
-// Measured (us a step, pass / two halves, one pole, layers of 4 to 16 cells):
-//   24^3 23.1 / 26.0 (float64), 64^3 34.1 / 36.9 (with residuals 37.4 / 34.2, 56^3 30.3 / 32.0): the
-//   launch decides; 96^3 97 / 83, 256^3 932 / 899, with residuals 256^3 829 / 726; float64 from
-//   about 2^25 cells on: 320^3 1598 / 1696, 512^3 6138 / 6480; float32 with and without residuals
-//   draws level there (512^3 5061 / 5059 with).
-// Without layers the pass has no auxiliaries to wait for: float64 24^3 18.7 / 24.1, 128^3 98 / 107,
-// 256^3 698 / 734; float32 128^3 78 / 84, 256^3 520 / 488.
+// Measured, us a step, pass / two halves, no source:
+// - With layers along x or y the pass waits for auxiliaries at every plane: one pole 24^3 16.3 / 12.0 (float64), 64^3
+//   28.1 / 21.1, 128^3 108 / 106; float32 64^3 22.4 / 15.6, 256^3 559 / 534; with residuals 64^3
+//   27.4 / 19.2, 256^3 655 / 640.  Float64 alone gains from the pass: without poles from about
+//   6 million cells (176^3 206 / 193, 192^3 221 / 239, 200^3 296 / 339, 300x310x290 849 / 893); with
+//   poles where every z tile is whole -- lanes past a row's end cost the pass more -- and the grid large
+//   (one pole 256^3 770 / 806, 256x256x250 886 / 820, 320^3 1442 / 1531; two 256^3 1107 / 1104, 320^3
+//   2107 / 2137).
+// - With layers along z alone the pass waits less: without poles float64 always (48^3 11.7 / 14.2, 256^3
+//   402 / 543), float32 from 2^21 cells (60x75x260 38.6 / 33.7, 128^3 47.4 / 49.5; residuals 46.8 / 40.4,
+//   58.7 / 59.7); with poles whole z tiles beyond 2^18 cells (one, float64 64^3 21.9 / 19.0, 128^3 91 / 103,
+//   160^3 213 / 194; float32 128^3 71 / 75, 160^3 158 / 138; residuals 81 / 86, 182 / 159).
+// - Without layers the launch decides up to 2^22 cells (24^3 9.1 / 9.2, 64^3 17.7 / 18.2, 128^3 83 / 90).
+//   Beyond: float64 the pass (256^3 643 / 696); no poles the pass (256^3 float32 195 / 214, with
+//   residuals 259 / 292); with poles residuals where z tiles are whole (one 320^3 1053 / 1131, two 1693 /
+//   1739; one 200^3 347 / 313), three on large grids alone (256^3 1173 / 1124, 448^3 6277 / 6488), float32
+//   where the grid is large too (one 256^3 482 / 463, 320^3 936 / 950; two 320^3 1583 / 1525, 448^3
+//   4177 / 4359; three 512^3 8750 / 8690).
+// - Plasma without layers: 64^3 16.5 / 18.7; beyond 2^18 cells float64 without poles (160^3 136 / 148) or
+//   with whole z tiles (256^3 745 / 795, 200^3 467 / 424), residuals with whole z tiles (256^3 636 / 660,
+//   200^3 425 / 362), float32 with those on large grids (256^3 580 / 574, 320^3 1099 / 1134).  With layers
+//   along z float64 with whole z tiles (320^3 1583 / 1640; 160^3 176 / 166, residuals 128^3 104 / 95).
+//   With layers along x or y the halves (float64 24^3 15.3 / 12.3, 256^3 886 / 892).
 // A pass_kernel, march_seg or march_rows set by the user asks for the pass.
 static bool pass_in_one(const mpx_solver *s)
 {
     if (s->pass_kernel == 1 && !march_fits(s)) return false;
     if (s->pass_set) return true;
     const double cells = (double)s->g.n[0] * s->g.n[1] * s->g.n[2];
-    const bool layers = !s->efaces.empty() || !s->hfaces.empty();
-    if (cells <= (s->res ? 3 << 16 : 1 << 18)) return true;
-    if (layers || s->plasma || s->pcur) return s->esz == 8 && !s->plasma && !s->pcur && cells >= (1 << 25);
-    return s->esz == 8 || cells <= (1 << 22);
+    bool across = false, along = false;  // layers along x or y, along z
+    for (const std::vector<CpmlFace> *faces : {&s->efaces, &s->hfaces})
+        for (const CpmlFace &F : *faces) (F.dim == 2 ? along : across) = true;
+    const bool plasma = s->plasma || s->pcur, whole = s->g.n[2] % 64 == 0, f64 = s->esz == 8;
+    if (across) {
+        if (!f64 || plasma) return false;
+        return s->np == 0 ? cells >= (3 << 21) : whole && cells >= (s->np == 1 ? 1 << 24 : 3 << 23);
+    }
+    if (plasma) {
+        if (along) return f64 && whole && cells > (1 << 18);
+        return cells <= (1 << 18) || (f64 && s->np == 0) || (whole && (f64 || s->res || cells >= (3 << 23)));
+    }
+    if (along) {
+        if (s->np == 0) return f64 || cells >= (1 << 21);
+        return whole && cells > (1 << 18) && (f64 || s->res || s->np == 1);
+    }
+    if (f64 || s->np == 0 || cells <= (1 << 22)) return true;
+    if (s->res) return whole && (s->np < 3 || cells >= (3 << 24));
+    return whole && s->np < 3 && cells >= (s->np == 1 ? 3 << 23 : 3 << 24);
 }
 
 // One step on the pass path.  Settled state at time t (E^t, B^t): the E half of step t.
