@@ -431,6 +431,25 @@ __device__ __forceinline__ void cpml_request(const CpmlDim D[3], int i, int j, i
             s.x[d] = cpml_load<T, RES>(D[d], s.side[d] >= 0 ? cpml_index(D[d], s.side[d], i, j, k) : 0u);
     }
 }
+// The current totals gain the auxiliaries of a cell of dimension d's layers (D, coordinate `at`); x: those
+// of the layer on `side`.  d0, d1: the differences that feed psi0 and psi1; Jp, Jq: the currents these feed.
+template <typename T, bool HSIDE, bool RES>
+__device__ __forceinline__ void cpml_dim_add(const CpmlDim &D, int at, int side, int i, int j, int k, const Aux<T, RES> &x,
+                                             double d1, double d0, bool store, double &Jp, double &Jq)
+{
+    double v0, v1;
+    const double *line = D.bc + (2 * side * D.len + at);
+    cpml_update<T, HSIDE, RES>(D, gld(line), gld(line + D.len), cpml_index(D, side, i, j, k), x, d1, d0, store, v0, v1);
+    Jp += v0;
+    Jq += v1;
+    if (D.two && side == 0 && at >= D.lo[1] && at <= D.hi[1]) {
+        const unsigned l = cpml_index(D, 1, i, j, k);
+        line = D.bc + (2 * D.len + at);
+        cpml_update<T, HSIDE, RES>(D, gld(line), gld(line + D.len), l, cpml_load<T, RES>(D, l), d1, d0, store, v0, v1);
+        Jp += v0;
+        Jq += v1;
+    }
+}
 // The current totals gain the cell's auxiliaries in the reference's list order: faces N,S (y),
 // E,W (x), U,D (z), the high face first.  df[d][0], df[d][1]: the differences along d of the field
 // components d + 1 and d + 2, which feed psi1 and psi0; those feed the currents d + 2 and d + 1.
@@ -442,23 +461,24 @@ __device__ __forceinline__ void cpml_add(const CpmlDim D[3], int i, int j, int k
 #pragma unroll
     for (int u = 0; u < 3; ++u) {
         constexpr int order[3] = {1, 0, 2};
-        const int d = order[u], c0 = (d + 1) % 3, c1 = (d + 2) % 3;
-        if (s.side[d] >= 0) {
-            double v0, v1;
-            const double *line = D[d].bc + (2 * s.side[d] * D[d].len + at[d]);
-            cpml_update<T, HSIDE, RES>(D[d], gld(line), gld(line + D[d].len), cpml_index(D[d], s.side[d], i, j, k), s.x[d],
-                                       df[d][1], df[d][0], store, v0, v1);
-            J[c0] += v0;
-            J[c1] += v1;
-            if (D[d].two && s.side[d] == 0 && at[d] >= D[d].lo[1] && at[d] <= D[d].hi[1]) {
-                const unsigned l = cpml_index(D[d], 1, i, j, k);
-                line = D[d].bc + (2 * D[d].len + at[d]);
-                cpml_update<T, HSIDE, RES>(D[d], gld(line), gld(line + D[d].len), l, cpml_load<T, RES>(D[d], l), df[d][1],
-                                           df[d][0], store, v0, v1);
-                J[c0] += v0;
-                J[c1] += v1;
-            }
-        }
+        const int d = order[u];
+        if (s.side[d] >= 0)
+            cpml_dim_add<T, HSIDE, RES>(D[d], at[d], s.side[d], i, j, k, s.x[d], df[d][1], df[d][0], store, J[(d + 1) % 3],
+                                        J[(d + 2) % 3]);
+    }
+}
+// the same, each dimension's auxiliaries loaded where they are used
+template <typename T, bool HSIDE, bool RES>
+__device__ __forceinline__ void cpml_each(const CpmlDim D[3], int i, int j, int k, const double df[3][2], double J[3])
+{
+    const int at[3] = {i, j, k};
+#pragma unroll
+    for (int u = 0; u < 3; ++u) {
+        constexpr int order[3] = {1, 0, 2};
+        const int d = order[u], side = cpml_side(D[d], at[d]);
+        if (side >= 0)
+            cpml_dim_add<T, HSIDE, RES>(D[d], at[d], side, i, j, k, cpml_load<T, RES>(D[d], cpml_index(D[d], side, i, j, k)),
+                                        df[d][1], df[d][0], true, J[(d + 1) % 3], J[(d + 2) % 3]);
     }
 }
 

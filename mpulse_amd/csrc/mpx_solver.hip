@@ -726,12 +726,6 @@ static int build(mpx_solver *s, const mpx_desc *desc)
         return fail(MPX_ERR_INVALID, "unknown precision " + std::to_string(s->prec));
     s->res = s->prec == MPX_PREC_FP32_RES;
     s->esz = (s->prec == MPX_PREC_FP64) ? 8 : 4;
-    // Planes per thread of the fused B kernel: a second plane saves a read of E but holds its words
-    // in registers and halves the waves.  One is faster in both float32 forms (us, one against two
-    // planes with CPML: 24^3 7.2 / 9.1, 256^3 188 / 205, 512^3 1059 / 1118; with residuals 1348 /
-    // 1573) and for small float64 grids (24^3 7.3 / 9.1, 64^3 11.3 / 12.2); from about 2^21 cells
-    // float64 gains a little from two (131x158x177 74.5 / 73.2, 512^3 2014 / 1969).
-    s->march_b = s->esz == 8 && (double)desc->nx * desc->ny * desc->nz >= (1 << 21) ? 2 : 1;
     s->delta[0] = desc->dx;
     s->delta[1] = desc->dy;
     s->delta[2] = desc->dz;
@@ -1192,6 +1186,17 @@ static int build(mpx_solver *s, const mpx_desc *desc)
             if (rc) return rc;
         }
         if ((rc = second_faces(s, s->hfaces, s->hcur, s->hpsi2, s->hface_layer, &s->hrw2))) return rc;
+    }
+    // Planes per thread of the fused B kernel: a second plane saves a read of E but holds its words in
+    // registers and halves the waves.  Measured, us, one / two planes: float64 with layers 24^3 6.8 / 8.5, 64^3
+    // 10.2 / 10.8, 80^3 19.1 / 20.0, 96^3 25.4 / 24.1, 128^3 42.2 / 41.4, 512^3 2014 / 1969, without layers
+    // 24^3 6.2 / 6.3, 58^3 8.6 / 8.3, 96^3 20.0 / 19.0, 256^3 232 / 220; float32 with layers 24^3 6.8 / 8.7,
+    // 96^3 15.2 / 15.7, 112^3 20.4 / 19.4, 200^3 95 / 84, without 64^3 6.5 / 6.7, 200^3 71 / 64; with
+    // residuals and layers 24^3 7.1 / 9.2, 256^3 200 / 235, without 128^3 23.3 / 25.0, 256^3 153 / 149.
+    {
+        const double cells = (double)g.n[0] * g.n[1] * g.n[2];
+        const bool two = s->res ? false : (s->esz == 8 ? s->hfaces.empty() || cells >= (3 << 18) : cells >= (5 << 18));
+        s->march_b = two ? 2 : 1;
     }
     s->d_status = s->dalloc<unsigned>(1, rc);
     if (rc) return rc;
