@@ -150,12 +150,15 @@ struct PsiCell {
 // adds a latency to every wave.  Every word of a cell -- its own, the three lower neighbours',
 // the accumulators', the CPML auxiliaries' -- is therefore requested unconditionally before the
 // first is used.  The z - 1 neighbour is in the previous lane (DPP) except for the first lane of
-// a wave and the first cell of a row; that word too is loaded by all lanes (at their own cell's
-// address where it is not needed), since under a branch its decoding waited for it at once.
-// Measured against that form (face by face CPML, per-lane 64-bit addresses, tile divisions in
-// the kernel), us for E and B with a 16-cell CPML and one pole: 512^3 float32 + residual 3627 +
-// 1707 -> 3166 + 1345, float32 3184 + 1054 -> 2832 + 1059, float64 4204 + 2187 -> 3764 + 1969;
-// 256^3 float32 + residual 513 + 268 -> 464 + 236; 64^3 float64 14.8 + 14.2 -> 14.4 + 11.3.
+// a wave and the first cell of a row.  With residuals that word too is loaded by all lanes (at
+// their own cell's address where it is not needed), since under a branch its decoding waited for it
+// at once; a plain word has nothing to wait for there, and the lanes that need it load it (all / those,
+// float64: 64^3 with one pole and plasma 12.6 / 11.6, 131x158x177 120 / 117).
+// Measured against the form before (face by face CPML, per-lane 64-bit addresses, tile divisions in
+// the kernel), us for E + B with a 16-cell CPML, one pole and the pulse under way: 512^3 float32 +
+// residual 3616 + 1709 -> 3533 + 1447, float32 3191 + 1058 -> 3179 + 1066, float64 4235 + 2160 -> 4197 +
+// 2187; 256^3 float32 + residual 509 + 271 -> 470 + 232, float32 418 + 180 -> 402 + 182; 64^3 float64, 4-cell
+// layers, 13.5 + 12.3 -> 12.8 + 9.8.
 template <typename T, int NP, bool NONLIN, bool CPML, int L, bool LIN = false, bool RES = false>
 __device__ __forceinline__ void fused_E_tile(const StepArgs<T> &a, int tbx, int tby, int tbz, int soff)
 {
@@ -184,7 +187,9 @@ __device__ __forceinline__ void fused_E_tile(const StepArgs<T> &a, int tbx, int 
         const int i = i0 + u;
         if (i > i1) break;
         const Words<T, RES> b = read3<RES>(c, B, a.Blo);
-        const Pair<T, RES> bk = read2<RES>(c.along(zload ? okm : 0), B[0], B[1], a.Blo);
+        Pair<T, RES> bk;
+        if constexpr (RES) bk = read2<RES>(c.along(zload ? okm : 0), B[0], B[1], a.Blo);
+        else if (zload) bk = read2<RES>(c.along(okm), B[0], B[1], a.Blo);
         const Pair<T, RES> bj = read2<RES>(c.shift(ojm), B[0], B[2], a.Blo);
         const Words<T, RES> e = read3_once<RES>(c, (const T *const *)a.E, a.Elo);
         const size_t prow = c.psi_row();
@@ -293,12 +298,12 @@ __device__ __forceinline__ void fused_E_tile(const StepArgs<T> &a, int tbx, int 
 
 // Fused B side of one step: a thread walks L planes along x keeping E of the next plane as the
 // centre of the following iteration.  Bound and built as the E side: every word of the L planes
-// is requested before the first is used, the z + 1 neighbour by all lanes.  Plain float32 is the
-// exception: its words need no decoding, so the z + 1 neighbour costs nothing under its branch and
-// the few lanes that need it load it, and a layer's auxiliaries ahead of their use cost it registers
-// (78 against 68 for two planes) that its waves are worth more.  Two planes with the auxiliaries
-// ahead and all lanes loading / as it is, us: layers of 8 cells 128^3 25.5 / 23.9, 200^3 93.1 / 82.3,
-// 256^3 161 / 142, 320^3 258 / 234; without layers 200^3 68.7 / 63.6.
+// is requested before the first is used, the z + 1 neighbour by all lanes with residuals, else by
+// those that need it (float64 two planes 256^3 all / those 280 / 276, without layers 222 / 214).  Plain
+// float32 loads a layer's auxiliaries where they are used: ahead of their use they cost it registers
+// (78 against 66 for two planes) that its waves are worth more.  Two planes with the auxiliaries ahead
+// and all lanes loading / as it is, us: layers of 8 cells 128^3 25.5 / 23.9, 200^3 93.1 / 82.3, 256^3
+// 161 / 142, 320^3 258 / 234; without layers 200^3 68.7 / 63.6.
 template <typename T, bool CPML, int L, bool LIN = false, bool RES = false>
 __device__ __forceinline__ void fused_B_tile(const StepArgs<T> &a, int tbx, int tby, int tbz, int soff)
 {
@@ -329,7 +334,7 @@ __device__ __forceinline__ void fused_B_tile(const StepArgs<T> &a, int tbx, int 
         const At<LIN> cu = c.shift(u * sx);
         en[u] = read3<RES>(cu.shift((i == g.n[0] && a.periodic[0]) ? -(g.n[0] - 1) * sx : sx), E, a.Elo);
         ej[u] = read2<RES>(cu.shift(ojp), E[0], E[2], a.Elo);
-        if constexpr (!F32) ek[u] = read2<RES>(cu.along(zload ? okp : 0), E[0], E[1], a.Elo);
+        if constexpr (RES) ek[u] = read2<RES>(cu.along(zload ? okp : 0), E[0], E[1], a.Elo);
         else if (zload) ek[u] = read2<RES>(cu.along(okp), E[0], E[1], a.Elo);
         b0[u] = read3_once<RES>(cu, (const T *const *)a.B, a.Blo);
     }
