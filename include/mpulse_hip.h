@@ -75,10 +75,11 @@ extern "C" {
 #define MPX_PATH_FUSED     0  /* one fused E-side and one fused B-side kernel per step */
 #define MPX_PATH_REFERENCE 1  /* one kernel per reference loop: currents, totals, update, wrap */
 #define MPX_PATH_SWEEP     2  /* one kernel per step (E and B in a single x sweep; periodic boundary) */
-#define MPX_PATH_PASS      3  /* one kernel per step: B of step n and E of step n+1 in one x sweep, so E,
-                                 B and the accumulators cross HBM once per step; the first E half and
-                                 the B half owed at a read run on the fused kernels; PLRC solvers,
-                                 either boundary */
+#define MPX_PATH_PASS      3  /* B of step n and E of step n+1 together: in one kernel (one x sweep, E, B
+                                 and the accumulators cross HBM once per step) or, where that is
+                                 faster by size, form, layers and poles, as the two fused kernels,
+                                 with the same bits; the first E half and the B half owed at a read
+                                 run on the fused kernels; PLRC solvers, either boundary */
 
 /* CurrentFactory registry keys, src/fdtd_plrc.t:431-469 */
 #define MPX_FACTORY_CPML          1  /* "cpml_border"          src/cpml_border.cpp:14-140   */
@@ -286,11 +287,14 @@ int  mpx_state_bytes(mpx_solver *s, size_t *bytes);
    kernel, so it starts on the tiles the E-side kernel wrote last (0: forwards).  No
    counterpart in the reference: the hook of
    the tile autotuner.  "newton_cap" (>= 1, default 200) bounds the Kerr Newton iterations of a
-   cell (see mpx_sync).  Pass path: "pass_kernel" 1, the default, marches each block over
-   "march_seg" x planes (0, the default: 16, halved down to 2 on grids too small to fill the
-   chip) of a 64-cell x "march_rows" tile (3 or 7; 0, the default, takes
-   7 where the kernel variant fits four waves per SIMD, else 3);
-   0 updates one cell per thread. */
+   cell (see mpx_sync).  Pass path: a step runs as one kernel or as the two fused kernels, the faster
+   by size, form, layers and poles, until one of these three keys is set, which asks for the one
+   kernel from then on (the bits are the same): "pass_kernel" 1 marches each block over "march_seg"
+   x planes (0, the default: 16, halved down to 2 on grids too small to fill the chip) of a
+   64-cell x "march_rows" tile (3 or 7; 0, the default, takes 7 where the kernel variant fits four
+   waves per SIMD, else 3); "pass_kernel" 0 updates one cell per thread.  "march_seg" and
+   "march_rows" set to 0 leave the choice of kernels as it is.  Layers along z whose faces lie 2 GiB
+   or more apart are beyond the march: such a run takes the two kernels unless "pass_kernel" is 0. */
 int  mpx_set_tuning(mpx_solver *s, const char *key, int value);
 
 /* Streaming copy of `bytes` between two fresh device buffers, `reps` times; mean ms per copy.
@@ -319,7 +323,8 @@ int  mpx_batch_get_time(mpx_batch *b, int *time);
 /* "structure" (0: fused E and fused B kernels over all runs, the default; 1: single-pass sweep;
    2: x-march pass kernel, one launch per step for B of one step and E of the next, with the
    fused E kernel opening and the fused B kernel closing every mpx_batch_step call, so that E
-   and B belong to the same step between calls), "march_b" (fused B: x planes per thread,
+   and B belong to the same step between calls; a batch with a run whose layers along z lie 2 GiB
+   or more apart runs structure 0 in its place, with the same bits), "march_b" (fused B: x planes per thread,
    1 / 2 / 4), "fused_blocks_per_cu" (fused persistent grid = value x CUs), "variant" (sweep
    block shape 0..2, as sweep_variant), "seg" (sweep x planes per tile), "blocks_per_cu" (sweep
    persistent grid), "pass_seg" (x-march planes per block), "pass_rows" (x-march rows per

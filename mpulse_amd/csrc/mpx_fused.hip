@@ -394,9 +394,10 @@ __device__ __forceinline__ void fused_B_tile(const StepArgs<T> &a, int tbx, int 
     }
 }
 
-// The argument block is read from device memory (the solver keeps a copy there): the face
-// tables are indexed at run time, which a by-value kernel argument would have to copy into
-// per-lane scratch.
+// The argument block is read from device memory, where the solver keeps a copy: one upload when it
+// changes instead of 2 KB of kernel arguments a launch.  Nothing here indexes it at run time, so a
+// compact by-value block is possible and would spare the head of a wave one dependent scalar load;
+// it has not been measured.
 // Waves per SIMD the E kernel is compiled for: 6 (at most 80 registers) for the float32 Kerr
 // kernel with one pole and one plane per thread, measured 0.3 % faster than the 5 its registers
 // allow; no constraint otherwise (other variants would spill).

@@ -300,7 +300,7 @@ __global__ __launch_bounds__(256) void k_pass(const PassArgs<T> *__restrict__ pa
 // z tile) read and write the front padding of their row (storage positions 0 .. 30 of a row,
 // before the ghost cell k = 0, hold no cell and are read by no kernel), the last plane of a
 // segment prefetches position 0 of the plane (padding), and the CPML auxiliaries, which only
-// some cells have, are updated under a per-lane mask.
+// some cells have, go through buffer descriptors that drop the other lanes (below).
 // ---------------------------------------------------------------------------------------
 
 // a cell of E or B as stored: three words and the residual word (zero without residuals)
@@ -1032,8 +1032,8 @@ static void launch_march_r(const PassArgs<T> &a, const PassArgs<T> *dev, int np,
 
 // Tile height when none is set: 7 rows (8-wave blocks, two per CU) when the variant fits four
 // waves per SIMD (<= 128 VGPRs), else 3 rows (4-wave blocks, three per CU at three waves per
-// SIMD; the two- and three-pole float32 + residual variants, the plasma variants).  Read once
-// per variant from the compiled kernel.
+// SIMD: three poles, two without layers in float64 or with residuals, the plasma variants).  Read
+// once per variant from the compiled kernel.
 template <typename T, bool RES, bool PL>
 static int march_auto_rows(int np, bool nonlin, bool cp)
 {

@@ -1214,8 +1214,8 @@ static int build(mpx_solver *s, const mpx_desc *desc)
 
 // Band height of the banded block order: the largest power of two that keeps a band-plane
 // near 512 tiles (E side) or 256 tiles (B side) of 64 z cells; on 512^3 that is 64 and 32
-// rows, the fastest of the heights measured (power-of-two bands keep the XCD shares of the
-// block order aligned to whole bands).
+// rows, the fastest of the heights measured.  Without layers, where the XCDs' shares are equal, a
+// power of two keeps them aligned to whole bands; balance_shares moves them off those lines.
 static int auto_band(const mpx::GridDims &g, const int *blo, bool hside)
 {
     const int lo1 = blo ? blo[1] : 1, lo2 = blo ? blo[2] : 1;

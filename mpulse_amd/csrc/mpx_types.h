@@ -96,10 +96,6 @@ struct CpmlFace {
     {
         return ((size_t)(i - lo[0]) * (size_t)n1 + (size_t)(j - lo[1])) * (size_t)n2 + (size_t)(k - lo[2]);
     }
-    __host__ __device__ __forceinline__ bool contains(int i, int j, int k) const
-    {
-        return i >= lo[0] && i <= hi[0] && j >= lo[1] && j <= hi[1] && k >= lo[2] && k <= hi[2];
-    }
 };
 
 // The cells of a face whose stencil lies in the storage box 0 .. n + 1: the layer itself unless it is
