@@ -3268,7 +3268,7 @@ int mpx_batch_create(const mpx_desc *descs, int nruns, mpx_batch **out)
         b->march_ok = b->march_ok && march_fits(s);
     }
     // B planes per thread, ms for 60 steps with 1 / 2 / 4: float64 10 runs of 48^3 to 160^3 76.0 / 74.1 /
-    // 76.2, 4 of 30^3 to 60^3 2.97 / 2.84 / 3.08; float32 55.5 / 56.8 / 57.0 and 2.20 / 2.28 / 2.58
+    // 76.2, 4 of 30^3 to 60^3 2.97 / 2.84 / 3.08; float32 55.1 / 56.2 / 56.5 and, 8 of 40^3 to 60^3, 4.36 / 4.37 / 4.47
     b->march_b = b->esz == 8 ? 2 : 1;
     // shorter x-march segments while 16 planes a block would give fewer than 2048 blocks (pass_args);
     // 8 runs of 40^3 to 60^3 took 130 us a step with 16 planes throughout
